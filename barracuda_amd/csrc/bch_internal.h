@@ -65,6 +65,54 @@ __device__ __forceinline__ float activate(float v, int act) {
   return v;
 }
 
+// ---- f32 products on the bf16 matrix cores ----
+// An f32 x is split into three bf16 parts, x = x0 + x1 + x2 exactly: x0 is x rounded to 8
+// significant bits, x1 the remainder rounded, x2 the rest (8 + 8 + 8 bits and the parts' signs
+// hold 24).  x y then is the sum of nine part products; the six of weight 2^-18 and above
+// (kPartA, kPartB, smallest first) are accumulated in f32 on v_mfma_f32_32x32x16_bf16, whose
+// products are exact.  What is left out is below 2^-26 of each product, a quarter of the
+// rounding of one f32 addition.  This is the scheme of Henry, Tang and Heinecke, "Leveraging the
+// bfloat16 artificial intelligence datatype for higher-precision computations" (ARITH 2019).
+// Why: v_mfma_f32_32x32x2_f32 does 256 FLOP a clock and CU, the bf16 instruction 4096, so six of
+// them still leave 2.7 times the f32 rate.  Integers whose product is below 2^24 stay exact.
+// An infinite x has x0 = x and x1 NaN, and parts of |x| below 2^-103 reach past bf16's normal
+// range: callers look for both (kSplitTiny) and redo such blocks in f32.
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+constexpr float kSplitTiny = 0x1p-100f;
+constexpr int kPartA[6] = {2, 1, 0, 1, 0, 0}, kPartB[6] = {0, 1, 2, 0, 1, 0};
+
+// Two floats rounded to bf16, x in the low half.
+__device__ __forceinline__ unsigned bf16_pack(float x, float y) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x, y}), bf16x2));
+}
+// Parts p[0..2] of eight floats; returns max(m, |v[0]|, ..., |v[7]|) (NaN left out).
+__device__ __forceinline__ float split8(const float (&v)[8], u32x4 (&p)[3], float m) {
+  float x[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = v[e];
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) m = fmaxf(m, fmaxf(fabsf(x[e]), fabsf(x[e + 1])));
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      p[q][e] = bf16_pack(x[2 * e], x[2 * e + 1]);
+      if (q < 2) {
+        x[2 * e] -= __builtin_bit_cast(float, p[q][e] << 16);
+        x[2 * e + 1] -= __builtin_bit_cast(float, p[q][e] & 0xffff0000u);
+      }
+    }
+  return m;
+}
+__device__ __forceinline__ f32x16 bf16_mm(u32x4 a, u32x4 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
+                                                 0);
+}
+
 struct OpMax {
   __device__ float operator()(float a, float b) const { return fmaxf(a, b); }
 };

@@ -1,4 +1,4 @@
-// sgemm_mfma.hip -- f32 GEMM on the gfx950 FP32 matrix cores.
+// sgemm_mfma.hip -- f32 GEMM on the gfx950 matrix cores.
 //
 // Replaces MatMul::execute (crates/barracuda/src/ops/matmul.rs:89-214; WGSL
 // kernels K1 shaders/math/matmul_gpu_evolved_f64.wgsl, K2
@@ -8,44 +8,26 @@
 // inputs, f32 accumulation, row-major.
 //
 // Design:
-//   * v_mfma_f32_32x32x2_f32: a wavefront multiplies a 32x2 A block by a 2x32
-//     B block into a 32x32 f32 accumulator (16 values per lane).  Lane l
-//     supplies A[l%32][l/32] and B[l/32][l%32]; result value r of lane l is
-//     C[8*(r/4) + 4*(l/32) + r%4][l%32].
-//   * The k index each lane half feeds is free (the MFMA sums over it), so
-//     lane half h takes k = 8c + 4h + s in MFMA step s of 8-wide chunk c.
-//     Both operands are then 4 consecutive k values per lane: one
-//     ds_read_b128 per 32-row block feeds four MFMAs.  To make that true for
-//     B as well, B tiles are stored k-contiguous ([n][k]) in LDS: each thread
-//     loads a 4(k) x 4(n) block with four 128-bit global loads and writes it
-//     transposed with four 128-bit LDS stores, the lanes of a store phase
-//     covering one LDS row.  The unguarded 256-row tiles instead keep B
-//     row-major in LDS and read each lane's four k as four 32-bit values
-//     (BROW in the kernel).
-//   * Block tile BM x BN x BK (256x256, 256x128 or 128x128 by shape, see
-//     pick_tile), four wavefronts in a 2x2 grid, each owning a (BM/2) x (BN/2)
-//     sub-tile of (BM/64) x (BN/64) MFMA blocks (the 256x256 tile with the
-//     bias and activation epilogue: eight wavefronts, 2 x 4).  LDS rows
-//     are padded by 4 floats so the 128-bit reads of 32 consecutive rows do
-//     not collide on banks.  LDS is double-buffered, with one register set
-//     staging the global loads: tile t + 1 goes from registers to the other
-//     LDS buffer in chunk NC - 2 of tile t, and the loads of tile t + 2 are
-//     issued right behind those stores, so every load has a whole tile of
-//     MFMAs (and the barrier) to land; one barrier per k-tile.  Measured at
-//     4096^3 against issuing tile t + 1's loads at the top of tile t (two
-//     chunks to land): 136.8 -> 143.1 TFLOP/s (NN), 141.6 -> 148.1 (B as
-//     [n][k], bias + ReLU), 131.6 -> 137.6 (16 x 1024^3 batched).  Two
-//     register sets (loads two tiles ahead) spill 274 VGPRs.
-//   * Software pipeline inside a tile: the operand fragments are
-//     double-buffered by 8-wide chunk, so the LDS reads of chunk c + 1 issue
-//     between the MFMAs of chunk c, the next tile's LDS stores issue between
-//     the MFMAs of the second-to-last chunk, and the barrier sits before the
-//     last chunk's MFMAs (whose fragments are already in registers) while
-//     the next tile's first reads overlap them.  Scheduling groups pin that
-//     order.  Measured at 4096^3 against the same tiles with each chunk's
-//     reads after the previous chunk's MFMAs and the stores, a full LDS wait
-//     and the barrier after all of them: 133.0 -> 138.6 TFLOP/s (NN), 135.2
-//     -> 142.2 (B as [n][k]), 124 -> 129 (16 x 1024^3 batched).
+//   * Each f32 is split exactly into three bf16 parts on its way into LDS and a product is six
+//     bf16 part products accumulated in f32 (bch_internal.h, split8): 16 k of a 32 x 32 block are
+//     six v_mfma_f32_32x32x16_bf16 (192 matrix-core cycles) instead of eight
+//     v_mfma_f32_32x32x2_f32 (512).  Error against 64 bits (2-norm, N(0,1) inputs, f32 -> split):
+//     4096^3 1.1e-6 -> 1.0e-6, 1024^3 5.7e-7 -> 4.9e-7, 256^3 2.9e-7 -> 2.3e-7 (fewer roundings of
+//     the accumulator per k).  Blocks whose operands the parts cannot stand for are redone on
+//     the f32 instruction (end of the kernel).  Same box, against f32 MFMAs (us): 4096^3 934 -> 578
+//     (147 -> 238 TFLOP/s), 16 x 1024^3 247 -> 159, 2047 x 3001 x 1537 284 -> 110, 512 x 11008 x
+//     4096 and back with bias and GELU 717 -> 500.
+//   * What bounds it: with a workgroup on every CU the clock.  64 workgroups of 256 x 256 run
+//     at 80% of the matrix-core peak (3.2 us per 32 k), 256 of them at 57% (4.5 us).  Splitting
+//     once per workgroup on the way into LDS, not once per fragment, keeps the conversions (5.5
+//     VALU operations per element) at a sixth of the issue slots.
+//   * Operand layout of the 32x32x16 instruction: lane l holds row l % 32 of A (column of B), k
+//     8 (l / 32) .. + 7; result value r of lane l is C[8 (r / 4) + 4 (l / 32) + r % 4][l % 32].
+//     LDS keeps each part as [k octet][row][8 k]: a fragment is one 128-bit read of 32
+//     consecutive rows, free of bank conflicts, and B given as [k][n] is transposed by the
+//     conversion itself, which packs pairs along k.
+//   * LDS is double-buffered, one barrier per pass, the next pass's first fragments read across
+//     it (see the loop); one register set stages the global loads.
 //   * Workgroup -> tile mapping is XCD-aware: gfx950 dispatches workgroups
 //     round-robin over 8 XCDs, so consecutive workgroup ids are remapped to
 //     one XCD's contiguous range of tiles, then walked in groups of 8 tile
@@ -53,81 +35,90 @@
 //     XCD's L2.  A batched launch gives each XCD a contiguous run of
 //     (batch, tile) slots, i.e. whole batches where they divide the run.
 //   * CHECK=false needs m % BM == 0, n % BN == 0, k % BK == 0, lda/ldb/
-//     strides multiples of 4 and 16-byte aligned A/B; CHECK=true guards
-//     every load (zero fill) and store and handles any shape and alignment.
+//     strides multiples of 4 and 16-byte aligned A/B; CHECK=true handles any shape and alignment:
+//     rows and columns outside the matrix are read from its last ones and not stored, and only
+//     the pass with the k remainder, taken first, loads element by element.
 //   * TB: B is given as [n][k] (ldb >= k), C = A B^T -- the linear layer's
 //     y = x W^T with W [out, in] (shaders/misc/linear_f64.wgsl, the layers of
-//     nn/fused_mlp.rs:38-168).  Its tile is already k-contiguous, so it is
-//     loaded like the A tile (128-bit rows straight into LDS [n][k]).
+//     nn/fused_mlp.rs:38-168); it is loaded like A.
 //   * Epilogue: C = act(acc (+ bias[col])) with act none, ReLU or GELU (tanh
 //     form), fused into the store -- linear_f64.wgsl adds the bias after the
 //     dot product, and fused_mlp runs relu_f64.wgsl (gelu_f64.wgsl for a GELU
-//     layer) as a separate pass over the output.  EPI is a
-//     template flag so the plain GEMM stores straight from the accumulators
-//     (420 VGPRs, no spill at 256x256); the bias/activation variant of that tile
-//     parks 8 accumulators in scratch for the epilogue only (36 bytes per
-//     lane, no AGPR copies in the k-loop; measured at the plain kernel's
-//     rate).
+//     layer) as a separate pass over the output.
 #include "bch_internal.h"
 
 #include <stdint.h>
 
 #include <algorithm>
 #include <string>
+#include <type_traits>
 
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+using bch::bf16_mm;
+using bch::f32x16;
+using bch::split8;
+using bch::u32x4;
 
+// Workgroup shapes.  BM x BN x BK name the tile; KS is the k-depth of one LDS buffer (a pass of
+// the loop), WM x WN the wavefront grid.  Two wavefronts per SIMD everywhere but on the small
+// tile: one's conversions and LDS reads run under the other's MFMAs.  Measured on one box
+// (TFLOP/s, the first number four wavefronts with KS 16): 256 x 128 at 2048 x 4096 x 2048 166 ->
+// 209 (4 x 2, KS 32), 128 x 128 at 2048^3 156 -> 189 (2 x 4, KS 32).
+template <int BM, int BN>
+struct Shape {};
+template <>
+struct Shape<256, 256> { static constexpr int WM = 2, WN = 4, KG = 1, KS = 16; };
+template <>
+struct Shape<256, 128> { static constexpr int WM = 4, WN = 2, KG = 1, KS = 32; };
+template <>
+struct Shape<128, 128> { static constexpr int WM = 2, WN = 4, KG = 1, KS = 32; };
+template <>
+struct Shape<64, 64> { static constexpr int WM = 2, WN = 2, KG = 2, KS = 64; };
 
-// W8: eight wavefronts (2 x 4, each (BM/2) x (BN/4)) instead of four, two per SIMD.  Taken by the
-// 256x256 tile with the bias and activation epilogue, where a SIMD's second wavefront overlaps
-// the epilogue's VALU work.  Same box, two runs each (us, 4 -> 8 wavefronts, [out, in] weights
-// with bias): GELU 4096^3 951.6 -> 940.0-940.5, 8192 x 4096 x 4096 1895-1897 -> 1873-1874,
-// 4096 x 11008 x 4096 2630-2631 -> 2603-2607, 6144^3 3164-3165 -> 3144-3145, 4000^3 (float4
-// guards) 941-942 -> 917-918; ReLU 4000^3 922-924 -> 904-905, the others within 0.3%.  Without
-// an epilogue the 256x256 tile stays on four wavefronts: eight took 4096^3 146.5 -> 144.8
-// TFLOP/s.
-template <int BM, int BN, int BK, bool W8 = false>
+template <int BM, int BN, int BK>
 struct Cfg {
-  static constexpr int NT = W8 ? 512 : 256;          // threads per workgroup
-  static constexpr int WN = NT / 128;                // waves along n (2 or 4)
-  static constexpr int LDK = BK + 4;                 // padded LDS row (floats)
-  static constexpr int A_F4 = BM * BK / 4 / NT;  // float4 of A per thread
-  static constexpr int B_BLK = BK * BN / 16 / NT;  // 4x4 B blocks per thread
-  static constexpr int TM = BM / 64;                 // MFMA blocks per wave (m)
-  static constexpr int TN = BN / 32 / WN;            // MFMA blocks per wave (n)
-  static constexpr int LDS_FLOATS = 2 * (BM + BN) * LDK;
-  static_assert(BM % 64 == 0 && BN % 64 == 0, "tile must be a multiple of 64");
-  static_assert(BK % 8 == 0, "BK must be a multiple of 8");
-  static_assert(A_F4 * NT * 4 == BM * BK, "A tile must split evenly");
-  static_assert(B_BLK * NT * 16 == BK * BN, "B tile must split evenly");
+  using S = Shape<BM, BN>;
+  static constexpr int KS = S::KS, WM = S::WM, WN = S::WN, KG = S::KG;
+  static constexpr int NT = 64 * WM * WN * KG;              // threads per workgroup
+  static constexpr int NO = KS / 8;                         // 8-wide k octets per pass
+  static constexpr int PAD = 128 / NO;                      // bytes between octets (see the kernel)
+  static constexpr int ASTR = BM * 16 + PAD, BSTR = BN * 16 + PAD;  // bytes of one octet of one part
+  static constexpr int ABYTES = 3 * NO * ASTR, BUF = ABYTES + 3 * NO * BSTR;
+  static constexpr int LDS_BYTES = 2 * BUF;
+  static constexpr int CA = BM * NO / NT, CB = BN * NO / NT;  // octets of A and of B per thread
+  static constexpr int TM = BM / WM / 32, TN = BN / WN / 32;  // MFMA blocks per wavefront
+  static_assert(CA * NT == BM * NO && CB * NT == BN * NO, "tile must split evenly over the threads");
+  static_assert(BK % KS == 0, "a k-tile is whole passes");
+  static_assert(BN % 64 == 0, "a wavefront's columns of a [k][n] B share one octet");
+  static_assert(LDS_BYTES <= 160 * 1024, "LDS");
 };
 
-__device__ __forceinline__ float4 ld4(const float* p) {
-  return *reinterpret_cast<const float4*>(p);
+// Eight consecutive floats; only 4-byte aligned unless ALIGNED.
+template <bool ALIGNED>
+__device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
+  typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+  using V = std::conditional_t<ALIGNED, bch::f32x4, f32x4u>;
+  const V x = *reinterpret_cast<const V*>(p), y = *reinterpret_cast<const V*>(p + 4);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    v[e] = x[e];
+    v[4 + e] = y[e];
+  }
 }
 
-// The kernel without epilogue stores C block by block during its last k-tile
-// (kernel's ES path) when set.  Against storing after the last k-tile (same
-// box, three runs each): 16 x 1024^3 batched 248.1 -> 244.4 us (+1.5%),
-// 16384 x 4096 x 512 +2.4%, 4096 x 4096 x 1024 +1.6%, 8192^3 +0.4%, 4096^3
-// +0.3%, 4000^3 (float4 guards) +0.7%, 2000 x 2000 x 95 and 4095 x 4096 x 33
-// (scalar guards) +6% and +4%.
-constexpr bool kEarlyStore = true;
-
-template <int BM, int BN, int BK, bool CHECK, bool TB, bool EPI, bool V4 = false, bool KF = false, bool HY = false>
-__global__ __launch_bounds__((EPI && BM == 256 && BN == 256) ? 512 : 256) void sgemm_mfma_kernel(
+// CHECK: any sizes (rows and columns outside the matrix are read from its last ones and not
+// stored; a k remainder is taken by the first pass).  V4: 16-byte aligned rows.
+template <int BM, int BN, int BK, bool CHECK, bool TB, bool EPI, bool V4 = false, bool HY = false>
+__global__ __launch_bounds__((Cfg<BM, BN, BK>::NT)) void sgemm_mfma_kernel(
     int M, int N, int K, const float* __restrict__ A, int lda, long long sA,
     const float* __restrict__ B, int ldb, long long sB, float* __restrict__ C,
     int ldc, long long sC, int tiles_m, int tiles_n, const float* __restrict__ bias, int act,
     int hy_ndp, int hy_r, int hy_kt, float* __restrict__ hy_P, long long sAz, long long sBz, long long sCz) {
-  using G = Cfg<BM, BN, BK, EPI && BM == 256 && BN == 256>;
-  constexpr int LDK = G::LDK;
+  using G = Cfg<BM, BN, BK>;
+  constexpr int KS = G::KS, NO = G::NO, TM = G::TM, TN = G::TN;
   extern __shared__ float4 smem4[];
-  float* smem = reinterpret_cast<float*>(smem4);
-  float* As = smem;                      // [2][BM][LDK]
-  float* Bs = smem + 2 * BM * LDK;       // [2][BN][LDK], k-contiguous
+  char* const smem = reinterpret_cast<char*>(smem4);
 
   // ---- tile mapping (XCD-aware, grouped) ----
   const int ntiles = tiles_m * tiles_n;
@@ -205,376 +196,279 @@ __global__ __launch_bounds__((EPI && BM == 256 && BN == 256) ? 512 : 256) void s
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 31, lh = lane >> 5;
-  const int wm = (wave / G::WN) * (BM / 2);
+  const int kg = G::KG > 1 ? wave / (G::WM * G::WN) : 0;  // this wavefront's share of a pass's k
+  const int wm = (wave / G::WN % G::WM) * (BM / G::WM);
   const int wn = (wave % G::WN) * (BN / G::WN);
 
-  // ---- global -> register staging ----
-  // A: float4 f covers row (tid / (BK/4)) + f * (NT / (BK/4)), cols
-  //    4*(tid % (BK/4)) .. +3 of the k-tile.
-  constexpr int A_TPR = BK / 4;                 // threads per A row
-  constexpr int A_RSTEP = G::NT / A_TPR;     // rows per float4 round
-  const int a_r = tid / A_TPR, a_c = (tid % A_TPR) * 4;
-  // B: 4x4 block q covers k rows 4*kq .. +3 and n cols 4*nq .. +3 where
-  //    blk = tid + q*NT, kq = blk % (BK/4), nq = blk / (BK/4).  The 8
-  //    lanes of an LDS store phase then write one row's 8 consecutive float4
-  //    (128 contiguous bytes, no bank conflict); with nq varying fastest
-  //    they wrote rows 4 apart, 16-way conflicted (measured: 130.5 vs 134.3
-  //    TFLOP/s at 4096^3).  A global load still covers whole 128-byte lines.
-  constexpr int B_KQ = BK / 4;
-  // BROW (unguarded [K][N] B, 256-row tiles): B is kept row-major in LDS ([k][LDN], rows
-  // copied with 128-bit loads and stores like A) and its fragments are read as four 32-bit
-  // values per block.  The 4 x 4 transpose through registers it replaces left the staged
-  // registers permuted across the loop's back edge, so every iteration ended copying them
-  // behind a wait for all of the next tile's loads.  Same box, two runs each, TFLOP/s: 4096^3
-  // 145.4 -> 147.1, 16 x 1024^3 batched 135.7 -> 138.5, 8192 x 8192 x 2048 144.2 -> 145.8,
-  // 4096 x 4096 x 1024 138.2 -> 139.3, 3072^3 (256 x 128 tiles) 137.0 -> 137.8; the 128 x 128
-  // tile, with 16 MFMAs a chunk for its 8 extra LDS reads, lost (2048 x 2048 x 4096 136.1 ->
-  // 121.5) and keeps the transpose.  (The compiler pairs those reads into ds_read2_b32; with the
-  // scheduling groups counting the pairs its loop waits only for the previous tile's loads, and
-  // it measured even: 128 x 11008 x 4096 109.2-110.3 -> 108.2 us, 2048 x 2048 x 4096 250.2 ->
-  // 252.8, 2048 x 2048 x 1024 68.9 -> 68.3, 1024 x 1024 x 4096 unchanged.)
-  // The 64 x 64 small tile (BK 64) takes the row layout too, with its fragments' B values counted
-  // as read pairs in the scheduling groups (the compiler merges them into ds_read2_b32; counted
-  // singly they overfill its 4-MFMA chunks): its loop had ended copying the staged B registers
-  // behind a wait for the next tile's loads.  Same box, two runs each (us): 256^3 8.6-8.7 ->
-  // 8.0-8.1, 512^3 13.5-13.7 -> 13.4, 768^3 19.1-19.2 -> 18.8-18.9, 1024^3 24.4 -> 24.5-24.6,
-  // 1024 x 2048 x 1024 even.
-  constexpr bool BROW = !TB && !CHECK && (BM == 256 || (BM == 64 && BN == 64));
-  constexpr int LDN = BN + 4;                   // padded [k] row of B (floats)
-  constexpr int B_TPR = BN / 4;                 // threads per B row
-  constexpr int B_RSTEP = G::NT / B_TPR;     // B rows per float4 round
-  static_assert(!BROW || (BK * LDN <= BN * LDK && 4 * G::B_BLK * B_RSTEP == BK), "B row layout");
-  const int b_r = tid / B_TPR, b_c = (tid % B_TPR) * 4;
-
-  float4 ra[G::A_F4];
-  float4 rb[G::B_BLK][4];  // TB: rb[q][e] is float4 number 4q + e of the [n][k] tile rows
-
-  // V4 (with CHECK): K, N, the leading dimensions and strides are multiples
-  // of 4, A and B 16-byte aligned, and each operand's extent below 2 GiB.  A
-  // float4 then lies wholly inside or wholly outside the matrix, and the
-  // guarded load is one range-checked buffer load: outside, its offset is
-  // set past the resource's end and the hardware returns zeros.  The guard
-  // acts on the address only, so nothing waits on the data before the LDS
-  // store a tile later (a select on the loaded value made every load's
-  // latency exposed: 4000^3 at 87 TFLOP/s against 97 for scalar guards).
-  // Offsets stay below 2^32: kBad plus at most 2^31 - 1 (the host checks that
-  // (K + BK) rows of a [K][N] B fit in 2^31 bytes).  A row (column) outside
-  // the matrix keeps kBad in its base offset, so adding the column of the
-  // load leaves it past the end.  Only the k check remains: a [K][N] B never
-  // needs it (rows from K on are past the resource's end), and with K a
-  // multiple of BK (KF) no load of A or of a [N][K] B reaches past K either,
-  // so those loads are one add.  Against the compare-and-select on every
-  // load (same box, clocks settled): 4100 x 4100 x 4096 and 6000 x 6000 x
-  // 3200 (128 x 128 tile) +3.2%, 3000 x 3000 x 1000 (ragged K, only the
-  // [K][N] check gone) +2.3%, 4000^3 +1.7%, 2000 x 8000 x 4096 +1.2%.
-  constexpr unsigned kBad = 0x80000000u;  // an offset past every resource's end
-  // (unused, and removed, unless CHECK && V4)
-  const int a_bytes = (int)(((long long)(M - 1) * lda + K) * 4);
-  const int b_bytes = TB ? (int)(((long long)(N - 1) * ldb + K) * 4) : (int)(((long long)(K - 1) * ldb + N) * 4);
-  const __amdgpu_buffer_rsrc_t ra_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(A), 0, a_bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(B), 0, b_bytes, 0x00020000);
-  unsigned aoff[G::A_F4], boff[TB ? 4 * G::B_BLK : G::B_BLK];
-  if constexpr (CHECK && V4) {
+  // ---- global -> registers: octets of 8 k of one row of A (column of B) ----
+  // A row-major operand (A, and B given as [n][k]): octet ch covers row ch / NO, k 8 (ch % NO) ..
+  // +7 of the pass, two 128-bit loads.  A [k][n] B: octet ch covers column ch % BN, k 8 (ch / BN)
+  // .. +7, eight 32-bit loads of 64 consecutive columns by a wavefront, its row offsets scalar;
+  // packing pairs along k in the conversion is the transpose.
+  constexpr bool AL = !CHECK || V4;
+  float ra[G::CA][8], rb[G::CB][8];
+  const float* pa[G::CA];
+  const float* pb[G::CB];
 #pragma unroll
-    for (int f = 0; f < G::A_F4; ++f) {
-      const int gr = m0 + a_r + f * A_RSTEP;
-      aoff[f] = gr < M ? (unsigned)gr * (unsigned)lda * 4u : kBad;  // row start, or kBad
-    }
+  for (int c = 0; c < G::CA; ++c) {
+    const int ch = tid + c * G::NT;
+    const int r = CHECK ? min(m0 + ch / NO, M - 1) : m0 + ch / NO;
+    pa[c] = A + (long long)r * lda + 8 * (ch % NO);
+  }
+#pragma unroll
+  for (int c = 0; c < G::CB; ++c) {
+    const int ch = tid + c * G::NT;
     if constexpr (TB) {
-#pragma unroll
-      for (int f = 0; f < 4 * G::B_BLK; ++f) {
-        const int gr = n0 + a_r + f * A_RSTEP;
-        boff[f] = gr < N ? (unsigned)gr * (unsigned)ldb * 4u : kBad;
-      }
+      const int r = CHECK ? min(n0 + ch / NO, N - 1) : n0 + ch / NO;
+      pb[c] = B + (long long)r * ldb + 8 * (ch % NO);
     } else {
-#pragma unroll
-      for (int q = 0; q < G::B_BLK; ++q) {
-        const int gn = n0 + 4 * ((tid + q * G::NT) / B_KQ);
-        boff[q] = gn < N ? (unsigned)gn * 4u : kBad;  // column, or kBad
-      }
+      const int oct = wave / (BN / 64) + c * (G::NT / BN);  // ch / BN, uniform over the wavefront
+      pb[c] = B + (long long)(8 * oct) * ldb;
     }
   }
-  auto ld4_rs = [&](__amdgpu_buffer_rsrc_t rs, unsigned off) {
-    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
-  };
-  auto load_tile = [&](int k0) {
+  // (TB unset) this thread's column of B; NT % BN == 0 or BN % NT == 0 keeps ch % BN simple
+  int cb[G::CB];
 #pragma unroll
-    for (int f = 0; f < G::A_F4; ++f) {
-      const int r = a_r + f * A_RSTEP;
-      const int gr = m0 + r, gc = k0 + a_c;
-      if (!CHECK) {
-        ra[f] = ld4(A + (long long)gr * lda + gc);
-      } else if (V4) {
-        ra[f] = ld4_rs(ra_rs, KF ? aoff[f] + (unsigned)gc * 4u
-                                : (aoff[f] != kBad && gc < K) ? aoff[f] + (unsigned)gc * 4u : kBad);
+  for (int c = 0; c < G::CB; ++c) {
+    const int col = n0 + (tid + c * G::NT) % BN;
+    cb[c] = CHECK ? min(col, N - 1) : col;
+  }
+  auto load_pass = [&](int k0) {
+#pragma unroll
+    for (int c = 0; c < G::CA; ++c) load8<AL>(pa[c] + k0, ra[c]);
+#pragma unroll
+    for (int c = 0; c < G::CB; ++c) {
+      if constexpr (TB) {
+        load8<AL>(pb[c] + k0, rb[c]);
       } else {
-        float t[4];
+        const float* s = pb[c] + (long long)k0 * ldb;
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          t[e] = (gr < M && gc + e < K) ? A[(long long)gr * lda + gc + e] : 0.0f;
-        ra[f] = make_float4(t[0], t[1], t[2], t[3]);
+        for (int e = 0; e < 8; ++e) rb[c][e] = s[(long long)e * ldb + (unsigned)cb[c]];
       }
     }
-    if constexpr (TB) {
-      // rows of B^T are rows of the [n][k] input: same pattern as A
+  };
+  // the k remainder: k0 .. K - 1, zeros from K on (loads past K read the last k instead)
+  auto load_rest = [&](int k0) {
 #pragma unroll
-      for (int f = 0; f < 4 * G::B_BLK; ++f) {
-        const int r = a_r + f * A_RSTEP;
-        const int gr = n0 + r, gc = k0 + a_c;
-        if (!CHECK) {
-          rb[f >> 2][f & 3] = ld4(B + (long long)gr * ldb + gc);
-        } else if (V4) {
-          rb[f >> 2][f & 3] = ld4_rs(rb_rs, KF ? boff[f] + (unsigned)gc * 4u
-                                           : (boff[f] != kBad && gc < K) ? boff[f] + (unsigned)gc * 4u : kBad);
-        } else {
-          float t[4];
+    for (int c = 0; c < G::CA; ++c) {
+      const int k = k0 + 8 * ((tid + c * G::NT) % NO);
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            t[e] = (gr < N && gc + e < K) ? B[(long long)gr * ldb + gc + e] : 0.0f;
-          rb[f >> 2][f & 3] = make_float4(t[0], t[1], t[2], t[3]);
-        }
+      for (int e = 0; e < 8; ++e) {
+        const float v = pa[c][min(k + e, K - 1) - k + k0];
+        ra[c][e] = k + e < K ? v : 0.0f;
       }
-    } else if constexpr (BROW) {
+    }
 #pragma unroll
-      for (int f = 0; f < 4 * G::B_BLK; ++f)
-        rb[f >> 2][f & 3] = ld4(B + (long long)(k0 + b_r + f * B_RSTEP) * ldb + n0 + b_c);
-    } else {
+    for (int c = 0; c < G::CB; ++c) {
+      const int k = k0 + 8 * (TB ? (tid + c * G::NT) % NO : wave / (BN / 64) + c * (G::NT / BN));
 #pragma unroll
-      for (int q = 0; q < G::B_BLK; ++q) {
-        const int blk = tid + q * G::NT;
-        const int kq = blk % B_KQ, nq = blk / B_KQ;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int gk = k0 + 4 * kq + e, gn = n0 + 4 * nq;
-          if (!CHECK) {
-            rb[q][e] = ld4(B + (long long)gk * ldb + gn);
-          } else if (V4) {
-            rb[q][e] = ld4_rs(rb_rs, (unsigned)gk * (unsigned)ldb * 4u + boff[q]);
-          } else {
-            float t[4];
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-              t[c] = (gk < K && gn + c < N) ? B[(long long)gk * ldb + gn + c] : 0.0f;
-            rb[q][e] = make_float4(t[0], t[1], t[2], t[3]);
-          }
-        }
+      for (int e = 0; e < 8; ++e) {
+        const int d = min(k + e, K - 1) - k + k0;
+        const float v = TB ? pb[c][d] : pb[c][(long long)d * ldb + cb[c]];
+        rb[c][e] = k + e < K ? v : 0.0f;
       }
     }
   };
 
-  auto store_tile = [&](int buf) {
-    float* as = As + buf * BM * LDK;
-    float* bs = Bs + buf * BN * LDK;
+  // ---- registers -> LDS: three bf16 parts per float ----
+  // [buffer][A or B][part][octet][row][8 k]: a fragment read takes 16 bytes of 32 consecutive
+  // rows, so it needs no padding; PAD shifts the octets so that the eight lanes of a store phase
+  // (128 / NO bytes of each of NO octets of a row-major operand) cover different banks.
+  float ma[G::CA], mb[G::CB];  // largest magnitude each octet position has held
 #pragma unroll
-    for (int f = 0; f < G::A_F4; ++f) {
-      const int r = a_r + f * A_RSTEP;
-      *reinterpret_cast<float4*>(as + r * LDK + a_c) = ra[f];
+  for (int c = 0; c < G::CA; ++c) ma[c] = 0.0f;
+#pragma unroll
+  for (int c = 0; c < G::CB; ++c) mb[c] = 0.0f;
+  auto store_a = [&](int buf) {
+    char* s = smem + buf * G::BUF;
+#pragma unroll
+    for (int c = 0; c < G::CA; ++c) {
+      const int ch = tid + c * G::NT;
+      u32x4 q[3];
+      ma[c] = split8(ra[c], q, ma[c]);
+#pragma unroll
+      for (int p3 = 0; p3 < 3; ++p3)
+        *reinterpret_cast<u32x4*>(s + (p3 * NO + ch % NO) * G::ASTR + (ch / NO) * 16) = q[p3];
     }
-    if constexpr (TB) {
+  };
+  auto store_b = [&](int buf) {
+    char* s = smem + buf * G::BUF + G::ABYTES;
 #pragma unroll
-      for (int f = 0; f < 4 * G::B_BLK; ++f) {
-        const int r = a_r + f * A_RSTEP;
-        *reinterpret_cast<float4*>(bs + r * LDK + a_c) = rb[f >> 2][f & 3];
-      }
-      return;
-    }
-    if constexpr (BROW) {
+    for (int c = 0; c < G::CB; ++c) {
+      const int ch = tid + c * G::NT;
+      const int row = TB ? ch / NO : ch % BN, oct = TB ? ch % NO : ch / BN;
+      u32x4 q[3];
+      mb[c] = split8(rb[c], q, mb[c]);
 #pragma unroll
-      for (int f = 0; f < 4 * G::B_BLK; ++f)
-        *reinterpret_cast<float4*>(bs + (b_r + f * B_RSTEP) * LDN + b_c) = rb[f >> 2][f & 3];
-      return;
-    }
-#pragma unroll
-    for (int q = 0; q < G::B_BLK; ++q) {
-      const int blk = tid + q * G::NT;
-      const int kq = blk % B_KQ, nq = blk / B_KQ;
-      // transpose the 4(k) x 4(n) block: column c of rb -> LDS row n
-      float* base = bs + (4 * nq) * LDK + 4 * kq;
-      *reinterpret_cast<float4*>(base + 0 * LDK) =
-          make_float4(rb[q][0].x, rb[q][1].x, rb[q][2].x, rb[q][3].x);
-      *reinterpret_cast<float4*>(base + 1 * LDK) =
-          make_float4(rb[q][0].y, rb[q][1].y, rb[q][2].y, rb[q][3].y);
-      *reinterpret_cast<float4*>(base + 2 * LDK) =
-          make_float4(rb[q][0].z, rb[q][1].z, rb[q][2].z, rb[q][3].z);
-      *reinterpret_cast<float4*>(base + 3 * LDK) =
-          make_float4(rb[q][0].w, rb[q][1].w, rb[q][2].w, rb[q][3].w);
+      for (int p3 = 0; p3 < 3; ++p3) *reinterpret_cast<u32x4*>(s + (p3 * NO + oct) * G::BSTR + row * 16) = q[p3];
     }
   };
 
-  f32x16 acc[G::TM][G::TN];
+  // ---- LDS -> operand fragments: lane l takes row l % 32, k octet l / 32 ----
+  constexpr int NS = KS / 16 / G::KG, NB = NS * TM;  // 16-k steps, block steps of a wavefront's pass
+  const char* const a_base = smem + (2 * NS * kg + lh) * G::ASTR + (wm + li) * 16;
+  const char* const b_base = smem + G::ABYTES + (2 * NS * kg + lh) * G::BSTR + (wn + li) * 16;
+  auto read_a = [&](int buf, int kk, int i, u32x4 (&f)[3]) {
 #pragma unroll
-  for (int i = 0; i < G::TM; ++i)
+    for (int p3 = 0; p3 < 3; ++p3)
+      f[p3] = *reinterpret_cast<const u32x4*>(a_base + buf * G::BUF + (p3 * NO + 2 * kk) * G::ASTR + i * 512);
+  };
+  auto read_b = [&](int buf, int kk, u32x4 (&f)[TN][3]) {
 #pragma unroll
-    for (int j = 0; j < G::TN; ++j)
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int p3 = 0; p3 < 3; ++p3)
+        f[j][p3] = *reinterpret_cast<const u32x4*>(b_base + buf * G::BUF + (p3 * NO + 2 * kk) * G::BSTR + j * 512);
+  };
+
+  f32x16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-  // Fragments are double-buffered by chunk (8 k): the LDS reads of chunk c + 1
-  // are issued before the MFMAs of chunk c, the next tile's LDS stores go out
-  // with chunk NC - 2, and the one barrier per tile sits before the MFMAs of
-  // the last chunk, whose fragments are already in registers.  The reads of
-  // the next tile's chunk 0 then overlap those MFMAs.  Buffer cur ^ 1 was
-  // last read before the previous tile's barrier, so storing it after that
-  // barrier is safe; its reads come after this tile's barrier.
-  constexpr int NC = BK / 8;
-  static_assert(NC % 2 == 0 && NC >= 2, "chunk count must be even");
-  float4 fa[2][G::TM], fb[2][G::TN];
-  auto read_frags = [&](int buf, int c, float4 (&a)[G::TM], float4 (&b)[G::TN]) {
-    const float* as = As + buf * BM * LDK + (wm + li) * LDK + 4 * lh + 8 * c;
+  // Pass t runs NB block steps (row block i of 16-k step kk); each reads the next step's
+  // fragments first, so LDS latency hides under its 6 TN MFMAs.  Pass t + 1's octets are
+  // converted and stored to the other buffer at the start of pass t, and pass t + 2's loads issue
+  // right behind.  The barrier sits before the last step's MFMAs (fragments in registers): every
+  // read of this buffer and every store of the next one is done, and the next pass's first reads
+  // overlap those MFMAs.  The last pass reloads the last tile into the buffer no one reads again.
+  // (A copy of the pass without them, for the end of the loop, spilled 256 VGPRs at 256 x 256.)
+  u32x4 fa[2][3], fb[2][TN][3];
+  const int nk = (K + KS - 1) / KS;
+  const int rest = CHECK && K % KS != 0 ? 1 : 0;  // the remainder runs first, as pass 0
+  auto pass = [&](auto par, int t) {
+    constexpr int P = decltype(par)::value;  // pass parity: LDS buffer and fragment sets
 #pragma unroll
-    for (int i = 0; i < G::TM; ++i) a[i] = *reinterpret_cast<const float4*>(as + i * 32 * LDK);
-    if constexpr (BROW) {
-      // B[k = 8c + 4lh + s][n = wn + 32j + li], s = 0..3: four rows of the [k][n] tile
-      const float* bs = Bs + buf * BN * LDK + (8 * c + 4 * lh) * LDN + wn + li;
-#pragma unroll
-      for (int j = 0; j < G::TN; ++j)
-        b[j] = make_float4(bs[j * 32], bs[LDN + j * 32], bs[2 * LDN + j * 32], bs[3 * LDN + j * 32]);
-    } else {
-      const float* bs = Bs + buf * BN * LDK + (wn + li) * LDK + 4 * lh + 8 * c;
-#pragma unroll
-      for (int j = 0; j < G::TN; ++j) b[j] = *reinterpret_cast<const float4*>(bs + j * 32 * LDK);
-    }
-  };
-  auto mfma_chunk = [&](const float4 (&a)[G::TM], const float4 (&b)[G::TN]) {
-#pragma unroll
-    for (int i = 0; i < G::TM; ++i)
-#pragma unroll
-      for (int j = 0; j < G::TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i].x, b[j].x, acc[i][j], 0, 0, 0);
-#pragma unroll
-    for (int i = 0; i < G::TM; ++i)
-#pragma unroll
-      for (int j = 0; j < G::TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i].y, b[j].y, acc[i][j], 0, 0, 0);
-#pragma unroll
-    for (int i = 0; i < G::TM; ++i)
-#pragma unroll
-      for (int j = 0; j < G::TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i].z, b[j].z, acc[i][j], 0, 0, 0);
-#pragma unroll
-    for (int i = 0; i < G::TM; ++i)
-#pragma unroll
-      for (int j = 0; j < G::TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i].w, b[j].w, acc[i][j], 0, 0, 0);
-  };
-
-  const int nk = (K + BK - 1) / BK;
-  if (nk > 0) {
-    load_tile(0);
-    store_tile(0);
-    load_tile(min(1, nk - 1) * BK);
-  }
-  __syncthreads();
-  if (nk > 0) read_frags(0, 0, fa[0], fb[0]);
-
-  // Branch-free body (one basic block the scheduler can interleave): the
-  // last iteration reloads the last tile into the buffer no one reads again.
-  // The order is pinned with scheduling groups (mask 0x008 MFMA, 0x100 LDS
-  // read, 0x200 LDS write): left alone, the scheduler sank the global loads
-  // to the end of the body behind a vmcnt(0) and clustered the LDS traffic.
-  constexpr int NR = G::TM + (BROW ? (BM == 64 ? 2 : 4) : 1) * G::TN;       // LDS reads per chunk
-  constexpr int NW = G::A_F4 + 4 * G::B_BLK;               // LDS stores per tile
-  constexpr int NM = 4 * G::TM * G::TN;                    // MFMAs per chunk
-  // the small tile (one MFMA block per wavefront) has too few MFMAs in a chunk to pin its
-  // stores between them; they go where the scheduler puts them within their chunk
-  constexpr bool PIN = NM >= NR + NW;
-  constexpr int MPW = !PIN ? 0 : (NM - NR) / NW >= 2 ? 2 : 1;  // MFMAs after each store
-  static_assert(NM >= NR + MPW * NW, "chunk too small to cover its LDS traffic");
-  // ES: the last k-tile is peeled (below) so that C leaves block by block
-  // (the 256 x 128 tile in every load mode, and the scalar-guarded 128 x 128 tile: the
-  // float4-guarded and unguarded 128 x 128 tiles measured 0.2-1.1% slower with it).  The
-  // 256 x 256 tile stores after the loop: with B row-major in LDS, holding the last tile's four
-  // chunks of fragments spilled 64-101 VGPRs to scratch in every load mode, and without the peel
-  // it spills none.  Same box, two runs each (us, peeled -> not): 16 x 1024^3 246.3-247.9 ->
-  // 243.7-243.8, 32 x 1024 x 1024 x 512 264.5 -> 254.5-254.8, 16384 x 4096 x 512 518-520 ->
-  // 502, 4096 x 4096 x 1024 247.3-247.5 -> 243.9-244.5, 4095 x 4096 x 33 (scalar guards)
-  // 38.9-39.0 -> 35.0, 4096^3 and 8192^3 even, 4000^3 (float4 guards) 922.5-924.7 ->
-  // 925.6-927.9.
-  constexpr bool ES = kEarlyStore && !EPI && !HY && G::TN % 2 == 0 && !(BM == 256 && BN == 256) &&
-                      (BM == 256 || (CHECK && !V4));
-  const int nloop = ES ? nk - 1 : nk;
-  for (int t = 0; t < nloop; ++t) {
-    const int cur = t & 1;
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      if (c == NC - 1) __syncthreads();
-      read_frags(c == NC - 1 ? cur ^ 1 : cur, (c + 1) % NC, fa[(c + 1) & 1], fb[(c + 1) & 1]);
-      if (c == NC - 2) {
-        store_tile(cur ^ 1);
-        load_tile(min(t + 2, nk - 1) * BK);
+    for (int b = 0; b < NB; ++b) {
+      const int kk = b / TM, i = b % TM;
+      const int fs = (P * NB + b) & 1, bs = (P * NS + kk) & 1;
+      constexpr int b1 = NB > 2 ? 1 : 0;
+      if (b == 0) store_a(P ^ 1);
+      if (b == b1) {
+        store_b(P ^ 1);
+        load_pass((min(t + 2, nk - 1) - rest) * KS);
       }
-      mfma_chunk(fa[c & 1], fb[c & 1]);
-#pragma unroll
-      for (int r = 0; r < NR; ++r) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      }
-      if (PIN && c == NC - 2) {
-#pragma unroll
-        for (int w = 0; w < NW; ++w) {
-          __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x008, MPW, 0);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x008, NM - NR - MPW * NW, 0);
+      if (b < NB - 1) {
+        const int kn = (b + 1) / TM, in = (b + 1) % TM;
+        read_a(P, kn, in, fa[fs ^ 1]);
+        if (in == 0) read_b(P, kn, fb[bs ^ 1]);
       } else {
-        __builtin_amdgcn_sched_group_barrier(0x008, NM - NR, 0);
+        __syncthreads();
+        read_a(P ^ 1, 0, 0, fa[fs ^ 1]);
+        read_b(P ^ 1, 0, fb[bs ^ 1]);
       }
+#pragma unroll
+      for (int q = 0; q < 6; ++q)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = bf16_mm(fa[fs][bch::kPartA[q]], fb[bs][j][bch::kPartB[q]], acc[i][j]);
       __builtin_amdgcn_sched_barrier(0);
     }
+  };
+  // Fewer k than one pass holds (K = 0 too): the f32 loop below alone, at most KS / 2 steps.
+  const bool short_k = K < KS;
+  __shared__ int tiny_seen;
+  if (tid == 0) tiny_seen = 0;
+  if (!short_k) {
+    if (rest)
+      load_rest((nk - 1) * KS);
+    else
+      load_pass(0);
+    store_a(0);
+    store_b(0);
+    load_pass((min(1, nk - 1) - (nk > 1 ? rest : 0)) * KS);
+    __syncthreads();
+    read_a(0, 0, 0, fa[0]);
+    read_b(0, 0, fb[0]);
+    int t = 0;
+    for (; t + 1 < nk; t += 2) {
+      pass(std::integral_constant<int, 0>{}, t);
+      pass(std::integral_constant<int, 1>{}, t + 1);
+    }
+    if (t < nk) pass(std::integral_constant<int, 0>{}, t);
   }
 
-  if constexpr (ES) {
-    // The last k-tile block-major: its four chunks' fragments at once (chunk 0 is
-    // already in fa[0] / fb[0]; nothing writes LDS any more), then two 32 x 32
-    // blocks' 32 MFMAs at a time, each pair stored while the next pair's MFMAs
-    // run, so C goes out during the last k-tile instead of after it.
-    if (nk > 0) {
-      const int cur = (nk - 1) & 1;
-      float4 la[NC][G::TM], lb[NC][G::TN];
+  // ---- the k shares of a block added up, in share order ----
+  if constexpr (G::KG > 1) {
+    static_assert(G::KG == 2 && TM == 1 && TN == 1 && G::WM * G::WN * 4096 <= G::LDS_BYTES, "one block a wavefront");
+    __syncthreads();  // the last pass's reads are done
+    f32x16* const part = reinterpret_cast<f32x16*>(smem) + (wave % (G::WM * G::WN)) * 64 + lane;
+    if (kg != 0) *part = acc[0][0];
+    __syncthreads();
+    if (kg == 0) acc[0][0] += *part;
+  }
+
+  // ---- where the parts cannot stand for the floats, the tile again in f32 ----
+  // An infinite or NaN operand (or a part product that overflows) leaves a result that is not
+  // finite; a row of A or column of B whose largest magnitude is below 2^-100 has third parts
+  // below bf16's range.  Either is rare, and the wavefront then redoes its blocks on
+  // v_mfma_f32_32x32x2_f32 from global memory.
+  bool redo = short_k;
+  if (!short_k) {
+    float z = 0.0f;
 #pragma unroll
-      for (int i = 0; i < G::TM; ++i) la[0][i] = fa[0][i];
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < G::TN; ++j) lb[0][j] = fb[0][j];
+      for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int c = 1; c < NC; ++c) read_frags(cur, c, la[c], lb[c]);
-      constexpr int NP = G::TM * G::TN / 2;  // block pairs (i, 2q), (i, 2q + 1)
-      auto mm_pair = [&](int pr) {
-        const int i = pr / (G::TN / 2), j = 2 * (pr % (G::TN / 2));
+        for (int r = 0; r < 16; ++r) z = fmaf(acc[i][j][r], 0.0f, z);
+    redo = z != 0.0f;  // NaN
+    bool tiny = false;
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(la[c][i].x, lb[c][j].x, acc[i][j], 0, 0, 0);
-          acc[i][j + 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(la[c][i].x, lb[c][j + 1].x, acc[i][j + 1], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(la[c][i].y, lb[c][j].y, acc[i][j], 0, 0, 0);
-          acc[i][j + 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(la[c][i].y, lb[c][j + 1].y, acc[i][j + 1], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(la[c][i].z, lb[c][j].z, acc[i][j], 0, 0, 0);
-          acc[i][j + 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(la[c][i].z, lb[c][j + 1].z, acc[i][j + 1], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(la[c][i].w, lb[c][j].w, acc[i][j], 0, 0, 0);
-          acc[i][j + 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(la[c][i].w, lb[c][j + 1].w, acc[i][j + 1], 0, 0, 0);
-        }
-      };
-      auto st_pair = [&](int pr) {
-        const int i = pr / (G::TN / 2), j = 2 * (pr % (G::TN / 2));
+    for (int c = 0; c < G::CA; ++c) {
+      float m = ma[c];  // the row's octets sit in NO neighbouring lanes
 #pragma unroll
-        for (int jj = j; jj < j + 2; ++jj) {
-          const int col = n0 + wn + jj * 32 + li;
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int row = m0 + wm + i * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-            if (!CHECK || (row < M && col < N)) C[(long long)row * ldc + col] = acc[i][jj][r];
-          }
-        }
-      };
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int pr = 0; pr < NP; ++pr) {
-        mm_pair(pr);
-        if (pr > 0) st_pair(pr - 1);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      st_pair(NP - 1);
-      return;
+      for (int o = 1; o < NO; o <<= 1) m = fmaxf(m, __shfl_xor(m, o));
+      tiny |= m > 0.0f && m < bch::kSplitTiny;
     }
-    // K = 0: no k-tile to peel; the epilogue below stores the zero accumulators
+#pragma unroll
+    for (int c = 0; c < G::CB; ++c) {
+      float m = mb[c];
+      if constexpr (TB) {
+#pragma unroll
+        for (int o = 1; o < NO; o <<= 1) m = fmaxf(m, __shfl_xor(m, o));
+      }
+      tiny |= m > 0.0f && m < bch::kSplitTiny;
+    }
+    // a wavefront's rows and columns were loaded by others
+    if (tiny) tiny_seen = 1;
+    __syncthreads();
+    redo = tiny_seen != 0 || __any(redo);
+  }
+  if (G::KG > 1 && kg != 0) return;
+  if (redo) {
+    const float* qb[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int n = min(n0 + wn + j * 32 + li, N - 1);
+      qb[j] = TB ? B + (long long)n * ldb : B + n;
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const float* qa = A + (long long)min(m0 + wm + i * 32 + li, M - 1) * lda;
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+#pragma unroll 1
+      for (int k0 = 0; k0 < K; k0 += 2) {
+        const int k = min(k0 + lh, K - 1);
+        const bool in = k0 + lh < K;
+        const float va = qa[k];
+        const float a = in ? va : 0.0f;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const float vb = TB ? qb[j][k] : qb[j][(long long)k * ldb];
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, in ? vb : 0.0f, acc[i][j], 0, 0, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
 
   // ---- epilogue: value r of lane l is row 8*(r/4) + 4*lh + r%4, col li ----
@@ -582,9 +476,9 @@ __global__ __launch_bounds__((EPI && BM == 256 && BN == 256) ? 512 : 256) void s
     if (tail) {  // the slice's sums, a whole BM x BN tile, into its slot of the partials
       float* Pt = hy_P + ((long long)hy_slice * hy_r + hy_slot) * (BM * BN);
 #pragma unroll
-      for (int i = 0; i < G::TM; ++i)
+      for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < G::TN; ++j)
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
           for (int r = 0; r < 16; ++r)
             Pt[(wm + i * 32 + 8 * (r >> 2) + 4 * lh + (r & 3)) * BN + wn + j * 32 + li] = acc[i][j][r];
@@ -593,26 +487,27 @@ __global__ __launch_bounds__((EPI && BM == 256 && BN == 256) ? 512 : 256) void s
   }
   if constexpr (!EPI) {
 #pragma unroll
-    for (int i = 0; i < G::TM; ++i) {
+    for (int i = 0; i < TM; ++i) {
 #pragma unroll
-      for (int j = 0; j < G::TN; ++j) {
+      for (int j = 0; j < TN; ++j) {
         const int col = n0 + wn + j * 32 + li;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int row = m0 + wm + i * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
           if (!CHECK || (row < M && col < N)) C[(long long)row * ldc + col] = acc[i][j][r];
         }
+        __builtin_amdgcn_sched_barrier(0);  // one block's addresses at a time: no spills
       }
     }
   } else {
     // bias and the activation are uniform over the launch (no divergence); one 32 x 32
     // block at a time, so only 16 accumulators are out of the AGPRs at once
 #pragma unroll
-    for (int j = 0; j < G::TN; ++j) {
+    for (int j = 0; j < TN; ++j) {
       const int col = n0 + wn + j * 32 + li;
       const float bj = bias ? (!CHECK || col < N ? bias[col] : 0.0f) : 0.0f;
 #pragma unroll
-      for (int i = 0; i < G::TM; ++i) {
+      for (int i = 0; i < TM; ++i) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int row = m0 + wm + i * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
@@ -626,16 +521,16 @@ __global__ __launch_bounds__((EPI && BM == 256 && BN == 256) ? 512 : 256) void s
   }
 }
 
-template <int BM, int BN, int BK, bool CHECK, bool TB, bool EPI, bool V4 = false, bool KF = false>
+template <int BM, int BN, int BK, bool CHECK, bool TB, bool EPI, bool V4 = false>
 hipError_t launch_tiles(hipStream_t s, int batch, int m, int n, int k,
                         const float* A, int lda, long long sA, const float* B,
                         int ldb, long long sB, float* C, int ldc, long long sC,
                         const float* bias, int act, int nz = 1, long long sAz = 0, long long sBz = 0,
                         long long sCz = 0) {
-  using G = Cfg<BM, BN, BK, EPI && BM == 256 && BN == 256>;
+  using G = Cfg<BM, BN, BK>;
   const int tm = (m + BM - 1) / BM, tn = (n + BN - 1) / BN;
-  const size_t lds = sizeof(float) * G::LDS_FLOATS;
-  auto kern = sgemm_mfma_kernel<BM, BN, BK, CHECK, TB, EPI, V4, KF>;
+  const size_t lds = G::LDS_BYTES;
+  auto kern = sgemm_mfma_kernel<BM, BN, BK, CHECK, TB, EPI, V4>;
   hipError_t e = bch::ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (int)lds);
   if (e != hipSuccess) return e;
   if (batch > 65535 || nz > 65535) return hipErrorInvalidValue;
@@ -646,13 +541,13 @@ hipError_t launch_tiles(hipStream_t s, int batch, int m, int n, int k,
 
 // The hybrid launch (batch 1, K a multiple of BK): ndp whole tiles, then r tiles in
 // S k-slices of kt k-tiles each into P (see HybPlan).
-template <int BM, int BN, int BK, bool CHECK, bool TB, bool EPI, bool V4, bool KF>
+template <int BM, int BN, int BK, bool CHECK, bool TB, bool EPI, bool V4>
 hipError_t launch_hyb_tiles(hipStream_t s, int m, int n, int k, const float* A, int lda, const float* B, int ldb,
                             float* C, int ldc, const float* bias, int act, int ndp, int r, int S, int kt, float* P) {
-  using G = Cfg<BM, BN, BK, EPI && BM == 256 && BN == 256>;
+  using G = Cfg<BM, BN, BK>;
   const int tm = (m + BM - 1) / BM, tn = (n + BN - 1) / BN;
-  const size_t lds = sizeof(float) * G::LDS_FLOATS;
-  auto kern = sgemm_mfma_kernel<BM, BN, BK, CHECK, TB, EPI, V4, KF, true>;
+  const size_t lds = G::LDS_BYTES;
+  auto kern = sgemm_mfma_kernel<BM, BN, BK, CHECK, TB, EPI, V4, true>;
   hipError_t e = bch::ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (int)lds);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kern, dim3(ndp + r * S), dim3(G::NT), lds, s, m, n, k, A, lda, 0LL, B, ldb, 0LL, C, ldc,
@@ -664,28 +559,35 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 constexpr int kBK = 32;
 
-// Tile choice: the tile with the least modelled time, rounds x tile area /
-// efficiency, where a round is one workgroup per CU (one 256x256 workgroup
-// fits a CU; the smaller tiles are timed at full rounds) and the efficiencies
-// are the tiles' measured rates at whole rounds relative to 256x256 (TFLOP/s
-// on MI355X: 256x256 145 at 4096^3, 256x128 140 at 8192 x 1024 x 8192,
-// 128x128 128 at 2048^3).  The largest tile that still fills every CU is
-// what this gives when the counts come out even; otherwise a part-filled last
-// round of large tiles can cost more than more rounds of smaller ones
-// (6144^3: three rounds of 256x256, 107 TFLOP/s).
+// Tile choice: the tile with the least modelled time per 32 k of depth.  One workgroup of a tile
+// alone on the chip takes `idle` us per 32 k, with one on every CU `full` us (the clock falls as
+// more matrix cores run, and L2 is shared): measured at K 2048-4096 on one box, 256 x 256 3.2 /
+// 4.5 (4096^3), 256 x 128 1.9 / 2.45, 128 x 128 1.1 / 1.42 (2048^3).  Whole rounds take `full`, a
+// part-filled last one in between by its share of the CUs.  eff: the tiles' rates at whole
+// rounds relative to 256 x 256, for the hybrid and mixed plans.
 enum class Tile { k256x256, k256x128, k128x128 };
 
-struct TileOpt { Tile t; int bm, bn; double eff; };
-constexpr TileOpt kTileOpts[] = {{Tile::k256x256, 256, 256, 1.0}, {Tile::k256x128, 256, 128, 0.966},
-                                 {Tile::k128x128, 128, 128, 0.92}};
+struct TileOpt { Tile t; int bm, bn; double eff, idle, full; };
+constexpr TileOpt kTileOpts[] = {{Tile::k256x256, 256, 256, 1.0, 3.3, 4.65}, {Tile::k256x128, 256, 128, 0.966, 1.9, 2.45},
+                                 {Tile::k128x128, 128, 128, 0.92, 1.08, 1.42}};
+constexpr double kTileKtUs = 4.6;  // one 256 x 256 k-tile of 32 at whole rounds
+
+// us per 32 k of `wgs` workgroups of tile o
+double tile_kt_us(const TileOpt& o, long long wgs) {
+  const long long cu = bch::device_cu_count();
+  const long long r = wgs % cu;
+  return (double)(wgs / cu) * o.full + (r ? o.idle + (o.full - o.idle) * (double)r / (double)cu : 0.0);
+}
+
+long long tile_count(const TileOpt& o, int batch, int m, int n) {
+  return (long long)batch * ((m + o.bm - 1) / o.bm) * ((n + o.bn - 1) / o.bn);
+}
 
 Tile pick_tile(int batch, int m, int n) {
-  const long long cu = bch::device_cu_count();
   Tile best = Tile::k256x256;
   double best_cost = 0.0;
   for (const TileOpt& o : kTileOpts) {
-    const long long tiles = (long long)batch * ((m + o.bm - 1) / o.bm) * ((n + o.bn - 1) / o.bn);
-    const double cost = (double)((tiles + cu - 1) / cu) * o.bm * o.bn / o.eff;
+    const double cost = tile_kt_us(o, tile_count(o, batch, m, n));
     if (o.t == Tile::k256x256 || cost < best_cost * 0.999) {
       best = o.t;
       best_cost = cost;
@@ -722,19 +624,19 @@ struct ZSplit {
   long long sA = 0, sB = 0, sC = 0;
 };
 
-template <bool CHECK, bool TB, bool EPI, bool V4, bool KF = false>
+template <bool CHECK, bool TB, bool EPI, bool V4>
 hipError_t launch_tile(Tile t, hipStream_t s, int batch, int m, int n, int k, const float* A, int lda,
                        long long sA, const float* B, int ldb, long long sB, float* C, int ldc, long long sC,
                        const float* bias, int act, const ZSplit& z) {
   switch (t) {
     case Tile::k256x256:
-      return launch_tiles<256, 256, kBK, CHECK, TB, EPI, V4, KF>(s, batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC,
+      return launch_tiles<256, 256, kBK, CHECK, TB, EPI, V4>(s, batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC,
                                                              bias, act, z.nz, z.sA, z.sB, z.sC);
     case Tile::k256x128:
-      return launch_tiles<256, 128, kBK, CHECK, TB, EPI, V4, KF>(s, batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC,
+      return launch_tiles<256, 128, kBK, CHECK, TB, EPI, V4>(s, batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC,
                                                              bias, act, z.nz, z.sA, z.sB, z.sC);
     default:
-      return launch_tiles<128, 128, kBK, CHECK, TB, EPI, V4, KF>(s, batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC,
+      return launch_tiles<128, 128, kBK, CHECK, TB, EPI, V4>(s, batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC,
                                                              bias, act, z.nz, z.sA, z.sB, z.sC);
   }
 }
@@ -746,9 +648,6 @@ hipError_t launch_tile_any(int mode, Tile t, hipStream_t s, int batch, int m, in
                            long long sC, const float* bias, int act, const ZSplit& z = ZSplit{}) {
   if (mode == 0)
     return launch_tile<false, TB, EPI, false>(t, s, batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC, bias, act, z);
-  if (mode == 1 && k % kBK == 0)
-    return launch_tile<true, TB, EPI, true, true>(t, s, batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC, bias, act,
-                                                  z);
   if (mode == 1)
     return launch_tile<true, TB, EPI, true>(t, s, batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC, bias, act, z);
   return launch_tile<true, TB, EPI, false>(t, s, batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC, bias, act, z);
@@ -769,80 +668,91 @@ const char* tile_name(Tile t, int mode) {
 // an m x n partial), then sgemm_splitk_reduce sums the S partials of each
 // output in slice order (deterministic) and applies the epilogue.  Batches
 // split the same way when all of their tiles together fill less than a
-// round (4 x 512 x 512 x 4096: 64 tiles).  S is the modelled fastest:
-// rounds(tiles x S) x k-tiles per slice x the tile's k-tile time (7.4 us for
-// 256 x 256 at full rate, scaled by area / efficiency), plus the partials'
-// round trip ((2S + 1) M N floats at 5 TB/s) and a launch; S divides the
-// k-tile count, leaves at least kSplitMinKt k-tiles per slice, and its
-// partials fit the cap.  The plan is made against a fixed cap, not the
-// workspace at hand, so a shape always rounds the same way through
-// bch_sgemm; bch_sgemm_noalloc plans against its 16 MiB scratch and can take
-// fewer slices (within tolerance of bch_sgemm).  Several rounds of slices
-// can beat one part-filled round: 128 x 11008 x 4096 on 86 tiles of 128 x
-// 128 takes 8 slices in 3 rounds rather than 2 in one.  Measured at 1024^3
-// (64 tiles of 128 x 128): 64.8 us on 64 CUs without the split.
+// round (4 x 512 x 512 x 4096: 64 tiles).  Tile and S are the modelled
+// fastest: the rounds' time per 32 k (below) x k-tiles per slice, plus the
+// partials' round trip ((2S + 1) M N floats at 5 TB/s), the reduce launch and
+// each further round; S divides the k-tile count, leaves at least kSplitMinKt
+// k-tiles per slice, and its partials fit the cap.  The plan is made against
+// a fixed cap, not the workspace at hand, so a shape always rounds the same
+// way through bch_sgemm; bch_sgemm_noalloc plans against its 16 MiB scratch
+// and can take fewer slices (within tolerance of bch_sgemm).  Measured (one
+// box, us): 512 x 4096 x 11008 as 256 x 128 tiles in 4 slices 222 (128 x 128 in
+// 2: 246, no split 381), 512 x 11008 x 4096 as 256 x 256 in 2 245 (256 x 128
+// unsplit 262), 1024 x 1024 x 4096 as 128 x 128 in 4 60 (64 x 64 unsplit 76).
 constexpr size_t kSplitWsMax = (size_t)256 << 20;
 constexpr size_t kSplitWsSmall = (size_t)16 << 20;  // bch_sgemm_noalloc's fixed scratch
 constexpr int kSplitMinKt = 8;  // k-tiles per slice at least
+constexpr double kTileFixedUs = 3.0;    // an unsplit launch's prologue and stores
+constexpr double kSplitBytesUs = 5e6;   // the partials' round trip
+constexpr double kSplitRoundUs = 1.5;   // a further round's prologue and stores
+constexpr double kSplitFixedUs = 5.0;   // the reduce launch
 
-int split_slices(int batch, int m, int n, int k, size_t cap = kSplitWsMax, double* cost_us = nullptr) {
-  if (batch < 1 || k <= 0 || k % kBK != 0) return 1;
+struct SplitPlan {
+  Tile t = Tile::k128x128;
+  int S = 1;          // slices; 1: no split
+  double us = 0.0;    // modelled time
+};
+
+SplitPlan split_plan(int batch, int m, int n, int k, size_t cap = kSplitWsMax) {
+  SplitPlan p;
+  if (batch < 1 || k <= 0 || k % kBK != 0) return p;
   const long long cu = bch::device_cu_count();
-  const Tile t = pick_tile(batch, m, n);
-  const long long tiles =
-      (long long)batch * ((m + tile_m(t) - 1) / tile_m(t)) * ((n + tile_n(t) - 1) / tile_n(t));
-  if (tiles >= cu) return 1;  // whole rounds: the data-parallel tiling or the hybrid plan
-  double eff = 1.0;
-  for (const TileOpt& o : kTileOpts)
-    if (o.t == t) eff = o.eff;
-  const double tk = 7.4 * tile_m(t) * tile_n(t) / 65536.0 / eff;  // us per k-tile of this tile
+  p.t = pick_tile(batch, m, n);
   const double mn = (double)batch * m * n * sizeof(float);
   const int nk = k / kBK;
-  double best = nk * tk;
-  int bs = 1;
-  for (int sl = 2; nk / sl >= kSplitMinKt; ++sl) {
-    if (nk % sl != 0) continue;
-    if ((size_t)sl * batch * m * n * sizeof(float) > cap) break;
-    const double cost = (double)((tiles * sl + cu - 1) / cu) * (nk / sl) * tk + (2.0 * sl + 1.0) * mn / 5e6 + 2.0;
-    if (cost < best) {
-      best = cost;
-      bs = sl;
+  // a part-filled round stays near `idle` up to half of the CUs (256 x 256: 64, 128 and 172
+  // workgroups 3.2, 3.26 and 3.4 us per 32 k; 256 x 128: 1.85, 1.93 and 2.05)
+  auto kt_us = [&](const TileOpt& o, long long wgs) {
+    const double r = (double)(wgs % cu) / (double)cu;
+    return (double)(wgs / cu) * o.full + (r > 0.0 ? o.idle + (o.full - o.idle) * r * r * r * r : 0.0);
+  };
+  for (const TileOpt& o : kTileOpts)
+    if (o.t == p.t) {
+      const long long tiles = tile_count(o, batch, m, n);
+      if (tiles >= cu) return p;  // whole rounds: the data-parallel tiling or the hybrid plan
+      p.us = nk * kt_us(o, tiles) + kTileFixedUs;
+    }
+  for (const TileOpt& o : kTileOpts) {
+    const long long tiles = tile_count(o, batch, m, n);
+    for (int sl = 2; nk / sl >= kSplitMinKt; ++sl) {
+      if (nk % sl != 0) continue;
+      if ((size_t)sl * batch * m * n * sizeof(float) > cap) break;
+      const long long rounds = (tiles * sl + cu - 1) / cu;
+      const double us = (nk / sl) * kt_us(o, tiles * sl) + kSplitRoundUs * (double)(rounds - 1) +
+                        (2.0 * sl + 1.0) * mn / kSplitBytesUs + kSplitFixedUs;
+      if (us < p.us) {
+        p.t = o.t;
+        p.S = sl;
+        p.us = us;
+      }
     }
   }
-  if (cost_us) *cost_us = best;
-  return bs;
+  return p;
+}
+
+int split_slices(int batch, int m, int n, int k, size_t cap = kSplitWsMax) {
+  return split_plan(batch, m, n, k, cap).S;
 }
 
 // ---- small shapes: 64 x 64 x 64 tiles ----
-// Where the planned tiles fill less than one round, 64 x 64 tiles (each wavefront one 32 x 32
-// MFMA block; k-tiles of 64 so that a tile's loads split evenly over the 256 threads) put 16x
-// the workgroups of the 128 x 128 tiling on the CUs, with no k split, partials or reduce
-// launch.  A 64 x 64 x 64 k-tile takes ~1.32 us at any count of tiles up to a round (256^3 to
-// 1024^3; 63% of the matrix cores' rate, against 92% for 128 x 128); two workgroups share a CU
-// (70 KB of LDS each) at ~2.29 us per k-tile of both.  Taken when its modelled time, rounds x
-// k-tiles x that time, is under 0.9 of the split-K plan's; unguarded loads only (m, n, k
-// multiples of 64, aligned operands), else the usual path.  Same box, two runs each, against
-// the split-K plan: 256^3 19.4 -> 8.8 us, 512^3 23.0 -> 13.9, 768^3 25.8 -> 19.3, 1024^3 28.3
-// -> 24.4, 1024 x 2048 x 1024 43.9 -> 40.1 (two per CU); where split-K stays ahead the model
-// keeps it (1024 x 1024 x 4096 74 against 89 us, 1024 x 1024 x 2048 43.5 against 47.6, 512 x
-// 1024 x 2048 28.7 against 46.9).
+// Where the planned tiles fill less than one round, 64 x 64 tiles put 4 to 16 times the
+// workgroups on the CUs, with no k split, partials or reduce launch.  A pass is 64 k deep; the
+// two halves of its k go to two sets of four wavefronts, whose sums meet in LDS at the end, so a
+// SIMD always has a second wavefront to run while one converts, stores or waits.  Against four
+// wavefronts and passes of 32 (same box, us): 256^3 8.3 -> 7.05, 512^3 13.7 -> 10.6, 1024^3 25.6 ->
+// 20.6, 1024 x 1024 x 4096 95 -> 76.  (More loads in flight, 2 or 4 passes, changed nothing.)  A
+// 64-k pass takes 1.0-1.2 us whatever the tile count up to a round.  Taken when the modelled time
+// is under the split plan's; unguarded loads only (m, n, k multiples of 64, aligned operands).
 constexpr int kSmallBK = 64;
-constexpr double kSmallKtUs = 1.32;   // one workgroup per CU
-constexpr double kSmallKt2Us = 2.29;  // two per CU, both k-tiles
+constexpr double kSmallKtUs = 1.12;
 
 bool small_tile_plan(int batch, int m, int n, int k) {
   if (batch < 1 || m % 64 != 0 || n % 64 != 0 || k <= 0 || k % kSmallBK != 0) return false;
+  const SplitPlan p = split_plan(batch, m, n, k);
+  if (p.us == 0.0) return false;  // whole rounds of the other tiles
   const long long cu = bch::device_cu_count();
-  const Tile t = pick_tile(batch, m, n);
-  const long long tiles =
-      (long long)batch * ((m + tile_m(t) - 1) / tile_m(t)) * ((n + tile_n(t) - 1) / tile_n(t));
-  if (tiles >= cu) return false;
-  double cur = 0.0;
-  split_slices(batch, m, n, k, kSplitWsMax, &cur);
   const long long t64 = (long long)batch * (m / 64) * (n / 64);
-  const double nk = k / kSmallBK;
-  const double small = t64 <= cu ? nk * kSmallKtUs : (double)((t64 + 2 * cu - 1) / (2 * cu)) * nk * kSmallKt2Us;
-  return small < 0.9 * cur;
+  return (double)((t64 + cu - 1) / cu) * (k / kSmallBK) * kSmallKtUs < p.us;
 }
 
 bool small_tile_ok(int batch, int m, int n, int k, const float* A, int lda, long long sA, const float* B, int ldb,
@@ -904,8 +814,8 @@ __global__ __launch_bounds__(256) void sgemm_splitk_reduce(int M, int N, int S, 
 // in the kernel.  Every slice covers the same k-tiles of neighbouring tiles,
 // so the slices of a round share A and B panels in L2 the way whole tiles do.
 // The plan is modelled like the tile choice (k-tiles x tile area /
-// efficiency per round; the partials' HBM traffic at 5 TB/s, one 256 x 256
-// k-tile taking 7.4 us) and used when it beats the best data-parallel tiling
+// efficiency per round; the partials' HBM traffic at 6.3 TB/s, one 256 x 256
+// k-tile taking kTileKtUs) and used when it beats the best data-parallel tiling
 // by 3%.  It needs K a multiple of 32 and unguarded or float4-guarded loads;
 // without the workspace (up to kHybWsMax) the data-parallel tiling runs.
 constexpr size_t kHybWsMax = (size_t)256 << 20;
@@ -918,7 +828,7 @@ struct HybPlan {
 size_t hyb_bytes(const HybPlan& h) { return (size_t)h.S * h.r * tile_m(h.t) * tile_n(h.t) * sizeof(float); }
 
 // cost_us (nullable): the modelled time of what the tile path then runs, the hybrid plan or the
-// best data-parallel tiling (7.4 us per 256 x 256 k-tile)
+// best data-parallel tiling
 bool hyb_plan(int batch, int m, int n, int k, HybPlan& out, double* cost_us = nullptr) {
   if (batch != 1 || k <= 0 || k % kBK != 0 || split_slices(batch, m, n, k) > 1) return false;
   const long long cu = bch::device_cu_count();
@@ -940,7 +850,7 @@ bool hyb_plan(int batch, int m, int n, int k, HybPlan& out, double* cost_us = nu
         break;
       }
     if (S == 0) continue;
-    const double cost = (double)(R * nk + nk / S) * per + (2.0 * S + 1.0) * r * (o.bm * o.bn / 65536.0) * 0.00709 + 0.3;
+    const double cost = (double)(R * nk + nk / S) * per + (2.0 * S + 1.0) * r * (o.bm * o.bn / 65536.0) * 0.009 + 0.45;
     if (!found || cost < best) {
       found = true;
       best = cost;
@@ -952,7 +862,7 @@ bool hyb_plan(int batch, int m, int n, int k, HybPlan& out, double* cost_us = nu
     }
   }
   const bool use = found && best < 0.97 * best_dp;
-  if (cost_us) *cost_us = 7.4 * (use ? best : best_dp);
+  if (cost_us) *cost_us = kTileKtUs * (use ? best : best_dp);
   return use;
 }
 
@@ -960,7 +870,8 @@ bool hyb_plan(int batch, int m, int n, int k, HybPlan& out, double* cost_us = nu
 // data-parallel tiling, whichever the tile path takes (given its workspace).
 double tile_path_cost_us(int m, int n, int k) {
   double c = 0.0;
-  if (split_slices(1, m, n, k, kSplitWsMax, &c) > 1) return c;
+  const SplitPlan sp = split_plan(1, m, n, k);
+  if (sp.S > 1) return sp.us;
   HybPlan h;
   if (k > 0 && k % kBK == 0) {
     hyb_plan(1, m, n, k, h, &c);
@@ -971,7 +882,7 @@ double tile_path_cost_us(int m, int n, int k) {
   double best = 0.0;
   for (const TileOpt& o : kTileOpts) {
     const long long T = (long long)((m + o.bm - 1) / o.bm) * ((n + o.bn - 1) / o.bn);
-    const double t = (double)((T + cu - 1) / cu) * ((k + kBK - 1) / kBK) * 7.4 * o.bm * o.bn / 65536.0 / o.eff;
+    const double t = (double)((T + cu - 1) / cu) * ((k + kBK - 1) / kBK) * kTileKtUs * o.bm * o.bn / 65536.0 / o.eff;
     if (best == 0.0 || t < best) best = t;
   }
   return best;
@@ -990,11 +901,11 @@ double tile_path_cost_us(int m, int n, int k) {
 // plan; the split runs along rows or columns, with j from 1 to the whole rounds available.
 // Only the first level splits: the rest is planned without the mixed plan.
 // The second launch's fixed cost in the model: its prologue, the first launch's last C stores
-// that nothing overlaps, and the gap between the launches.  At 16 us the model picks, among
+// that nothing overlaps, and the gap between the launches.  At 16 us (10 us at the present rates) the model picked, among
 // 26 shapes measured both ways (K 1024 and 4096), every one that gained (1.1-6.0%) at K 4096
 // and leaves out the two that lost (6144 x 6144 x 1024 -2.9%, 4100 x 4100 x 1024 -1.2%); two
 // it still takes at K 1024 measured within 0.4% either way.
-constexpr double kMixFixedUs = 16.0;
+constexpr double kMixFixedUs = 10.0;
 
 struct MixPlan {
   int axis = -1;  // 0: rows [0, split) first; 1: columns [0, split) first
@@ -1016,7 +927,7 @@ bool mix_plan(int batch, int m, int n, int k, MixPlan& out) {
       const long long c = j * cu / across;  // whole tile rows (columns) that fit j rounds
       if (c < 1 || c >= along) continue;
       const int split = (int)(256 * c);
-      const double first = (double)((c * across + cu - 1) / cu) * nk * 7.4;
+      const double first = (double)((c * across + cu - 1) / cu) * nk * kTileKtUs;
       const double rest = axis == 0 ? tile_path_cost_us(m - split, n, k) : tile_path_cost_us(m, n - split, k);
       const double cost = first + rest + kMixFixedUs;
       if (cost < best) {
@@ -1098,9 +1009,9 @@ template <bool TB, bool EPI>
 hipError_t launch_hyb(int mode, const HybPlan& h, hipStream_t s, int m, int n, int k, const float* A, int lda,
                       const float* B, int ldb, float* C, int ldc, const float* bias, int act, float* P) {
 #define BCH_HYB(BM_, BN_)                                                                                         \
-  (mode == 0 ? launch_hyb_tiles<BM_, BN_, kBK, false, TB, EPI, false, false>(s, m, n, k, A, lda, B, ldb, C, ldc,  \
+  (mode == 0 ? launch_hyb_tiles<BM_, BN_, kBK, false, TB, EPI, false>(s, m, n, k, A, lda, B, ldb, C, ldc,  \
                                                                             bias, act, h.ndp, h.r, h.S, h.kt, P) \
-             : launch_hyb_tiles<BM_, BN_, kBK, true, TB, EPI, true, true>(s, m, n, k, A, lda, B, ldb, C, ldc, bias, \
+             : launch_hyb_tiles<BM_, BN_, kBK, true, TB, EPI, true>(s, m, n, k, A, lda, B, ldb, C, ldc, bias, \
                                                                          act, h.ndp, h.r, h.S, h.kt, P))
   hipError_t e = h.t == Tile::k256x256   ? BCH_HYB(256, 256)
                  : h.t == Tile::k256x128 ? BCH_HYB(256, 128)
@@ -1144,11 +1055,12 @@ static const char* tile_path_name(int m, int n, int k, bool allow_mix) {
     return name.c_str();
   }
   if (small_tile_plan(1, m, n, k)) return "sgemm_mfma_kernel<64,64,64,false>";
-  const Tile t = pick_tile(1, m, n);
+  const SplitPlan sp = split_plan(1, m, n, k);
+  const Tile t = sp.S > 1 ? sp.t : pick_tile(1, m, n);
   // with lda = k and ldb = n, and 16-byte aligned operands
   const bool check = !(m % tile_m(t) == 0 && n % tile_n(t) == 0 && k % kBK == 0 && k % 4 == 0 && n % 4 == 0);
   const bool v4 = k >= 4 && k % 4 == 0 && n % 4 == 0;
-  if (split_slices(1, m, n, k) > 1) {  // slices of 32-k tiles (k % 32 == 0)
+  if (sp.S > 1) {  // slices of 32-k tiles (k % 32 == 0)
     const bool fast = m % tile_m(t) == 0 && n % tile_n(t) == 0 && n % 4 == 0;
     static const char* const split_names[3][3] = {
         {"sgemm_mfma_kernel<256,256,32,false>+sgemm_splitk_reduce", "sgemm_mfma_kernel<256,256,32,true,v4>+sgemm_splitk_reduce",
@@ -1265,11 +1177,12 @@ hipError_t launch_tile_path(hipStream_t s, bool transb, int batch, int m, int n,
                   : (epi ? BCH_SMALL(false, true) : BCH_SMALL(false, false));
 #undef BCH_SMALL
   }
-  const Tile t = pick_tile(batch, m, n);
-  int sl = split_slices(batch, m, n, k);
+  SplitPlan sp = split_plan(batch, m, n, k);
   const size_t pbytes = (size_t)batch * m * n * sizeof(float);  // one slice's partials, every batch
-  if (sl > 1 && (ws == nullptr || ws_bytes < (size_t)sl * pbytes))
-    sl = ws == nullptr ? 1 : split_slices(batch, m, n, k, ws_bytes);  // fewer slices within the scratch at hand
+  if (sp.S > 1 && (ws == nullptr || ws_bytes < (size_t)sp.S * pbytes))
+    sp = split_plan(batch, m, n, k, ws == nullptr ? 0 : ws_bytes);  // fewer slices within the scratch at hand
+  const Tile t = sp.S > 1 ? sp.t : pick_tile(batch, m, n);
+  const int sl = sp.S;
   if (sl > 1 && ws != nullptr && ws_bytes >= (size_t)sl * pbytes) {
     // batch b, slice j (grid.z): A + b sA + j kc, B + b sB + j kc rows (columns for [n][k]),
     // into P[b][j] (m x n)

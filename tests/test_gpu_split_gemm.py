@@ -1,0 +1,114 @@
+"""The tile GEMM's three-part bf16 products (bch_sgemm, bch_sgemm_ex) where they can go wrong:
+operands whose parts cannot stand for them (infinities, NaN, magnitudes at both ends of the f32
+range), remainders of k at every tile and load mode, and misaligned rows."""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from barracuda_amd import Tensor
+
+pytestmark = pytest.mark.gpu
+
+
+def _ex(dev, a, b, transb, lda=None, ldb=None, a_off=0, b_off=0):
+    """bch_sgemm_ex on copies of a and b with the given leading dimensions and start offsets."""
+    m, k = a.shape
+    n = b.shape[0] if transb else b.shape[1]
+    lda, ldb = lda or k, ldb or b.shape[1]
+
+    def put(x, ld, off):
+        buf = np.zeros(off + x.shape[0] * ld, dtype=np.float32)
+        buf[off:].reshape(x.shape[0], ld)[:, :x.shape[1]] = x
+        return Tensor.from_data(buf, [buf.size], dev)
+
+    ta, tb, tc = put(a, lda, a_off), put(b, ldb, b_off), Tensor.empty([m, n], dev)
+    dev.check(dev._lib.bch_sgemm_ex(dev.ctx, transb, m, n, k, C.c_void_p(ta.ptr + 4 * a_off), lda,
+                                    C.c_void_p(tb.ptr + 4 * b_off), ldb, None, 0, C.c_void_p(tc.ptr), n), "linear")
+    return tc.to_numpy()
+
+
+def _check_f32_sums(got, a, b):
+    """The bound of a sum of k products in f32: k 2^-24 of the sum of their magnitudes, and half
+    the smallest subnormal a term."""
+    k = a.shape[1]
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    bound = k * 2.0**-24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)) + k * 2.0**-150
+    worst = float(np.max(np.abs(got - want) / bound))
+    assert worst <= 1.0, worst
+
+
+# (m, n): 64 x 64 tiles, 128 x 128 tiles, 256 x 128 tiles, 256 x 256 tiles
+TILES = [(192, 128), (200, 136), (8190, 1020), (4095, 4090)]
+
+
+@pytest.mark.parametrize("transb", [0, 1])
+@pytest.mark.parametrize("m,n", TILES)
+@pytest.mark.parametrize("k", [1, 7, 15, 16, 17, 31, 32, 33, 47, 65, 95])
+def test_k_remainders_exact(dev, m, n, k, transb):
+    """Integers below 2^12: products below 2^24 and their sums are exact in f32, so three parts
+    have to give every bit, whatever the remainder of k."""
+    print(f"k remainder m={m} n={n} k={k} transb={transb}", flush=True)
+    rng = np.random.default_rng(m + n + k)
+    a = rng.integers(-400, 401, (m, k)).astype(np.float32)
+    b = rng.integers(-400, 401, (n, k) if transb else (k, n)).astype(np.float32)
+    want = a.astype(np.float64) @ (b.T if transb else b).astype(np.float64)
+    assert np.abs(want).max() < 2**24
+    assert np.array_equal(_ex(dev, a, b, transb), want.astype(np.float32))
+
+
+@pytest.mark.parametrize("m,n,k,a_off,b_off,lda_pad,ldb_pad", [
+    (260, 300, 100, 1, 3, 0, 0), (260, 300, 100, 0, 0, 1, 3), (300, 260, 67, 2, 1, 2, 2), (128, 128, 64, 1, 1, 0, 0)])
+@pytest.mark.parametrize("transb", [0, 1])
+def test_misaligned_rows_exact(dev, m, n, k, a_off, b_off, lda_pad, ldb_pad, transb):
+    print(f"misaligned m={m} n={n} k={k} transb={transb}", flush=True)
+    rng = np.random.default_rng(k)
+    a = rng.integers(-400, 401, (m, k)).astype(np.float32)
+    b = rng.integers(-400, 401, (n, k) if transb else (k, n)).astype(np.float32)
+    want = (a.astype(np.float64) @ (b.T if transb else b).astype(np.float64)).astype(np.float32)
+    assert np.array_equal(_ex(dev, a, b, transb, k + lda_pad, b.shape[1] + ldb_pad, a_off, b_off), want)
+
+
+@pytest.mark.parametrize("m,n,k", [(128, 128, 64), (200, 136, 100), (300, 260, 4096), (2048, 2048, 96)])
+@pytest.mark.parametrize("transb", [0, 1])
+def test_non_finite_operands(dev, m, n, k, transb):
+    """Infinities and NaN give what IEEE arithmetic gives: an infinite a reaches its row with the
+    sign of each b (NaN where b is zero or infinities meet), and no other row changes."""
+    print(f"non-finite m={m} n={n} k={k} transb={transb}", flush=True)
+    rng = np.random.default_rng(m + k)
+    a = rng.integers(-8, 9, (m, k)).astype(np.float32)
+    b = rng.integers(-8, 9, (k, n)).astype(np.float32)
+    a[3, 5], a[70, 0], a[100, k - 1] = np.inf, -np.inf, np.nan
+    b[7, 11], b[k - 1, 90] = -np.inf, np.nan
+    with np.errstate(invalid="ignore"):
+        want = np.einsum("mk,kn->mn", a.astype(np.float64), b.astype(np.float64)) if k <= 100 else None
+        if want is None:
+            want = a.astype(np.float64) @ b.astype(np.float64)
+    got = _ex(dev, a, np.ascontiguousarray(b.T) if transb else b, transb)
+    assert np.array_equal(got, want.astype(np.float32), equal_nan=True)
+
+
+@pytest.mark.parametrize("sa,sb", [(2.0**-120, 1.0), (2.0**-120, 2.0**100), (1.0, 2.0**-126), (2.0**-70, 2.0**-60),
+                                   (2.0**60, 2.0**56), (2.0**-149, 2.0**120), (2.0**124, 2.0**-20)])
+def test_ends_of_the_range(dev, sa, sb):
+    """Rows scaled by powers of two to both ends of the f32 range, subnormals among them: the
+    f32 product to 2^-24 a term (and half the smallest subnormal), as the f32 instruction gives."""
+    print(f"range sa={sa} sb={sb}", flush=True)
+    m, n, k = 160, 144, 128
+    rng = np.random.default_rng(5)
+    a = (rng.standard_normal((m, k)) * sa).astype(np.float32)
+    b = (rng.standard_normal((k, n)) * sb).astype(np.float32)
+    _check_f32_sums(_ex(dev, a, b, 0), a, b)
+
+
+def test_one_huge_element_in_a_row(dev):
+    """Parts keep each element's own exponent: a row with one element 2^60 times the others, and a
+    zero in B against it, still has the others' product to f32 accuracy."""
+    m, n, k = 256, 256, 512
+    rng = np.random.default_rng(9)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    a[:, 17] *= 2.0**60
+    b[17, :] = 0.0
+    _check_f32_sums(_ex(dev, a, b, 0), a, b)
