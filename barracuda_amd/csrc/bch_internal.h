@@ -301,6 +301,15 @@ hipError_t launch_sdpa_strided(hipStream_t s, int B, int H, int Hkv, int Sq,
                                const float* q, const float* k,
                                const float* v, float* o,
                                const SdpaStrides& st);
+// Few query rows over many keys (at most 16 rows a head, 128 a key/value head, 128 keys or more,
+// non-causal, D <= 128 and a multiple of 4, 16-byte aligned rows): split over the keys, the
+// partial results in ws; unsplit when ws_bytes is less than sdpa_decode_workspace_bytes.
+bool sdpa_decode_applies(int B, int H, int Hkv, int Sq, int Skv, int D, int causal, const float* q, const float* k,
+                         const float* v, const SdpaStrides& st);
+size_t sdpa_decode_workspace_bytes(int B, int H, int Hkv, int Sq, int Skv, int D);
+hipError_t launch_sdpa_decode(hipStream_t s, int B, int H, int Hkv, int Sq, int Skv, int D, float scale,
+                              const float* q, const float* k, const float* v, float* o, const SdpaStrides& st,
+                              void* ws, size_t ws_bytes);
 // D > kSdpaFusedMaxD: scores materialised one query chunk at a time (GEMM,
 // scaled and masked row softmax, GEMM) in ws, which must hold
 // sdpa_wide_workspace_bytes(...) bytes (q_row, k_row: the row strides of q

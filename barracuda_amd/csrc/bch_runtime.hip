@@ -767,6 +767,20 @@ bch_status sdpa_run(bch_ctx* ctx, int B, int H, int Hkv, int Sq, int Skv, int D,
                     const float* q, const float* k, const float* v, float* o, const bch::SdpaStrides& s) {
   bch_status st = use(ctx);
   if (st != BCH_OK) return st;
+  if (bch::sdpa_decode_applies(B, H, Hkv, Sq, Skv, D, causal, q, k, v, s)) {
+    // split over the keys where the workspace holds the partial results; else (it may not grow
+    // under capture, or there is no memory) one workgroup per row block runs all keys
+    const size_t need = bch::sdpa_decode_workspace_bytes(B, H, Hkv, Sq, Skv, D);
+    if (need > ctx->ws_bytes && !capturing(ctx)) {
+      st = ensure_ws(ctx, need);
+      if (st != BCH_OK && st != BCH_E_OOM) return st;
+      if (st == BCH_E_OOM) (void)hipGetLastError();
+    }
+    return from_hip(ctx,
+                    bch::launch_sdpa_decode(ctx->stream, B, H, Hkv, Sq, Skv, D, scale, q, k, v, o, s, ctx->ws,
+                                            ctx->ws_bytes),
+                    "attention launch");
+  }
   if (D <= bch::kSdpaFusedMaxD)
     return from_hip(ctx, bch::launch_sdpa_strided(ctx->stream, B, H, Hkv, Sq, Skv, D, scale, causal, q, k, v, o, s),
                     "attention launch");

@@ -298,7 +298,9 @@ bch_status bch_softmax_axis(bch_ctx *ctx, long long outer, long long axis,
  * causal ops take one seq_len).  Non-causal Sq may differ from Skv
  * (cross-attention).  Any D >= 1, as the reference's ops take: up to
  * D = 256 one fused kernel that never materialises the Sq x Skv score
- * matrix and uses no scratch; above D = 256 the scores of one chunk of
+ * matrix and uses no scratch (a few query rows over 128 keys or more, D <=
+ * 128: split over the keys, the partial results in the context's workspace,
+ * or unsplit where that may not grow: under capture, or out of memory); above D = 256 the scores of one chunk of
  * query rows at a time (at most 256 MiB) go through the context's
  * workspace (grown on demand, like the GEMM's) in three steps -- Q K^T,
  * scaled and masked row softmax, P V -- on the MFMA GEMM.  Replaces Attention::execute (ops/attention/
