@@ -89,23 +89,27 @@ __device__ __forceinline__ unsigned bf16_pack(float x, float y) {
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
   return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x, y}), bf16x2));
 }
+// Parts of two floats into element e of p[0..2] (x and y are left as remainders); returns
+// max(m, |x|, |y|) (NaN left out).
+__device__ __forceinline__ float split2(float& x, float& y, u32x4 (&p)[3], int e, float m) {
+  m = fmaxf(m, fmaxf(fabsf(x), fabsf(y)));
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    p[q][e] = bf16_pack(x, y);
+    if (q < 2) {
+      x -= __builtin_bit_cast(float, p[q][e] << 16);
+      y -= __builtin_bit_cast(float, p[q][e] & 0xffff0000u);
+    }
+  }
+  return m;
+}
 // Parts p[0..2] of eight floats; returns max(m, |v[0]|, ..., |v[7]|) (NaN left out).
 __device__ __forceinline__ float split8(const float (&v)[8], u32x4 (&p)[3], float m) {
-  float x[8];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] = v[e];
-#pragma unroll
-  for (int e = 0; e < 8; e += 2) m = fmaxf(m, fmaxf(fabsf(x[e]), fabsf(x[e + 1])));
-#pragma unroll
-  for (int q = 0; q < 3; ++q)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      p[q][e] = bf16_pack(x[2 * e], x[2 * e + 1]);
-      if (q < 2) {
-        x[2 * e] -= __builtin_bit_cast(float, p[q][e] << 16);
-        x[2 * e + 1] -= __builtin_bit_cast(float, p[q][e] & 0xffff0000u);
-      }
-    }
+  for (int e = 0; e < 4; ++e) {
+    float x = v[2 * e], y = v[2 * e + 1];
+    m = split2(x, y, p, e, m);
+  }
   return m;
 }
 __device__ __forceinline__ f32x16 bf16_mm(u32x4 a, u32x4 b, f32x16 c) {
@@ -282,11 +286,8 @@ hipError_t launch_head_permute(hipStream_t s, bool concat, int B, int S, int H, 
 // Device-to-device copy (16-byte path when aligned).
 hipError_t launch_copy(hipStream_t s, void* dst, const void* src, size_t bytes);
 
-// Fused attention forward over [B,H,S,D].
-hipError_t launch_sdpa(hipStream_t s, int B, int H, int Sq, int Skv, int D,
-                       float scale, int causal, const float* q,
-                       const float* k, const float* v, float* o);
-// Strided form: per tensor (batch, head, row) strides in elements, the head
+// Fused attention forward.
+// Per tensor (batch, head, row) strides in elements, the head
 // dimension contiguous; key/value head of query head h is h / (H / Hkv).
 struct SdpaLayout {
   long long batch, head, row;
@@ -300,7 +301,18 @@ hipError_t launch_sdpa_strided(hipStream_t s, int B, int H, int Hkv, int Sq,
                                int Skv, int D, float scale, int causal,
                                const float* q, const float* k,
                                const float* v, float* o,
-                               const SdpaStrides& st);
+                               const SdpaStrides& st, void* ws,
+                               size_t ws_bytes);
+// ws of launch_sdpa_strided (the results of split keys, where query blocks do not fill the chip);
+// with less it runs unsplit.
+size_t sdpa_fwd_workspace_bytes(int B, int H, int Sq, int Skv, int D);
+// Results of one split of the keys for `rows` queries of a head: rows x D floats of unnormalised O,
+// then rows x (reference max, sum).
+__host__ __device__ inline long long sdpa_part_floats(int rows, int D) { return (long long)rows * (D + 2); }
+// o = the splits' results added in split order and normalised; part[b * Hkv + hk][split] holds
+// (H / Hkv) * Sq rows.
+hipError_t launch_sdpa_combine(hipStream_t s, int B, int H, int Hkv, int Sq, int D, int splits, const float* part,
+                               float* o, const SdpaLayout& lo);
 // Few query rows over many keys (at most 16 rows a head, 128 a key/value head, 128 keys or more,
 // non-causal, D <= 128 and a multiple of 4, 16-byte aligned rows): split over the keys, the
 // partial results in ws; unsplit when ws_bytes is less than sdpa_decode_workspace_bytes.

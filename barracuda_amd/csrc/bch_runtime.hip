@@ -767,23 +767,24 @@ bch_status sdpa_run(bch_ctx* ctx, int B, int H, int Hkv, int Sq, int Skv, int D,
                     const float* q, const float* k, const float* v, float* o, const bch::SdpaStrides& s) {
   bch_status st = use(ctx);
   if (st != BCH_OK) return st;
-  if (bch::sdpa_decode_applies(B, H, Hkv, Sq, Skv, D, causal, q, k, v, s)) {
-    // split over the keys where the workspace holds the partial results; else (it may not grow
-    // under capture, or there is no memory) one workgroup per row block runs all keys
-    const size_t need = bch::sdpa_decode_workspace_bytes(B, H, Hkv, Sq, Skv, D);
+  if (D <= bch::kSdpaFusedMaxD) {
+    // the keys are split over workgroups where the workspace holds the partial results; else (it
+    // may not grow under capture, or there is no memory) each workgroup runs all of its keys
+    const bool decode = bch::sdpa_decode_applies(B, H, Hkv, Sq, Skv, D, causal, q, k, v, s);
+    const size_t need = decode ? bch::sdpa_decode_workspace_bytes(B, H, Hkv, Sq, Skv, D)
+                               : bch::sdpa_fwd_workspace_bytes(B, H, Sq, Skv, D);
     if (need > ctx->ws_bytes && !capturing(ctx)) {
       st = ensure_ws(ctx, need);
       if (st != BCH_OK && st != BCH_E_OOM) return st;
       if (st == BCH_E_OOM) (void)hipGetLastError();
     }
     return from_hip(ctx,
-                    bch::launch_sdpa_decode(ctx->stream, B, H, Hkv, Sq, Skv, D, scale, q, k, v, o, s, ctx->ws,
-                                            ctx->ws_bytes),
+                    decode ? bch::launch_sdpa_decode(ctx->stream, B, H, Hkv, Sq, Skv, D, scale, q, k, v, o, s, ctx->ws,
+                                                     ctx->ws_bytes)
+                           : bch::launch_sdpa_strided(ctx->stream, B, H, Hkv, Sq, Skv, D, scale, causal, q, k, v, o,
+                                                      s, ctx->ws, ctx->ws_bytes),
                     "attention launch");
   }
-  if (D <= bch::kSdpaFusedMaxD)
-    return from_hip(ctx, bch::launch_sdpa_strided(ctx->stream, B, H, Hkv, Sq, Skv, D, scale, causal, q, k, v, o, s),
-                    "attention launch");
   if (s.q.row > 0x7fffffffLL || s.k.row > 0x7fffffffLL || s.v.row > 0x7fffffffLL || s.o.row > 0x7fffffffLL)
     return fail(ctx, BCH_E_UNSUPPORTED, "attention: head dimension %d > %d needs row strides below 2^31", D,
                 bch::kSdpaFusedMaxD);

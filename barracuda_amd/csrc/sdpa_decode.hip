@@ -63,9 +63,6 @@ __device__ __forceinline__ float quad_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// Partial results of one split: rows x (D floats of O), then rows x (m, l).
-__host__ __device__ inline long long part_floats(int rows, int D) { return (long long)rows * (D + 2); }
-
 // DP: 64 or 128, the head dimension rounded up; FULL: D == DP.
 template <int DP, bool FULL>
 __global__ __launch_bounds__(64 * kWaves, 2) void sdpa_decode_kernel(
@@ -240,7 +237,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void sdpa_decode_kernel(
   float* dst;
   float inv = 1.0f;
   if (splits > 1) {
-    float* p = part + ((long long)bk * splits + sp) * part_floats(rows, D);
+    float* p = part + ((long long)bk * splits + sp) * bch::sdpa_part_floats(rows, D);
     dst = p + (long long)my * D;
     if (g == 0) {
       p[(long long)rows * D + 2 * my] = m;
@@ -270,7 +267,7 @@ __global__ __launch_bounds__(64) void sdpa_combine(int H, int Hkv, int Sq, int D
   const int group = H / Hkv, rows = group * Sq;
   const int bk = blockIdx.x / rows, row = blockIdx.x % rows;
   const int bi = bk / Hkv, hk = bk - bi * Hkv;
-  const long long per = part_floats(rows, D);
+  const long long per = bch::sdpa_part_floats(rows, D);
   const float* p = part + (long long)bk * splits * per;
   const float* ml = p + (long long)rows * D + 2 * row;
   const int lane = threadIdx.x;
@@ -326,7 +323,7 @@ bool sdpa_decode_applies(int B, int H, int Hkv, int Sq, int Skv, int D, int caus
 
 size_t sdpa_decode_workspace_bytes(int B, int H, int Hkv, int Sq, int Skv, int D) {
   const DecodePlan p = plan(B, H, Hkv, Sq, Skv, true);
-  return p.splits > 1 ? sizeof(float) * (size_t)B * Hkv * p.splits * part_floats((H / Hkv) * Sq, D) : 0;
+  return p.splits > 1 ? sizeof(float) * (size_t)B * Hkv * p.splits * bch::sdpa_part_floats((H / Hkv) * Sq, D) : 0;
 }
 
 hipError_t launch_sdpa_decode(hipStream_t s, int B, int H, int Hkv, int Sq, int Skv, int D, float scale,
@@ -346,8 +343,13 @@ hipError_t launch_sdpa_decode(hipStream_t s, int B, int H, int Hkv, int Sq, int 
 #undef BCH_DECODE
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.splits == 1) return e;
-  hipLaunchKernelGGL(sdpa_combine, dim3((unsigned)(B * H * Sq)), dim3(64), 0, s, H, Hkv, Sq, D, p.splits, part, o,
-                     st.o);
+  return launch_sdpa_combine(s, B, H, Hkv, Sq, D, p.splits, part, o, st.o);
+}
+
+hipError_t launch_sdpa_combine(hipStream_t s, int B, int H, int Hkv, int Sq, int D, int splits, const float* part,
+                               float* o, const SdpaLayout& lo) {
+  hipLaunchKernelGGL(sdpa_combine, dim3((unsigned)((long long)B * H * Sq)), dim3(64), 0, s, H, Hkv, Sq, D, splits, part,
+                     o, lo);
   return hipGetLastError();
 }
 

@@ -1,0 +1,81 @@
+"""The fused attention's three-part bf16 products (D <= 128) vs the f64 oracle: every head
+dimension class, remainders of queries and keys, grids on both workgroup shapes and with split
+keys, and operands whose parts cannot stand for them."""
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import pytest
+
+from barracuda_amd import Tensor
+from oracle import bc_oracle as O
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-5  # f32 softmax and sums over N(0, 1) inputs: about 1e-6 of the largest output
+
+
+def _run(dev, q, k, v, causal):
+    t = [Tensor.from_data(x, list(x.shape), dev) for x in (q, k, v)]
+    return (t[0].causal_attention(t[1], t[2]) if causal else t[0].attention(t[1], t[2])).to_numpy()
+
+
+def _inputs(b, h, sq, skv, d):
+    rng = np.random.default_rng(b + h * 3 + sq * 7 + skv + d)
+    return (rng.standard_normal((b, h, sq, d), dtype=np.float32), rng.standard_normal((b, h, skv, d), dtype=np.float32),
+            rng.standard_normal((b, h, skv, d), dtype=np.float32))
+
+
+@pytest.mark.parametrize("b,h,sq,skv,d", [
+    (1, 1, 33, 33, 1), (1, 2, 129, 129, 7), (2, 3, 100, 100, 31), (1, 4, 256, 256, 32), (1, 3, 300, 300, 33),
+    (1, 2, 512, 512, 64), (2, 2, 257, 257, 80), (1, 2, 95, 95, 96), (1, 5, 200, 200, 97), (1, 3, 700, 700, 127),
+    (1, 4, 1024, 1024, 128), (4, 64, 256, 256, 128), (4, 64, 255, 255, 128), (4, 64, 257, 257, 72), (16, 16, 31, 31, 64)])
+def test_parts_causal_vs_f64(dev, b, h, sq, skv, d):
+    print(f"sdpa parts causal b={b} h={h} s={sq} d={d}", flush=True)
+    q, k, v = _inputs(b, h, sq, skv, d)
+    got = _run(dev, q, k, v, True)
+    heads = range(min(h, 4))
+    assert O.max_rel_err(got[:1, heads], O.sdpa_f64(*(np.ascontiguousarray(x[:1, heads]) for x in (q, k, v)), True)) <= TOL
+    assert O.max_rel_err(got[-1:, -1:], O.sdpa_f64(*(np.ascontiguousarray(x[-1:, -1:]) for x in (q, k, v)), True)) <= TOL
+    assert np.array_equal(got, _run(dev, q, k, v, True)), "not deterministic"
+
+
+@pytest.mark.parametrize("b,h,sq,skv,d", [
+    (1, 1, 17, 1, 128), (1, 2, 40, 31, 64), (1, 2, 130, 63, 40), (1, 1, 128, 4097, 128), (2, 2, 64, 1000, 96),
+    (1, 3, 300, 65, 80), (4, 64, 250, 97, 128), (4, 64, 256, 128, 64)])
+def test_parts_cross_vs_f64(dev, b, h, sq, skv, d):
+    print(f"sdpa parts cross b={b} h={h} sq={sq} skv={skv} d={d}", flush=True)
+    q, k, v = _inputs(b, h, sq, skv, d)
+    got = _run(dev, q, k, v, False)
+    for sl in (np.s_[:1, :2], np.s_[-1:, -1:]):
+        assert O.max_rel_err(got[sl], O.sdpa_f64(*(np.ascontiguousarray(x[sl]) for x in (q, k, v)), False)) <= TOL
+
+
+@pytest.mark.parametrize("sq", [300, 2048])  # split keys; whole
+def test_parts_extreme_operands(dev, sq):
+    """-inf and the type's lowest value in K mask keys, NaN or +inf scores and rows of nothing but
+    -inf give NaN rows, an infinite value reaches its column, subnormal values keep their bits."""
+    h, d = 6 if sq == 300 else 40, 64
+    q, k, v = _inputs(1, h, sq, sq, d)
+    q[..., 0] = 1.0
+    k[..., 0] = 0.0
+    k[0, 0, 100:, 0] = -np.finfo(np.float32).max
+    k[0, 1, :, 0] = -np.inf
+    k[0, 2, 37, 0] = np.inf
+    k[0, 3, ::2, 0] = -np.inf
+    v[0, 0, 5, 3] = np.inf
+    v[0, 4] *= np.float32(2.0**-130)
+    v[0, 5, :, 7] *= np.float32(2.0**-110)
+    got = _run(dev, q, k, v, False)[:, :6]
+    q, k, v = (x[:, :6].astype(np.float64) for x in (q, k, v))
+    s = (q @ k.transpose(0, 1, 3, 2)) / math.sqrt(d)
+    with np.errstate(invalid="ignore"):
+        p = np.exp(s - s.max(-1, keepdims=True))
+        want = (p / p.sum(-1, keepdims=True)) @ v
+    assert np.all(np.isinf(got[0, 0, :, 3])) and np.all(np.isnan(got[0, 1])) and np.all(np.isnan(got[0, 2]))
+    for head, cols in ((0, [0, 1, 2] + list(range(4, d))), (3, list(range(d))), (4, list(range(d))), (5, list(range(d)))):
+        x, y = got[0, head][:, cols], want[0, head][:, cols]
+        # sums of sq terms of magnitude up to the largest value of the column, and half of the
+        # smallest subnormal a term
+        bound = 2e-6 * np.abs(v[0, head][:, cols]).max(0) + sq * 2.0**-150
+        assert np.all(np.isfinite(x)) and np.all(np.abs(x - y) <= bound), head
