@@ -188,6 +188,9 @@ size_t sgemm_workspace_bytes(int batch, int m, int n, int k);
 size_t sgemm_required_workspace_bytes(int batch, int m, int n, int k);
 // Scratch of launch_sgemm_ex (the skinny paths' partials, split-K partials, or the hybrid plan's).
 size_t sgemm_ex_workspace_bytes(bool transb, int batch, int m, int n, int k, int lda, int ldb);
+// Whether a call whose workspace may not grow runs all the same, unsplit (the tile path, except
+// where its plan has always needed the workspace).
+bool sgemm_runs_without_workspace(bool transb, int batch, int m, int n, int k, int lda, int ldb);
 const char* sgemm_kernel_name(int m, int n, int k);
 // With B given as [n][k] when transb (C = A B^T), and the linear layer's
 // epilogue C = act(acc + bias[col]): bias nullable, act kActNone / kActRelu /

@@ -539,6 +539,8 @@ bch_status bch_sgemm_ex(bch_ctx* ctx, int transb, int m, int n, int k, const flo
   bch_status st = use(ctx);
   if (st != BCH_OK) return st;
   size_t wsb = bch::sgemm_ex_workspace_bytes(transb != 0, 1, m, n, k, lda, ldb);
+  if (wsb > ctx->ws_bytes && capturing(ctx) && bch::sgemm_runs_without_workspace(transb != 0, 1, m, n, k, lda, ldb))
+    wsb = 0;
   if (wsb) {
     st = ensure_ws(ctx, wsb);
     if (st != BCH_OK) return st;
@@ -565,6 +567,7 @@ bch_status bch_sgemm(bch_ctx* ctx, int m, int n, int k, const float* A, int lda,
   bch_status st = use(ctx);
   if (st != BCH_OK) return st;
   size_t wsb = bch::sgemm_workspace_bytes(1, m, n, k);
+  if (wsb > ctx->ws_bytes && capturing(ctx) && bch::sgemm_runs_without_workspace(false, 1, m, n, k, lda, ldb)) wsb = 0;
   if (wsb) {
     st = ensure_ws(ctx, wsb);
     if (st != BCH_OK) return st;
@@ -615,6 +618,7 @@ bch_status bch_sgemm_strided_batched(bch_ctx* ctx, int batch, int m, int n, int 
   bch_status st = use(ctx);
   if (st != BCH_OK) return st;
   size_t wsb = bch::sgemm_workspace_bytes(batch, m, n, k);
+  if (wsb > ctx->ws_bytes && capturing(ctx) && bch::sgemm_runs_without_workspace(false, batch, m, n, k, k, n)) wsb = 0;
   if (wsb) {
     st = ensure_ws(ctx, wsb);
     if (st != BCH_OK) return st;

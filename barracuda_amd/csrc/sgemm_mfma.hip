@@ -179,11 +179,12 @@ __global__ __launch_bounds__((Cfg<BM, BN, BK>::NT)) void sgemm_mfma_kernel(
   A += bz * sA;
   B += bz * sB;
   C += bz * sC;
-  if (gridDim.z > 1) {  // split over k: blockIdx.z is the slice (its A, B offset and partial)
+  if (gridDim.z > 1) {  // split over k: blockIdx.z is the slice (its A, B offset and partial), hy_kt deep
     const long long zz = blockIdx.z;
     A += zz * sAz;
     B += zz * sBz;
     C += zz * sCz;
+    K = min(hy_kt, K - (int)zz * hy_kt);
   }
   if constexpr (HY) {
     if (tail) {  // k-tiles hy_slice * hy_kt .. + hy_kt - 1, as a product of K = hy_kt * BK
@@ -525,7 +526,7 @@ template <int BM, int BN, int BK, bool CHECK, bool TB, bool EPI, bool V4 = false
 hipError_t launch_tiles(hipStream_t s, int batch, int m, int n, int k,
                         const float* A, int lda, long long sA, const float* B,
                         int ldb, long long sB, float* C, int ldc, long long sC,
-                        const float* bias, int act, int nz = 1, long long sAz = 0, long long sBz = 0,
+                        const float* bias, int act, int nz = 1, int kc = 0, long long sAz = 0, long long sBz = 0,
                         long long sCz = 0) {
   using G = Cfg<BM, BN, BK>;
   const int tm = (m + BM - 1) / BM, tn = (n + BN - 1) / BN;
@@ -535,7 +536,7 @@ hipError_t launch_tiles(hipStream_t s, int batch, int m, int n, int k,
   if (e != hipSuccess) return e;
   if (batch > 65535 || nz > 65535) return hipErrorInvalidValue;
   hipLaunchKernelGGL(kern, dim3(tm * tn, batch, nz), dim3(G::NT), lds, s, m, n, k,
-                     A, lda, sA, B, ldb, sB, C, ldc, sC, tm, tn, bias, act, 0, 0, 0, nullptr, sAz, sBz, sCz);
+                     A, lda, sA, B, ldb, sB, C, ldc, sC, tm, tn, bias, act, 0, 0, kc, nullptr, sAz, sBz, sCz);
   return hipGetLastError();
 }
 
@@ -620,7 +621,7 @@ bool vec4_ok(bool transb, int m, int n, int k, const float* A, int lda, long lon
 
 // k slices in grid.z (the split-K launch): slice z adds z * (sA, sB, sC) to the batch's operands
 struct ZSplit {
-  int nz = 1;
+  int nz = 1, kc = 0;  // slices, their depth (the last one takes what is left)
   long long sA = 0, sB = 0, sC = 0;
 };
 
@@ -631,13 +632,13 @@ hipError_t launch_tile(Tile t, hipStream_t s, int batch, int m, int n, int k, co
   switch (t) {
     case Tile::k256x256:
       return launch_tiles<256, 256, kBK, CHECK, TB, EPI, V4>(s, batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC,
-                                                             bias, act, z.nz, z.sA, z.sB, z.sC);
+                                                             bias, act, z.nz, z.kc, z.sA, z.sB, z.sC);
     case Tile::k256x128:
       return launch_tiles<256, 128, kBK, CHECK, TB, EPI, V4>(s, batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC,
-                                                             bias, act, z.nz, z.sA, z.sB, z.sC);
+                                                             bias, act, z.nz, z.kc, z.sA, z.sB, z.sC);
     default:
       return launch_tiles<128, 128, kBK, CHECK, TB, EPI, V4>(s, batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC,
-                                                             bias, act, z.nz, z.sA, z.sB, z.sC);
+                                                             bias, act, z.nz, z.kc, z.sA, z.sB, z.sC);
   }
 }
 
@@ -671,8 +672,8 @@ const char* tile_name(Tile t, int mode) {
 // round (4 x 512 x 512 x 4096: 64 tiles).  Tile and S are the modelled
 // fastest: the rounds' time per 32 k (below) x k-tiles per slice, plus the
 // partials' round trip ((2S + 1) M N floats at 5 TB/s), the reduce launch and
-// each further round; S divides the k-tile count, leaves at least kSplitMinKt
-// k-tiles per slice, and its partials fit the cap.  The plan is made against
+// each further round; a slice has at least kSplitMinKt k-tiles (the last one
+// what is left, the remainder of K too), and the partials fit the cap.  The plan is made against
 // a fixed cap, not the workspace at hand, so a shape always rounds the same
 // way through bch_sgemm; bch_sgemm_noalloc plans against its 16 MiB scratch
 // and can take fewer slices (within tolerance of bch_sgemm).  Measured (one
@@ -681,7 +682,7 @@ const char* tile_name(Tile t, int mode) {
 // unsplit 262), 1024 x 1024 x 4096 as 128 x 128 in 4 60 (64 x 64 unsplit 76).
 constexpr size_t kSplitWsMax = (size_t)256 << 20;
 constexpr size_t kSplitWsSmall = (size_t)16 << 20;  // bch_sgemm_noalloc's fixed scratch
-constexpr int kSplitMinKt = 8;  // k-tiles per slice at least
+constexpr int kSplitMinKt = 4;  // k-tiles per slice at least
 constexpr double kTileFixedUs = 3.0;    // an unsplit launch's prologue and stores
 constexpr double kSplitBytesUs = 5e6;   // the partials' round trip
 constexpr double kSplitRoundUs = 1.5;   // a further round's prologue and stores
@@ -690,16 +691,17 @@ constexpr double kSplitFixedUs = 5.0;   // the reduce launch
 struct SplitPlan {
   Tile t = Tile::k128x128;
   int S = 1;          // slices; 1: no split
+  int kc = 0;         // their depth, a multiple of kBK
   double us = 0.0;    // modelled time
 };
 
 SplitPlan split_plan(int batch, int m, int n, int k, size_t cap = kSplitWsMax) {
   SplitPlan p;
-  if (batch < 1 || k <= 0 || k % kBK != 0) return p;
+  if (batch < 1 || k <= 0) return p;
   const long long cu = bch::device_cu_count();
   p.t = pick_tile(batch, m, n);
   const double mn = (double)batch * m * n * sizeof(float);
-  const int nk = k / kBK;
+  const int nk = (k + kBK - 1) / kBK;
   // a part-filled round stays near `idle` up to half of the CUs (256 x 256: 64, 128 and 172
   // workgroups 3.2, 3.26 and 3.4 us per 32 k; 256 x 128: 1.85, 1.93 and 2.05)
   auto kt_us = [&](const TileOpt& o, long long wgs) {
@@ -714,15 +716,17 @@ SplitPlan split_plan(int batch, int m, int n, int k, size_t cap = kSplitWsMax) {
     }
   for (const TileOpt& o : kTileOpts) {
     const long long tiles = tile_count(o, batch, m, n);
-    for (int sl = 2; nk / sl >= kSplitMinKt; ++sl) {
-      if (nk % sl != 0) continue;
+    for (int kt = (nk + 1) / 2; kt >= kSplitMinKt; --kt) {  // k-tiles per slice
+      const int sl = (nk + kt - 1) / kt;
+      if (sl < 2 || (nk + sl - 1) / sl != kt) continue;  // the evenest cut into sl slices
       if ((size_t)sl * batch * m * n * sizeof(float) > cap) break;
       const long long rounds = (tiles * sl + cu - 1) / cu;
-      const double us = (nk / sl) * kt_us(o, tiles * sl) + kSplitRoundUs * (double)(rounds - 1) +
+      const double us = kt * kt_us(o, tiles * sl) + kSplitRoundUs * (double)(rounds - 1) +
                         (2.0 * sl + 1.0) * mn / kSplitBytesUs + kSplitFixedUs;
       if (us < p.us) {
         p.t = o.t;
         p.S = sl;
+        p.kc = kt * kBK;
         p.us = us;
       }
     }
@@ -732,6 +736,34 @@ SplitPlan split_plan(int batch, int m, int n, int k, size_t cap = kSplitWsMax) {
 
 int split_slices(int batch, int m, int n, int k, size_t cap = kSplitWsMax) {
   return split_plan(batch, m, n, k, cap).S;
+}
+
+// Whether a call that needs more workspace than there is, and may not grow it (under capture), is
+// refused rather than run unsplit.  Callers that capture were told to size the workspace first
+// where the plan splits; that holds for the shapes that the split's first rule covered (slices
+// that divide K into 8 k-tiles or more, modelled at the f32 instruction's rate), and shapes that
+// have come to split since still run, unsplit.
+bool split_refused(int batch, int m, int n, int k) {
+  if (k % kBK != 0) return false;
+  const long long cu = bch::device_cu_count();
+  const TileOpt* best = nullptr;
+  double cost = 0.0;
+  for (const TileOpt& o : kTileOpts) {
+    const double c = (double)((tile_count(o, batch, m, n) + cu - 1) / cu) * o.bm * o.bn / o.eff;
+    if (best == nullptr || c < cost * 0.999) {
+      best = &o;
+      cost = c;
+    }
+  }
+  const long long tiles = tile_count(*best, batch, m, n);
+  if (tiles >= cu) return true;  // whole rounds: the hybrid plan's workspace
+  const double tk = 7.4 * best->bm * best->bn / 65536.0 / best->eff, mn = (double)batch * m * n * sizeof(float);
+  const int nk = k / kBK;
+  for (int sl = 2; nk / sl >= 8; ++sl)
+    if (nk % sl == 0 && sl * mn <= (double)kSplitWsMax &&
+        (double)((tiles * sl + cu - 1) / cu) * (nk / sl) * tk + (2.0 * sl + 1.0) * mn / 5e6 + 2.0 < nk * tk)
+      return true;
+  return false;
 }
 
 // ---- small shapes: 64 x 64 x 64 tiles ----
@@ -819,6 +851,7 @@ __global__ __launch_bounds__(256) void sgemm_splitk_reduce(int M, int N, int S, 
 // by 3%.  It needs K a multiple of 32 and unguarded or float4-guarded loads;
 // without the workspace (up to kHybWsMax) the data-parallel tiling runs.
 constexpr size_t kHybWsMax = (size_t)256 << 20;
+constexpr int kHybMinKt = 8;  // k-tiles per slice at least
 
 struct HybPlan {
   Tile t = Tile::k256x256;
@@ -844,7 +877,7 @@ bool hyb_plan(int batch, int m, int n, int k, HybPlan& out, double* cost_us = nu
     if (R < 1 || r == 0) continue;
     int S = 0;
     for (int sl = 8; sl >= 2; --sl)
-      if (sl * r <= cu && nk % sl == 0 && nk / sl >= kSplitMinKt &&
+      if (sl * r <= cu && nk % sl == 0 && nk / sl >= kHybMinKt &&
           (size_t)sl * r * o.bm * o.bn * sizeof(float) <= kHybWsMax) {
         S = sl;
         break;
@@ -1110,6 +1143,17 @@ size_t sgemm_required_workspace_bytes(int batch, int m, int n, int k) {
   return tile_workspace_bytes(batch, m, n, k, false);
 }
 
+bool sgemm_runs_without_workspace(bool transb, int batch, int m, int n, int k, int lda, int ldb) {
+  if (!transb && batch == 1 && sgemm_skinny_applies(m, n, k, nullptr, k, nullptr, n)) return false;
+  if (transb && batch == 1 && (sgemm_skinny_nt_applies(m, n, k, nullptr, lda, nullptr, ldb) ||
+                               nt_two_pass(m, n, k, nullptr, lda, nullptr, ldb)))
+    return false;
+  MixPlan mp;
+  if (mix_plan(batch, m, n, k, mp))
+    return mp.axis == 0 ? !split_refused(1, m - mp.split, n, k) : !split_refused(1, m, n - mp.split, k);
+  return !split_refused(batch, m, n, k);
+}
+
 size_t sgemm_ex_workspace_bytes(bool transb, int batch, int m, int n, int k, int lda, int ldb) {
   if (!transb) return sgemm_workspace_bytes(batch, m, n, k);
   if (batch == 1 && sgemm_skinny_nt_applies(m, n, k, nullptr, lda, nullptr, ldb))
@@ -1186,21 +1230,22 @@ hipError_t launch_tile_path(hipStream_t s, bool transb, int batch, int m, int n,
   if (sl > 1 && ws != nullptr && ws_bytes >= (size_t)sl * pbytes) {
     // batch b, slice j (grid.z): A + b sA + j kc, B + b sB + j kc rows (columns for [n][k]),
     // into P[b][j] (m x n)
-    const int kc = k / sl;
+    const int kc = sp.kc;
     float* P = static_cast<float*>(ws);
     const long long per = (long long)m * n;
     ZSplit z;
     z.nz = sl;
+    z.kc = kc;
     z.sA = kc;
     z.sB = transb ? (long long)kc : (long long)kc * ldb;
     z.sC = per;
     // the slice offsets (kc a multiple of 32, times ldb) keep the batch strides' alignment
-    const int mode = fast_ok(t, m, n, kc, A, lda, sA, B, ldb, sB)               ? 0
-                     : vec4_ok(transb, m, n, kc, A, lda, sA, B, ldb, sB) ? 1
+    const int mode = fast_ok(t, m, n, k, A, lda, sA, B, ldb, sB)               ? 0
+                     : vec4_ok(transb, m, n, k, A, lda, sA, B, ldb, sB) ? 1
                                                                            : 2;
-    hipError_t e = transb ? launch_tile_any<true, false>(mode, t, s, batch, m, n, kc, A, lda, sA, B, ldb, sB, P, n,
+    hipError_t e = transb ? launch_tile_any<true, false>(mode, t, s, batch, m, n, k, A, lda, sA, B, ldb, sB, P, n,
                                                          sl * per, nullptr, 0, z)
-                          : launch_tile_any<false, false>(mode, t, s, batch, m, n, kc, A, lda, sA, B, ldb, sB, P, n,
+                          : launch_tile_any<false, false>(mode, t, s, batch, m, n, k, A, lda, sA, B, ldb, sB, P, n,
                                                           sl * per, nullptr, 0, z);
     if (e != hipSuccess) return e;
     const bool v = n % 4 == 0 && ldc % 4 == 0 && aligned16(C) && (batch == 1 || sC % 4 == 0) &&

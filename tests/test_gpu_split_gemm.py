@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 from barracuda_amd import Tensor
+from tests.test_gpu_graph import CAPTURE_RELAXED, _FreshCtx, _hip
 
 pytestmark = pytest.mark.gpu
 
@@ -112,3 +113,51 @@ def test_one_huge_element_in_a_row(dev):
     a[:, 17] *= 2.0**60
     b[17, :] = 0.0
     _check_f32_sums(_ex(dev, a, b, 0), a, b)
+
+
+@pytest.mark.parametrize("transb", [0, 1])
+@pytest.mark.parametrize("m,n,k", [(171, 455, 1472), (67, 1536, 3056), (128, 150, 2624), (185, 192, 521), (3, 8001, 642),
+                                   (1, 130, 4097), (260, 129, 255), (515, 1030, 1999)])
+def test_uneven_k_slices_exact(dev, m, n, k, transb):
+    """Split-K where the slices do not divide K: the last slice is shorter and takes the remainder."""
+    print(f"uneven slices m={m} n={n} k={k} transb={transb}", flush=True)
+    rng = np.random.default_rng(m + n + k)
+    a = rng.integers(-40, 41, (m, k)).astype(np.float32)
+    b = rng.integers(-40, 41, (n, k) if transb else (k, n)).astype(np.float32)
+    want = (a.astype(np.float64) @ (b.T if transb else b).astype(np.float64)).astype(np.float32)
+    assert np.array_equal(_ex(dev, a, b, transb), want)
+
+
+def test_uneven_k_slices_batched(dev):
+    batch, m, n, k = 3, 150, 70, 1001
+    rng = np.random.default_rng(4)
+    a, b = (rng.integers(-40, 41, s).astype(np.float32) for s in ((batch, m, k), (batch, k, n)))
+    got = Tensor.from_data(a, list(a.shape), dev).batch_matmul(Tensor.from_data(b, list(b.shape), dev)).to_numpy()
+    assert np.array_equal(got, (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32))
+
+
+def test_capture_without_workspace_runs_unsplit(dev):
+    """A shape whose K no slices divide, first called under capture: no workspace may grow, the call
+    runs unsplit, and its graph replays to the product."""
+    hip = _hip()
+    m, n, k = 171, 455, 1471
+    rng = np.random.default_rng(6)
+    a, b = rng.integers(-40, 41, (m, k)).astype(np.float32), rng.integers(-40, 41, (k, n)).astype(np.float32)
+    want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
+    ta, tb, tc = (Tensor.from_data(x, list(x.shape), dev) for x in (a, b, np.zeros((m, n), np.float32)))
+    with _FreshCtx(dev) as f:
+        graph, exe = C.c_void_p(), C.c_void_p()
+        assert hip.hipStreamBeginCapture(f.stream, CAPTURE_RELAXED) == 0
+        st = f.lib.bch_sgemm(f.ctx, m, n, k, C.c_void_p(ta.ptr), k, C.c_void_p(tb.ptr), n, C.c_void_p(tc.ptr), n)
+        assert hip.hipStreamEndCapture(f.stream, C.byref(graph)) == 0
+        assert st == 0 and f.ws_bytes() == 0
+        try:
+            assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, 0) == 0
+            for _ in range(3):
+                dev.upload(tc.ptr, np.full((m, n), np.nan, np.float32))
+                assert hip.hipGraphLaunch(exe, f.stream) == 0
+                assert f.lib.bch_sync(f.ctx) == 0
+                assert np.array_equal(tc.to_numpy(), want)
+        finally:
+            hip.hipGraphExecDestroy(exe)
+            hip.hipGraphDestroy(graph)
