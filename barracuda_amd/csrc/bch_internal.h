@@ -186,8 +186,10 @@ size_t sgemm_workspace_bytes(int batch, int m, int n, int k);
 // The part of it a launch cannot do without (the skinny paths' and split-K's
 // partials); with less than sgemm_workspace_bytes the hybrid plan is skipped.
 size_t sgemm_required_workspace_bytes(int batch, int m, int n, int k);
-// Scratch of launch_sgemm_ex (the skinny paths' partials, split-K partials, or the hybrid plan's).
-size_t sgemm_ex_workspace_bytes(bool transb, int batch, int m, int n, int k, int lda, int ldb);
+// Scratch of launch_sgemm_ex (the skinny paths' and rows kernel's partials, split-K partials, or the
+// hybrid plan's).
+size_t sgemm_ex_workspace_bytes(bool transb, int batch, int m, int n, int k, const float* A, int lda, const float* B,
+                                int ldb);
 // Whether a call whose workspace may not grow runs all the same, unsplit (the tile path, except
 // where its plan has always needed the workspace).
 bool sgemm_runs_without_workspace(bool transb, int batch, int m, int n, int k, int lda, int ldb);

@@ -538,7 +538,7 @@ bch_status bch_sgemm_ex(bch_ctx* ctx, int transb, int m, int n, int k, const flo
   if (!C || (k > 0 && (!A || !B))) return fail(ctx, BCH_E_INVALID, "linear: NULL buffer");
   bch_status st = use(ctx);
   if (st != BCH_OK) return st;
-  size_t wsb = bch::sgemm_ex_workspace_bytes(transb != 0, 1, m, n, k, lda, ldb);
+  size_t wsb = bch::sgemm_ex_workspace_bytes(transb != 0, 1, m, n, k, A, lda, B, ldb);
   if (wsb > ctx->ws_bytes && capturing(ctx) && bch::sgemm_runs_without_workspace(transb != 0, 1, m, n, k, lda, ldb))
     wsb = 0;
   if (wsb) {
@@ -566,7 +566,7 @@ bch_status bch_sgemm(bch_ctx* ctx, int m, int n, int k, const float* A, int lda,
   if (!C || (k > 0 && (!A || !B))) return fail(ctx, BCH_E_INVALID, "matmul: NULL buffer");
   bch_status st = use(ctx);
   if (st != BCH_OK) return st;
-  size_t wsb = bch::sgemm_workspace_bytes(1, m, n, k);
+  size_t wsb = bch::sgemm_ex_workspace_bytes(false, 1, m, n, k, A, lda, B, ldb);
   if (wsb > ctx->ws_bytes && capturing(ctx) && bch::sgemm_runs_without_workspace(false, 1, m, n, k, lda, ldb)) wsb = 0;
   if (wsb) {
     st = ensure_ws(ctx, wsb);

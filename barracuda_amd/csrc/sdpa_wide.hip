@@ -90,7 +90,7 @@ WidePlan wide_plan(int Hkv, int Sq, int Skv, int D, bool causal, int lda, int ld
   for (int r0 = 0; r0 < Sq; r0 += p.rows) {
     int m, n;
     chunk_shape(p, Sq, Skv, causal, r0, m, n);
-    x = std::max(x, bch::sgemm_ex_workspace_bytes(true, Hkv, m, n, D, lda, ldb));
+    x = std::max(x, bch::sgemm_ex_workspace_bytes(true, Hkv, m, n, D, nullptr, lda, nullptr, ldb));
     x = std::max(x, bch::sgemm_workspace_bytes(Hkv, m, D, n));
     x = std::max(x, bch::softmax_workspace_bytes((long long)Hkv * m, n));
   }

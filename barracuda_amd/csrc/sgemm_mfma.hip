@@ -836,6 +836,21 @@ __global__ __launch_bounds__(256) void sgemm_splitk_reduce(int M, int N, int S, 
   }
 }
 
+hipError_t launch_splitk_reduce(hipStream_t s, int m, int n, int S, int batch, const float* P, float* C, int ldc,
+                                long long sC, const float* bias, int act) {
+  const bool v = n % 4 == 0 && ldc % 4 == 0 && aligned16(C) && (batch == 1 || sC % 4 == 0) &&
+                 (bias == nullptr || aligned16(bias));
+  const long long work = (long long)m * n * batch / (v ? 4 : 1);
+  const int blocks = (int)std::min<long long>((work + 255) / 256, 4096);
+  if (v)
+    hipLaunchKernelGGL(sgemm_splitk_reduce<true>, dim3(blocks), dim3(256), 0, s, m, n, S, batch, P, C, ldc, sC, bias,
+                       act);
+  else
+    hipLaunchKernelGGL(sgemm_splitk_reduce<false>, dim3(blocks), dim3(256), 0, s, m, n, S, batch, P, C, ldc, sC, bias,
+                       act);
+  return hipGetLastError();
+}
+
 // ---- whole rounds data-parallel, the last round's tiles split over k (the hybrid plan) ----
 // With T tiles on CU compute units, R = T / CU whole rounds and r = T mod CU
 // tiles left over, the last round would run r workgroups of full length on
@@ -1056,6 +1071,251 @@ hipError_t launch_hyb(int mode, const HybPlan& h, hipStream_t s, int m, int n, i
                                  : launch_tail_reduce<128, 128>(s, m, n, h, P, C, ldc, bias, act);
 }
 
+// ---- few rows: 32 or 64 x 128 tiles, k split over the chip (the rows kernel) ----
+// Up to 64 rows against [n][k] weights, or [k][n] weights that the skinny kernels do not take: the
+// job is streaming B once.  A workgroup owns 128 columns and one k-slice; its 512 threads load an
+// octet of B each per 32-k pass, two passes in flight (64 KB a CU with two workgroups), and
+// put the three parts into LDS as the large tiles do; four wavefronts side by side take 32 columns
+// each, a second set of four the other 16 k of the pass, so each wavefront runs 6 MFMAs per 32
+// rows and pass.  The slices' partials meet in sgemm_splitk_reduce.  At 32 rows the matrix work is
+// 7 us of the 29 us that 4096 x 11008 weights take to stream (18 us as v_mfma_f32_32x32x2_f32).
+// Measured (one box, us, MLP of [n][k] weights with bias and GELU, before -> now): 48 rows 4096 ->
+// 11008 -> 4096 175 -> 117, 32 rows 4095 -> 11007 -> 4095 1364 -> 116, 2 rows 640 -> 8001 -> 640
+// 738 -> 50.  It streams at 4.1 TB/s: conversion, LDS traffic and MFMAs of a pass each take 400 to
+// 600 cycles and overlap only between the two workgroups.
+template <int TM>
+struct RowsCfg {
+  static constexpr int BN = 128, KS = 32, NO = KS / 8, NT = 512;
+  static constexpr int ASTR = 32 * TM * 16 + 32, BSTR = BN * 16 + 32;  // bytes of one octet of one part
+  static constexpr int ABYTES = 3 * NO * ASTR, BUF = ABYTES + 3 * NO * BSTR;
+};
+
+template <int TM, bool TB>
+__global__ __launch_bounds__(512, 4) void sgemm_rows_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
+                                                            const float* __restrict__ B, int ldb, float* __restrict__ C,
+                                                            int ldc, long long sC, const float* __restrict__ bias,
+                                                            int act, int kc) {
+  using G = RowsCfg<TM>;
+  constexpr int KS = G::KS, NO = G::NO;
+  __shared__ __attribute__((aligned(16))) char lds[2 * G::BUF];
+  __shared__ int tiny_seen;
+  const int n0 = blockIdx.x * G::BN, z = blockIdx.y;
+  A += (long long)z * kc;
+  B += TB ? (long long)z * kc : (long long)z * kc * ldb;
+  C += z * sC;
+  K = min(kc, K - z * kc);
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 31, lh = lane >> 5;
+  const int kg = wave >> 2, wn = (wave & 3) * 32;
+  const bool a_wave = wave < 2 * TM;  // these load A's octets too
+  if (tid == 0) tiny_seen = 0;
+
+  const float* pa = A + (long long)min(tid / NO, M - 1) * lda + 8 * (tid % NO);
+  const int brow = TB ? tid / NO : tid % G::BN, boct = TB ? tid % NO : wave >> 1;
+  const int bcol = min(n0 + brow, N - 1);
+  const float* pb = TB ? B + (long long)bcol * ldb + 8 * boct : B + (long long)(8 * boct) * ldb;
+  float ra[2][8], rb[2][8];
+  float ma = 0.0f, mb = 0.0f;  // largest magnitude that this thread's octets have held
+  auto load = [&](int set, int k0) {
+    if (a_wave) load8<false>(pa + k0, ra[set]);
+    if constexpr (TB) {
+      load8<false>(pb + k0, rb[set]);
+    } else {
+      const float* s = pb + (long long)k0 * ldb;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) rb[set][e] = s[(long long)e * ldb + (unsigned)bcol];
+    }
+  };
+  auto load_rest = [&](int k0) {  // zeros from K on
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int ka = k0 + 8 * (tid % NO) + e, kb = k0 + 8 * boct + e;
+      const int da = min(ka, K - 1) - 8 * (tid % NO), db = min(kb, K - 1) - 8 * boct;
+      const float x = a_wave ? pa[da] : 0.0f, y = TB ? pb[db] : pb[(long long)db * ldb + bcol];
+      ra[0][e] = ka < K ? x : 0.0f;
+      rb[0][e] = kb < K ? y : 0.0f;
+    }
+  };
+  auto store = [&](int buf, int set) {
+    char* s = lds + buf * G::BUF;
+    u32x4 q[3];
+    if (a_wave) {
+      ma = split8(ra[set], q, ma);
+#pragma unroll
+      for (int p3 = 0; p3 < 3; ++p3)
+        *reinterpret_cast<u32x4*>(s + (p3 * NO + tid % NO) * G::ASTR + (tid / NO) * 16) = q[p3];
+    }
+    mb = split8(rb[set], q, mb);
+#pragma unroll
+    for (int p3 = 0; p3 < 3; ++p3)
+      *reinterpret_cast<u32x4*>(s + G::ABYTES + (p3 * NO + boct) * G::BSTR + brow * 16) = q[p3];
+  };
+  f32x16 acc[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
+  auto multiply = [&](int buf) {
+    const char* s = lds + buf * G::BUF;
+    u32x4 fa[TM][3], fb[3];
+#pragma unroll
+    for (int p3 = 0; p3 < 3; ++p3) {
+      const int oct = p3 * NO + 2 * kg + lh;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) fa[i][p3] = *reinterpret_cast<const u32x4*>(s + oct * G::ASTR + (32 * i + li) * 16);
+      fb[p3] = *reinterpret_cast<const u32x4*>(s + G::ABYTES + oct * G::BSTR + (wn + li) * 16);
+    }
+#pragma unroll
+    for (int q = 0; q < 6; ++q)
+#pragma unroll
+      for (int i = 0; i < TM; ++i) acc[i] = bf16_mm(fa[i][bch::kPartA[q]], fb[bch::kPartB[q]], acc[i]);
+  };
+
+  // pass t: parts of pass t + 1 to the other buffer, loads of pass t + 3, products of pass t
+  const int nk = (K + KS - 1) / KS, rest = K % KS != 0 ? 1 : 0;  // a remainder runs first
+  auto k_of = [&](int t) { return (min(t, nk - 1) - rest) * KS; };
+  if (rest)
+    load_rest((nk - 1) * KS);
+  else
+    load(0, 0);
+  store(0, 0);
+  if (nk > 1) {
+    load(1, k_of(1));
+    load(0, k_of(2));
+  }
+  __syncthreads();
+  int t = 0;
+  for (; t + 2 < nk; t += 2) {
+    store(1, 1);
+    load(1, k_of(t + 3));
+    multiply(0);
+    __syncthreads();
+    store(0, 0);
+    load(0, k_of(t + 4));
+    multiply(1);
+    __syncthreads();
+  }
+  if (t + 1 < nk) {
+    store(1, 1);
+    multiply(0);
+    __syncthreads();
+    multiply(1);
+  } else {
+    multiply(0);
+  }
+
+  // ---- the two halves of k added up ----
+  bool tiny = false;
+  {
+    float m = ma;
+    m = fmaxf(m, __shfl_xor(m, 1));
+    m = fmaxf(m, __shfl_xor(m, 2));
+    tiny |= a_wave && m > 0.0f && m < bch::kSplitTiny;
+    m = mb;
+    if constexpr (TB) {
+      m = fmaxf(m, __shfl_xor(m, 1));
+      m = fmaxf(m, __shfl_xor(m, 2));
+    }
+    tiny |= m > 0.0f && m < bch::kSplitTiny;
+  }
+  if (tiny) tiny_seen = 1;
+  __syncthreads();  // the last pass's reads are done
+  f32x16* const part = reinterpret_cast<f32x16*>(lds) + (wave & 3) * (64 * TM) + lane;
+  if (kg != 0) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) part[64 * i] = acc[i];
+  }
+  __syncthreads();
+  if (kg != 0) return;
+  float zf = 0.0f;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    acc[i] += part[64 * i];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) zf = fmaf(acc[i][r], 0.0f, zf);
+  }
+  const int col = n0 + wn + li;
+  if (tiny_seen != 0 || __any(zf != 0.0f)) {  // as for the large tiles: again in f32
+    const int c = min(col, N - 1);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const float* qa = A + (long long)min(32 * i + li, M - 1) * lda;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
+#pragma unroll 1
+      for (int k0 = 0; k0 < K; k0 += 2) {
+        const int k = min(k0 + lh, K - 1);
+        const bool in = k0 + lh < K;
+        const float va = qa[k], vb = TB ? B[(long long)c * ldb + k] : B[(long long)k * ldb + c];
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? va : 0.0f, in ? vb : 0.0f, acc[i], 0, 0, 0);
+      }
+    }
+  }
+  if (col >= N) return;
+  const float bj = bias ? bias[col] : 0.0f;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int row = 32 * i + 8 * (r >> 2) + 4 * lh + (r & 3);
+      if (row < M) C[(long long)row * ldc + col] = bch::activate(acc[i][r] + bj, act);
+    }
+}
+
+// Two workgroups per CU resident at once, slices of 4 passes or more; the partials stay under the
+// small scratch, so bch_sgemm_noalloc and bch_sgemm plan alike.
+struct RowsPlan {
+  int S = 1, kc = 0;
+};
+RowsPlan rows_plan(int m, int n, int k) {
+  RowsPlan p;
+  const int tiles = (n + 127) / 128, nk = (k + 31) / 32;
+  long long s = 2LL * bch::device_cu_count() / tiles;
+  s = std::min<long long>({s, nk / 4, (long long)(kSplitWsSmall / (sizeof(float) * (size_t)m * n))});
+  if (s < 1) s = 1;
+  p.kc = (int)((nk + s - 1) / s) * 32;
+  p.S = (k + p.kc - 1) / p.kc;
+  return p;
+}
+// Up to 64 rows where no skinny kernel takes the call (its K, N or alignment: against the tile
+// path's slices MLP of 20 rows 2890 -> 5248 53 -> 46 us), and 33 to 64 rows against [n][k]
+// weights too large for the tile path's slices to stay in step (in us, two passes of the 32-row
+// kernels or tile slices -> here: 48 x 11008 x 4096 78 -> 55, 64 x 4096 x 11008 75 -> 59, 48 x
+// 4096 x 1024 17.7 -> 16.9; 48 x 5120 x 2048 23.0 -> 24.2, so from 2^24 weights on).
+bool rows_applies(bool transb, int batch, int m, int n, int k, const float* A, int lda, const float* B, int ldb) {
+  if (batch != 1 || m > 64 || n < 1 || k < 1) return false;
+  if (transb)
+    return m > 32 ? (long long)n * k >= (1LL << 24) || k % 4 != 0
+                  : !bch::sgemm_skinny_nt_applies(m, n, k, A, lda, B, ldb);
+  return !bch::sgemm_skinny_applies(m, n, k, A, lda, B, ldb) && (m <= 32 || n % 4 != 0);
+}
+size_t rows_bytes(int m, int n, int k) {
+  const RowsPlan p = rows_plan(m, n, k);
+  return p.S > 1 ? (size_t)p.S * m * n * sizeof(float) : 0;
+}
+
+hipError_t launch_rows(hipStream_t s, bool transb, int m, int n, int k, const float* A, int lda, const float* B,
+                       int ldb, float* C, int ldc, const float* bias, int act, void* ws) {
+  const RowsPlan p = rows_plan(m, n, k);
+  const bool split = p.S > 1;
+  float* out = split ? static_cast<float*>(ws) : C;
+  const dim3 grid((n + 127) / 128, p.S);
+#define BCH_ROWS(TM_, TB_)                                                                                       \
+  hipLaunchKernelGGL((sgemm_rows_kernel<TM_, TB_>), grid, dim3(512), 0, s, m, n, k, A, lda, B, ldb, out,          \
+                     split ? n : ldc, split ? (long long)m * n : 0LL, split ? nullptr : bias, split ? 0 : act, p.kc)
+  if (m <= 32) {
+    if (transb) BCH_ROWS(1, true); else BCH_ROWS(1, false);
+  } else {
+    if (transb) BCH_ROWS(2, true); else BCH_ROWS(2, false);
+  }
+#undef BCH_ROWS
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || !split) return e;
+  return launch_splitk_reduce(s, m, n, p.S, 1, static_cast<const float*>(ws), C, ldc, 0, bias, act);
+}
+
 // [n][k] weights with 32 < m <= 64 and n >= 8192: two passes of the m <= 32 path.  Same box,
 // two runs each, against the tile path (bias + ReLU): 33 / 48 / 64 x 11008 x 4096 99.5 / 100.9
 // / 103.0 -> 70.7 / 76.0 / 83.0 us; at n = 4096 the tiles fill the CUs and stay ahead (48 x 4096
@@ -1154,7 +1414,9 @@ bool sgemm_runs_without_workspace(bool transb, int batch, int m, int n, int k, i
   return !split_refused(batch, m, n, k);
 }
 
-size_t sgemm_ex_workspace_bytes(bool transb, int batch, int m, int n, int k, int lda, int ldb) {
+size_t sgemm_ex_workspace_bytes(bool transb, int batch, int m, int n, int k, const float* A, int lda, const float* B,
+                                int ldb) {
+  if (rows_applies(transb, batch, m, n, k, A, lda, B, ldb)) return rows_bytes(m, n, k);
   if (!transb) return sgemm_workspace_bytes(batch, m, n, k);
   if (batch == 1 && sgemm_skinny_nt_applies(m, n, k, nullptr, lda, nullptr, ldb))
     return sgemm_skinny_nt_workspace_bytes(m, n, k);
@@ -1194,6 +1456,8 @@ hipError_t launch_sgemm_ex(hipStream_t s, bool transb, int batch, int m, int n, 
     return launch_sgemm_skinny(s, m, n, k, A, lda, B, ldb, C, ldc, ws, ws_bytes, bias, act);
   if (transb && batch == 1 && sgemm_skinny_nt_applies(m, n, k, A, lda, B, ldb))
     return launch_sgemm_skinny_nt(s, m, n, k, A, lda, B, ldb, C, ldc, ws, ws_bytes, bias, act);
+  if (rows_applies(transb, batch, m, n, k, A, lda, B, ldb) && ws_bytes >= rows_bytes(m, n, k))
+    return launch_rows(s, transb, m, n, k, A, lda, B, ldb, C, ldc, bias, act, ws);
   // 32 < m <= 64 with [n][k] weights: the 32-row kernels twice, on rows 0..31 and 32..m-1 (the
   // second pass streams the weights again, largely from the Infinity Cache)
   if (transb && batch == 1 && nt_two_pass(m, n, k, A, lda, B, ldb)) {
@@ -1248,17 +1512,7 @@ hipError_t launch_tile_path(hipStream_t s, bool transb, int batch, int m, int n,
                           : launch_tile_any<false, false>(mode, t, s, batch, m, n, k, A, lda, sA, B, ldb, sB, P, n,
                                                           sl * per, nullptr, 0, z);
     if (e != hipSuccess) return e;
-    const bool v = n % 4 == 0 && ldc % 4 == 0 && aligned16(C) && (batch == 1 || sC % 4 == 0) &&
-                   (bias == nullptr || aligned16(bias));
-    const long long work = per * batch / (v ? 4 : 1);
-    const int blocks = (int)std::min<long long>((work + 255) / 256, 4096);
-    if (v)
-      hipLaunchKernelGGL(sgemm_splitk_reduce<true>, dim3(blocks), dim3(256), 0, s, m, n, sl, batch, P, C, ldc, sC,
-                         bias, act);
-    else
-      hipLaunchKernelGGL(sgemm_splitk_reduce<false>, dim3(blocks), dim3(256), 0, s, m, n, sl, batch, P, C, ldc, sC,
-                         bias, act);
-    return hipGetLastError();
+    return launch_splitk_reduce(s, m, n, sl, batch, P, C, ldc, sC, bias, act);
   }
   const bool epi = bias != nullptr || act != 0;
   MixPlan mp;

@@ -161,3 +161,35 @@ def test_capture_without_workspace_runs_unsplit(dev):
         finally:
             hip.hipGraphExecDestroy(exe)
             hip.hipGraphDestroy(graph)
+
+
+@pytest.mark.parametrize("transb", [0, 1])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (1, 127, 31), (3, 129, 33), (20, 5247, 1001), (31, 257, 65), (32, 2890, 5249),
+                                   (33, 131, 4099), (64, 1021, 130), (48, 8192, 4096)])
+def test_few_rows_exact(dev, m, n, k, transb):
+    """Up to 64 rows that the skinny kernels do not take (and large [n][k] weights): one 32-column
+    pass, remainders of k, columns and rows, split and unsplit."""
+    print(f"few rows m={m} n={n} k={k} transb={transb}", flush=True)
+    rng = np.random.default_rng(m + n + k)
+    a = rng.integers(-40, 41, (m, k)).astype(np.float32)
+    b = rng.integers(-40, 41, (n, k) if transb else (k, n)).astype(np.float32)
+    want = (a.astype(np.float64) @ (b.T if transb else b).astype(np.float64)).astype(np.float32)
+    assert np.array_equal(_ex(dev, a, b, transb), want)
+
+
+@pytest.mark.parametrize("transb", [0, 1])
+@pytest.mark.parametrize("m,k", [(20, 333), (50, 2049)])
+def test_few_rows_extreme_operands(dev, m, k, transb):
+    """As the tiles: infinities and NaN as in IEEE arithmetic, rows at the low end of the range."""
+    n = 301
+    rng = np.random.default_rng(m)
+    a, b = rng.integers(-8, 9, (m, k)).astype(np.float32), rng.integers(-8, 9, (k, n)).astype(np.float32)
+    a[3, 5], a[10, 0], b[7, 11], b[k - 1, 90] = np.inf, np.nan, -np.inf, np.nan
+    with np.errstate(invalid="ignore"):
+        want = np.einsum("mk,kn->mn", a.astype(np.float64), b.astype(np.float64)).astype(np.float32)
+    bt = (lambda x: np.ascontiguousarray(x.T)) if transb else (lambda x: x)
+    assert np.array_equal(_ex(dev, a, bt(b), transb), want, equal_nan=True)
+    a, b = (rng.standard_normal(s).astype(np.float32) for s in ((m, k), (k, n)))
+    _check_f32_sums(_ex(dev, a * np.float32(2.0**-120), bt(b * np.float32(2.0**100)), transb),
+                    a * np.float32(2.0**-120), b * np.float32(2.0**100))
+    _check_f32_sums(_ex(dev, a, bt(b * np.float32(2.0**-140)), transb), a, b * np.float32(2.0**-140))
