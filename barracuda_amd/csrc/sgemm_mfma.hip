@@ -1071,6 +1071,180 @@ hipError_t launch_hyb(int mode, const HybPlan& h, hipStream_t s, int m, int n, i
                                  : launch_tail_reduce<128, 128>(s, m, n, h, P, C, ldc, bias, act);
 }
 
+// ---- small outputs: 32 x 32 tiles, k over the eight wavefronts of a workgroup ----
+// A product of few tiles and short k is latency: launch, one trip to memory, the sums, the store.
+// A wavefront takes every eighth 32-k unit of its workgroup's tile, loads the operands straight
+// into the MFMA's layout (no LDS, no barrier until the end) with the next unit in flight, and
+// the eight blocks are added in wavefront order through LDS: no partials in memory, no reduce
+// launch.  Each operand value is read and split once per 32 rows or columns, so larger outputs are
+// better off on the split plan's tiles (small_k_plan).
+template <bool TB, bool ALIGNED>
+__global__ __launch_bounds__(512, 4) void sgemm_small_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
+                                                             long long sA, const float* __restrict__ B, int ldb,
+                                                             long long sB, float* __restrict__ C, int ldc,
+                                                             long long sC, int tiles_m,
+                                                             const float* __restrict__ bias, int act) {
+  constexpr int W = 8;
+  __shared__ float part[W][1024];
+  __shared__ float mags[W][64];  // largest magnitudes: rows of A, columns of B
+  // an XCD's workgroups run neighbouring tiles, a column panel of B at a time
+  int lt = blockIdx.x;
+  const int nt = gridDim.x;
+  if ((nt & 7) == 0) lt = (lt & 7) * (nt >> 3) + (lt >> 3);
+  const int m0 = lt % tiles_m * 32, n0 = lt / tiles_m * 32;
+  A += blockIdx.y * sA;
+  B += blockIdx.y * sB;
+  C += blockIdx.y * sC;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 31, lh = lane >> 5;
+  const int row = min(m0 + li, M - 1), col = min(n0 + li, N - 1);
+  const float* const pa = A + (long long)row * lda;
+  const float* const pb = TB ? B + (long long)col * ldb : B + col;
+  const unsigned vb = 4u * (8u * lh * (unsigned)ldb + col);  // [k][n]: this lane's byte offset from a scalar row
+
+  // unit u: k 32 u .. + 31, as two octets of this lane's row and column, 32 u + 16 s + 8 lh ..
+  auto load = [&](int u, float (&a)[2][8], float (&b)[2][8]) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      load8<ALIGNED>(pa + 32 * u + 16 * s + 8 * lh, a[s]);
+      if constexpr (TB) {
+        load8<ALIGNED>(pb + 32 * u + 16 * s + 8 * lh, b[s]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          b[s][e] = *reinterpret_cast<const float*>(
+              reinterpret_cast<const char*>(B + (long long)(32 * u + 16 * s + e) * ldb) + vb);
+      }
+    }
+  };
+  auto load_rest = [&](int u, float (&a)[2][8], float (&b)[2][8]) {  // the k remainder: zeros from K on
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int k = 32 * u + 16 * s + 8 * lh + e, kc = min(k, K - 1);
+        const float x = pa[kc], y = TB ? pb[kc] : pb[(long long)kc * ldb];
+        a[s][e] = k < K ? x : 0.0f;
+        b[s][e] = k < K ? y : 0.0f;
+      }
+  };
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+  float ma = 0.0f, mb = 0.0f;
+  auto multiply = [&](const float (&a)[2][8], const float (&b)[2][8]) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      u32x4 fa[3], fb[3];
+      ma = split8(a[s], fa, ma);
+      mb = split8(b[s], fb, mb);
+#pragma unroll
+      for (int q = 0; q < 6; ++q) acc = bf16_mm(fa[bch::kPartA[q]], fb[bch::kPartB[q]], acc);
+    }
+  };
+  // wavefront w: units w, w + W, ..., its share of the remainder first
+  const int nf = K / 32, nu = (K + 31) / 32;
+  float a0[2][8], b0[2][8], a1[2][8], b1[2][8];
+  int u = wave;
+  bool more = true;
+  if (nf < nu && wave == nf % W) {
+    load_rest(nf, a0, b0);
+  } else if (u < nf) {
+    load(u, a0, b0);
+    u += W;
+  } else {
+    more = false;
+  }
+  while (more) {
+    if ((more = u < nf)) load(u, a1, b1);
+    multiply(a0, b0);
+    if (!more) break;
+    u += W;
+    if ((more = u < nf)) load(u, a0, b0);
+    multiply(a1, b1);
+    u += W;
+  }
+
+  // ---- where the parts cannot stand for the floats (as for the large tiles), again in f32 ----
+  ma = fmaxf(ma, __shfl_xor(ma, 32));
+  mb = fmaxf(mb, __shfl_xor(mb, 32));
+  mags[wave][lane] = lh == 0 ? ma : mb;
+  __syncthreads();
+  float m = mags[0][lane], z = 0.0f;
+#pragma unroll
+  for (int w = 1; w < W; ++w) m = fmaxf(m, mags[w][lane]);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) z = fmaf(acc[r], 0.0f, z);
+  if (__any((m > 0.0f && m < bch::kSplitTiny) || z != 0.0f)) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+#pragma unroll 1
+    for (int v = wave; v < nu; v += W)
+#pragma unroll 1
+      for (int k0 = 32 * v; k0 < min(32 * v + 32, K); k0 += 2) {
+        const int k = min(k0 + lh, K - 1);
+        const bool in = k0 + lh < K;
+        const float x = pa[k], y = TB ? pb[k] : pb[(long long)k * ldb];
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? x : 0.0f, in ? y : 0.0f, acc, 0, 0, 0);
+      }
+  }
+
+  // ---- the eight blocks added in wavefront order, two values a thread ----
+#pragma unroll
+  for (int r = 0; r < 16; ++r) part[wave][64 * r + lane] = acc[r];
+  __syncthreads();
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int i = tid + 512 * h, r = i >> 6;
+    float v = part[0][i];
+#pragma unroll
+    for (int w = 1; w < W; ++w) v += part[w][i];
+    const int om = m0 + 8 * (r >> 2) + 4 * lh + (r & 3), on = n0 + li;
+    if (om < M && on < N) C[(long long)om * ldc + on] = bch::activate(v + (bias ? bias[on] : 0.0f), act);
+  }
+}
+
+// Modelled us: a workgroup's pass of 256 k takes 1.35 us of its CU, alone on it or not, next to
+// 3.2 us of launch, first loads and store, against the split plan's model, which is 2 to 5 us low at
+// these sizes.  Measured, one box, us, before -> here: 65^3 7.5 -> 4.5, 300^3 11.8 -> 5.0, 171 x 455 x 1472
+// 15.0 -> 11.4, 100 x 4000 x 500 15.5 -> 9.6, 1001 x 999 x 333 17.9 -> 13.1, 256 x 1024 x 1024 (split) 15.8 -> 8.5,
+// 512 x 512 x 1024 15.8 -> 9.0; left to the split plan: 700 x 1200 x 1500 26.6 (38.2 here), 256 x 2048 x
+// 2048 22.9 (24.6).  From k 2048 on the split plan's shorter sums are the more exact (128 x 128 x 2048
+// 1.9e-7 against 2.5e-7) and the times within 15%.  Below 64 k, six part products of one product
+// keep 2.3 2^-24, where the tiles' f32 loop rounds once.
+bool small_k_plan(int batch, int m, int n, int k) {
+  if (batch < 1 || batch > 65535 || k < 64 || k >= 2048) return false;
+  const SplitPlan p = split_plan(batch, m, n, k);
+  if (p.us == 0.0) return false;  // whole rounds of the other tiles
+  const long long cu = bch::device_cu_count();
+  const long long wgs = (long long)batch * ((m + 31) / 32) * ((n + 31) / 32);
+  return 3.2 + 1.35 * (double)((wgs + cu - 1) / cu) * ((k + 255) / 256) < p.us + 2.0;
+}
+
+// the kernel's byte offsets of 8 rows of a [k][n] B and a column stay below 2^32
+bool small_k_ok(int batch, int m, int n, int k, int ldb) {
+  return ldb < (1 << 26) && small_k_plan(batch, m, n, k);
+}
+
+hipError_t launch_small_k(hipStream_t s, bool transb, int batch, int m, int n, int k, const float* A, int lda,
+                          long long sA, const float* B, int ldb, long long sB, const float* bias, int act, float* C,
+                          int ldc, long long sC) {
+  const int tm = (m + 31) / 32, tn = (n + 31) / 32;
+  const bool a16 = aligned16(A) && lda % 4 == 0 && (batch == 1 || sA % 4 == 0);
+  const bool b16 = aligned16(B) && ldb % 4 == 0 && (batch == 1 || sB % 4 == 0);
+#define BCH_SMALL_K(TB_, AL_)                                                                                    \
+  hipLaunchKernelGGL((sgemm_small_kernel<TB_, AL_>), dim3(tm * tn, batch), dim3(512), 0, s, m, n, k, A, lda, sA, \
+                     B, ldb, sB, C, ldc, sC, tm, bias, act)
+  if (transb) {
+    if (a16 && b16) BCH_SMALL_K(true, true); else BCH_SMALL_K(true, false);
+  } else {
+    if (a16) BCH_SMALL_K(false, true); else BCH_SMALL_K(false, false);
+  }
+#undef BCH_SMALL_K
+  return hipGetLastError();
+}
+
 // ---- few rows: 32 or 64 x 128 tiles, k split over the chip (the rows kernel) ----
 // Up to 64 rows against [n][k] weights, or [k][n] weights that the skinny kernels do not take: the
 // job is streaming B once.  A workgroup owns 128 columns and one k-slice; its 512 threads load an
@@ -1348,6 +1522,7 @@ static const char* tile_path_name(int m, int n, int k, bool allow_mix) {
     return name.c_str();
   }
   if (small_tile_plan(1, m, n, k)) return "sgemm_mfma_kernel<64,64,64,false>";
+  if (small_k_ok(1, m, n, k, n)) return "sgemm_small_kernel";
   const SplitPlan sp = split_plan(1, m, n, k);
   const Tile t = sp.S > 1 ? sp.t : pick_tile(1, m, n);
   // with lda = k and ldb = n, and 16-byte aligned operands
@@ -1485,6 +1660,8 @@ hipError_t launch_tile_path(hipStream_t s, bool transb, int batch, int m, int n,
                   : (epi ? BCH_SMALL(false, true) : BCH_SMALL(false, false));
 #undef BCH_SMALL
   }
+  if (small_k_ok(batch, m, n, k, ldb))
+    return launch_small_k(s, transb, batch, m, n, k, A, lda, sA, B, ldb, sB, bias, act, C, ldc, sC);
   SplitPlan sp = split_plan(batch, m, n, k);
   const size_t pbytes = (size_t)batch * m * n * sizeof(float);  // one slice's partials, every batch
   if (sp.S > 1 && (ws == nullptr || ws_bytes < (size_t)sp.S * pbytes))

@@ -193,3 +193,75 @@ def test_few_rows_extreme_operands(dev, m, k, transb):
     _check_f32_sums(_ex(dev, a * np.float32(2.0**-120), bt(b * np.float32(2.0**100)), transb),
                     a * np.float32(2.0**-120), b * np.float32(2.0**100))
     _check_f32_sums(_ex(dev, a, bt(b * np.float32(2.0**-140)), transb), a, b * np.float32(2.0**-140))
+
+
+# sgemm_small_kernel: 32 x 32 tiles, the 32-k units of a tile over eight wavefronts
+SMALL = [(65, 65), (70, 33), (96, 100), (128, 160), (255, 257)]
+
+
+@pytest.mark.parametrize("transb", [0, 1])
+@pytest.mark.parametrize("m,n", SMALL)
+@pytest.mark.parametrize("k", [64, 65, 96, 127, 255, 256, 257, 289, 511, 520, 777])
+def test_small_kernel_every_unit_count(dev, m, n, k, transb):
+    """Fewer units than wavefronts, one to four each, and a remainder on each wavefront; every element to
+    the bound of f32 sums, and integers to the last bit."""
+    assert dev._lib.bch_sgemm_kernel_name(m, n, k) == b"sgemm_small_kernel"
+    print(f"small kernel m={m} n={n} k={k} transb={transb}", flush=True)
+    rng = np.random.default_rng(m * n + k)
+    for ints in (False, True):
+        a = rng.integers(-120, 121, (m, k)) if ints else rng.standard_normal((m, k))
+        b = rng.integers(-120, 121, (k, n)) if ints else rng.standard_normal((k, n))
+        a, b = a.astype(np.float32), b.astype(np.float32)
+        got = _ex(dev, a, np.ascontiguousarray(b.T) if transb else b, transb)
+        if ints:  # |sums| <= 777 * 120^2 < 2^24
+            assert np.array_equal(got, (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32))
+        else:
+            _check_f32_sums(got, a, b)
+
+
+@pytest.mark.parametrize("transb", [0, 1])
+def test_small_kernel_operands_without_parts(dev, transb):
+    """Infinities, NaN, the largest floats and rows of tiny magnitudes, in a unit that the fourth
+    wavefront holds: as the f32 instruction gives them."""
+    print(f"small kernel, operands without parts, transb={transb}", flush=True)
+    rng = np.random.default_rng(5)
+    m, n, k = 96, 64, 300
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    a[3] *= np.float32(2.0**-120)
+    b[:, 40] *= np.float32(2.0**-110)
+    a[70, 100] = np.inf
+    a[71, 101] = np.nan
+    a[33], b[:, 9] = 0.0, 1.0
+    a[33, 110] = np.float32(3.4e38)
+    got = _ex(dev, a, np.ascontiguousarray(b.T) if transb else b, transb)
+    with np.errstate(invalid="ignore"):
+        want = a.astype(np.float64) @ b.astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[70], want[70].astype(np.float32))
+    assert got[33, 9] == np.float32(3.4e38)
+    rows = [r for r in range(m) if r not in (33, 70, 71)]
+    _check_f32_sums(got[rows], a[rows], b)
+
+
+def test_small_kernel_misaligned_strided_batched_with_epilogue(dev):
+    """Odd leading dimensions and start offsets, a bias with an activation, and batches."""
+    print("small kernel, misaligned, epilogue, batched", flush=True)
+    rng = np.random.default_rng(6)
+    m, n, k = 77, 90, 270
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    _check_f32_sums(_ex(dev, a, b, 1, lda=k + 3, ldb=k + 1, a_off=1, b_off=3), a, b.T)
+    bt = np.ascontiguousarray(b.T)
+    _check_f32_sums(_ex(dev, a, bt, 0, lda=k + 3, ldb=n + 1, a_off=1, b_off=3), a, bt)
+    bias = rng.standard_normal(n).astype(np.float32)
+    ta, tb, tbias = (Tensor.from_data(x, list(x.shape), dev) for x in (a, b, bias))
+    out = Tensor.empty([m, n], dev)
+    dev.check(dev._lib.bch_sgemm_ex(dev.ctx, 1, m, n, k, C.c_void_p(ta.ptr), k, C.c_void_p(tb.ptr), k,
+                                    C.c_void_p(tbias.ptr), 1, C.c_void_p(out.ptr), n), "linear")
+    want = np.maximum(a.astype(np.float64) @ b.T.astype(np.float64) + bias, 0.0)
+    # k + 1 roundings of sums of magnitudes below |a| |b| + |bias|
+    bound = (k + 1) * 2.0**-24 * (np.abs(a).astype(np.float64) @ np.abs(b.T) + np.abs(bias))
+    assert np.all(np.abs(out.to_numpy() - want) <= bound)
+    xs, ys = rng.standard_normal((5, m, k)).astype(np.float32), rng.standard_normal((5, k, n)).astype(np.float32)
+    got = Tensor.from_data(xs, [5, m, k], dev).batch_matmul(Tensor.from_data(ys, [5, k, n], dev)).to_numpy()
+    for g, x, y in zip(got, xs, ys):
+        _check_f32_sums(g, x, y)
