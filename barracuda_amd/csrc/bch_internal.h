@@ -66,21 +66,28 @@ __device__ __forceinline__ float activate(float v, int act) {
 }
 
 // ---- f32 products on the bf16 matrix cores ----
-// An f32 x is split into three bf16 parts, x = x0 + x1 + x2 exactly: x0 is x rounded to 8
-// significant bits, x1 the remainder rounded, x2 the rest (8 + 8 + 8 bits and the parts' signs
-// hold 24).  x y then is the sum of nine part products; the six of weight 2^-18 and above
-// (kPartA, kPartB, smallest first) are accumulated in f32 on v_mfma_f32_32x32x16_bf16, whose
-// products are exact.  What is left out is below 2^-26 of each product, a quarter of the
-// rounding of one f32 addition.  This is the scheme of Henry, Tang and Heinecke, "Leveraging the
-// bfloat16 artificial intelligence datatype for higher-precision computations" (ARITH 2019).
+// An f32 x is scaled by 2^16 and split into three bf16 parts, 2^16 x = x0 + x1 + x2 exactly: x0 is
+// it rounded to 8 significant bits, x1 the remainder rounded, x2 the rest (8 + 8 + 8 bits and the
+// parts' signs hold 24; a subnormal x is a multiple of 2^-149, and 2^-133 is bf16's smallest
+// subnormal, which the conversion and the matrix cores keep).  x y then is the sum of nine part
+// products; the six largest (kPartA, kPartB, smallest first) are accumulated in f32 on
+// v_mfma_f32_32x32x16_bf16, whose products are exact, and the sums scaled back by 2^-32.  This is
+// the scheme of Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial intelligence
+// datatype for higher-precision computations" (ARITH 2019).
+// What is left out: |x1| <= 2^-8 and |x2| <= 2^-17 of x's power of two, so x1 y2 + x2 y1 reaches
+// 2^-24 of |x y| at worst (x = y = 1.0039) and is 2^-27 in the root mean square; the rounding of
+// one f32 addition is up to 2^-24.  A single product alone in its sum thus can be off by 1.7 2^-24
+// where an f32 multiplication rounds by 2^-24; sums of many come out closer than on the f32
+// instruction, whose accumulator rounds once every two k instead of six times every sixteen.
+// Integers whose product is below 2^24 stay exact.
 // Why: v_mfma_f32_32x32x2_f32 does 256 FLOP a clock and CU, the bf16 instruction 4096, so six of
-// them still leave 2.7 times the f32 rate.  Integers whose product is below 2^24 stay exact.
-// An infinite x has x0 = x and x1 NaN, and parts of |x| below 2^-103 reach past bf16's normal
-// range: callers look for both (kSplitTiny) and redo such blocks in f32.
+// them still leave 2.7 times the f32 rate.
+// Infinities, NaN, |x| from 2^111 and sums from 2^96 leave results that are not finite (an infinite
+// x0 meets a NaN x1): callers look for those and compute them again in f32.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-constexpr float kSplitTiny = 0x1p-100f;
+constexpr float kSplitScale = 0x1p16f, kSplitUnscale = 0x1p-32f;
 constexpr int kPartA[6] = {2, 1, 0, 1, 0, 0}, kPartB[6] = {0, 1, 2, 0, 1, 0};
 
 // Two floats rounded to bf16, x in the low half.
@@ -89,10 +96,8 @@ __device__ __forceinline__ unsigned bf16_pack(float x, float y) {
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
   return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x, y}), bf16x2));
 }
-// Parts of two floats into element e of p[0..2] (x and y are left as remainders); returns
-// max(m, |x|, |y|) (NaN left out).
-__device__ __forceinline__ float split2(float& x, float& y, u32x4 (&p)[3], int e, float m) {
-  m = fmaxf(m, fmaxf(fabsf(x), fabsf(y)));
+// Parts of two floats, scaled already, into element e of p[0..2] (x and y are left as remainders).
+__device__ __forceinline__ void split2(float& x, float& y, u32x4 (&p)[3], int e) {
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
     p[q][e] = bf16_pack(x, y);
@@ -101,16 +106,14 @@ __device__ __forceinline__ float split2(float& x, float& y, u32x4 (&p)[3], int e
       y -= __builtin_bit_cast(float, p[q][e] & 0xffff0000u);
     }
   }
-  return m;
 }
-// Parts p[0..2] of eight floats; returns max(m, |v[0]|, ..., |v[7]|) (NaN left out).
-__device__ __forceinline__ float split8(const float (&v)[8], u32x4 (&p)[3], float m) {
+// Parts p[0..2] of eight floats times scale.
+__device__ __forceinline__ void split8(const float (&v)[8], u32x4 (&p)[3], float scale = kSplitScale) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    float x = v[2 * e], y = v[2 * e + 1];
-    m = split2(x, y, p, e, m);
+    float x = v[2 * e] * scale, y = v[2 * e + 1] * scale;
+    split2(x, y, p, e);
   }
-  return m;
 }
 __device__ __forceinline__ f32x16 bf16_mm(u32x4 a, u32x4 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,

@@ -60,9 +60,12 @@
 //     key/value head (grouped-query) are adjacent, so they share it in the same L2.
 //   * Too few query blocks for the chip: the keys of each are split over workgroups, whose
 //     results (unnormalised O, reference max, sum) meet in sdpa_combine (sdpa_decode.hip).
-//   * An operand that its parts cannot stand for (infinite, NaN, a column or octet of magnitudes
-//     below 2^-100) leaves a result that is not finite, or is seen while splitting: the
-//     wavefront then redoes its queries on v_mfma_f32_32x32x2_f32 from global memory.
+//   * Parts are of 2^16 times the operand (split8); scores are scaled back in the fused
+//     multiply-add that subtracts the reference max, O at the end.  Where the scaled numbers may pass
+//     f32's range, the wavefront redoes its queries on v_mfma_f32_32x32x2_f32 from global memory:
+//     an infinite, NaN or huge V (or a NaN score) leaves a result that is not finite; scores, of
+//     which one infinite before its sum ends could pass for a masked one, are bounded by their
+//     operands, |q scale log2(e)| and |K| below 2^43, seen while splitting.
 #include "bch_internal.h"
 
 #include <math.h>
@@ -81,6 +84,9 @@ constexpr int kBKV = 32;  // keys per block
 constexpr int kVLD = kBKV + 4;
 constexpr float kLog2E = 1.44269504088896340736f;
 constexpr float kLazy = 8.0f;  // log2 headroom before the reference max moves
+// 128 products of operands below this, scaled by 2^32 (and their leading parts, up to 2^-8 larger),
+// stay below 2^127.
+constexpr float kScoreBig = 0x1p43f;
 
 // NT threads per workgroup: NT / 64 wavefronts of 32 queries each.
 template <int DP, int NT>
@@ -226,7 +232,7 @@ __global__ __launch_bounds__(64 * NW) void sdpa_fwd_kernel(
   constexpr int NT = G::NT, NO = G::NO, NC = DP / 16, NBK = DP / 32;
   __shared__ __attribute__((aligned(16))) char k_lds[2 * G::KBYTES], v_lds[2 * G::VBYTES];
   __shared__ u32x4 q_lds[G::QL > 0 ? G::QL * NT : 1];
-  __shared__ int tiny_seen;
+  __shared__ int big_seen;
 
   // causal: query-block major, all heads' longest query blocks first.
   // non-causal: head-major over an XCD-contiguous remap of the grid.
@@ -256,7 +262,7 @@ __global__ __launch_bounds__(64 * NW) void sdpa_fwd_kernel(
   // queries past the end repeat the last one and are not stored
   const float* qr = q + bi * st.q.batch + hq * st.q.head + (long long)min(myq, Sq - 1) * st.q.row;
 
-  if (tid == 0) tiny_seen = 0;
+  if (tid == 0) big_seen = 0;
 
   // eight floats of a row from column d0 on, zeros from D on
   auto row8 = [&](const float* row, int d0, float (&x)[8]) {
@@ -279,15 +285,17 @@ __global__ __launch_bounds__(64 * NW) void sdpa_fwd_kernel(
 
   // ---- q parts: step c holds q[myq][16c + 8lh .. +7] * scale * log2(e) ----
   u32x4 qf[NC][3];
+  float mq = 0.0f;  // largest magnitude
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     float x[8];
     row8(qr, 16 * c + 8 * lh, x);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] *= qscale;
-    split8(x, qf[c], 0.0f);
+    for (int e = 0; e < 8; ++e) mq = fmaxf(mq, fabsf(x[e] * qscale));
+    split8(x, qf[c], qscale * bch::kSplitScale);
     if (c < G::QL) q_lds[c * NT + tid] = qf[c][2];  // read back by this lane alone
   }
+  const bool q_big = __any(mq >= kScoreBig);  // settled here: later, the floats of q would stay in registers
 
   f32x16 oacc[NBK];
   float m_ref, l_run;
@@ -312,9 +320,7 @@ __global__ __launch_bounds__(64 * NW) void sdpa_fwd_kernel(
   // 16 (oct / 2) + 4 (oct % 2) + {0..3, 8..11}).  Keys past the end repeat the last one; their
   // scores are masked and their V rows zeroed.
   float rk[G::CH][8], rv[G::CH][8];
-  float mk[G::CH], mv[G::CH];
-#pragma unroll
-  for (int c = 0; c < G::CH; ++c) mk[c] = mv[c] = 0.0f;
+  float mk = 0.0f;  // largest magnitude of the K that this thread has split
   auto load_k = [&](int t) {
 #pragma unroll
     for (int c = 0; c < G::CH; ++c) {
@@ -353,10 +359,12 @@ __global__ __launch_bounds__(64 * NW) void sdpa_fwd_kernel(
   constexpr int UNITS = 8 * G::CH;
   auto split_unit = [&](int u) {
     const int c = (u >> 2) % G::CH, e = u & 3;
-    if (u < UNITS / 2)
-      mv[c] = bch::split2(rv[c][2 * e], rv[c][2 * e + 1], vp[c], e, mv[c]);
-    else
-      mk[c] = bch::split2(rk[c][2 * e], rk[c][2 * e + 1], kp[c], e, mk[c]);
+    float& x = u < UNITS / 2 ? rv[c][2 * e] : rk[c][2 * e];
+    float& y = u < UNITS / 2 ? rv[c][2 * e + 1] : rk[c][2 * e + 1];
+    if (u >= UNITS / 2) mk = fmaxf(mk, fmaxf(fabsf(x), fabsf(y)));
+    x *= bch::kSplitScale;
+    y *= bch::kSplitScale;
+    bch::split2(x, y, u < UNITS / 2 ? vp[c] : kp[c], e);
   };
   auto store_k = [&](int buf) {
     char* s = k_lds + buf * G::KBYTES;
@@ -393,11 +401,13 @@ __global__ __launch_bounds__(64 * NW) void sdpa_fwd_kernel(
   };
   // Scores -> probabilities against the reference max, which moves when a block exceeds it by
   // more than 2^kLazy, and their parts pf, in kPieces pieces that a caller may set between MFMAs.
+  // unit: the scores' scale.  (A reference 16 lower would scale the probabilities for nothing, but
+  // larger exponents round more: error at the timed shape 3.8e-7 -> 4.4e-7.)
   // alpha: what the results so far are to be multiplied by (rescale).
   u32x4 pf[2][3];  // parts of the last block's probabilities
   float bm, m_use, rs, alpha;
   constexpr int kPieces = 20;
-  auto piece = [&](f32x16& s, int i) {
+  auto piece = [&](float unit, f32x16& s, int i) {
     if (i == 0) {
       bm = s[0];
 #pragma unroll
@@ -405,7 +415,7 @@ __global__ __launch_bounds__(64 * NW) void sdpa_fwd_kernel(
     } else if (i == 1) {
 #pragma unroll
       for (int r = 8; r < 16; ++r) bm = fmaxf(bm, s[r]);
-      bm = half_swap_max(bm);
+      bm = half_swap_max(bm) * unit;
     } else if (i == 2) {
       const bool move = bm > m_ref + kLazy;  // -inf reference: any finite block max moves it
       const float m_new = move ? bm : m_ref;
@@ -417,20 +427,20 @@ __global__ __launch_bounds__(64 * NW) void sdpa_fwd_kernel(
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         const int r = 2 * (i - 3) + e;
-        s[r] = __builtin_amdgcn_exp2f(s[r] - m_use);
+        s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], unit, -m_use));
         rs += s[r];
       }
     } else if (i == 11) {
       l_run = l_run * alpha + half_swap_sum(rs);
     } else {
       const int u = i - 12, h = u >> 2, e = u & 3;
-      float x = s[8 * h + 2 * e], y = s[8 * h + 2 * e + 1];
-      bch::split2(x, y, pf[h], e, 0.0f);
+      float x = s[8 * h + 2 * e] * bch::kSplitScale, y = s[8 * h + 2 * e + 1] * bch::kSplitScale;
+      bch::split2(x, y, pf[h], e);
     }
   };
-  auto softmax = [&](f32x16& s) {  // without the parts
+  auto softmax = [&](float unit, f32x16& s) {  // without the parts
 #pragma unroll
-    for (int i = 0; i < 12; ++i) piece(s, i);
+    for (int i = 0; i < 12; ++i) piece(unit, s, i);
     return alpha;
   };
   auto rescale = [&](float alpha) {
@@ -515,9 +525,9 @@ __global__ __launch_bounds__(64 * NW) void sdpa_fwd_kernel(
     stage(t);
     __builtin_amdgcn_sched_barrier(0);
     if (decltype(masked)::value) mask(s, t * kBKV);
-    rescale(softmax(s));
+    rescale(softmax(bch::kSplitUnscale, s));
 #pragma unroll
-    for (int i = 12; i < kPieces; ++i) piece(s, i);
+    for (int i = 12; i < kPieces; ++i) piece(bch::kSplitUnscale, s, i);
     __builtin_amdgcn_sched_barrier(0);
     pv(cur);
     __syncthreads();
@@ -552,21 +562,19 @@ __global__ __launch_bounds__(64 * NW) void sdpa_fwd_kernel(
     __syncthreads();
   }
 
-  // ---- where the parts cannot stand for the operands: these queries again in f32 ----
-  bool redo = false;
+  // ---- O scaled back; where the parts cannot stand for the operands, these queries again in f32 ----
+  bool redo;
   {
     float z = l_run * 0.0f;
 #pragma unroll
-    for (int b = 0; b < NBK; ++b)
+    for (int b = 0; b < NBK; ++b) {
+      oacc[b] *= bch::kSplitUnscale;
 #pragma unroll
       for (int r = 0; r < 16; ++r) z = fmaf(oacc[b][r], 0.0f, z);
-    bool tiny = false;
-#pragma unroll
-    for (int c = 0; c < G::CH; ++c)
-      tiny |= (mk[c] > 0.0f && mk[c] < bch::kSplitTiny) || (mv[c] > 0.0f && mv[c] < bch::kSplitTiny);
-    if (tiny) tiny_seen = 1;
+    }
+    if (mk >= kScoreBig) big_seen = 1;
     __syncthreads();
-    redo = tiny_seen != 0 || __any(z != 0.0f);
+    redo = q_big || big_seen != 0 || __any(z != 0.0f);
   }
   if (redo && q0w < Sq) {
     reset();
@@ -586,7 +594,7 @@ __global__ __launch_bounds__(64 * NW) void sdpa_fwd_kernel(
         s = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? kx : 0.0f, in ? qx : 0.0f, s, 0, 0, 0);
       }
       if (kb + kBKV > Skv || (causal && kb + kBKV - 1 > q0w)) mask(s, kb);
-      rescale(softmax(s));
+      rescale(softmax(1.0f, s));
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int key = kb + 8 * (r >> 2) + 4 * lh + (r & 3);

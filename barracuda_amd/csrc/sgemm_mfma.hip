@@ -277,18 +277,13 @@ __global__ __launch_bounds__((Cfg<BM, BN, BK>::NT)) void sgemm_mfma_kernel(
   // [buffer][A or B][part][octet][row][8 k]: a fragment read takes 16 bytes of 32 consecutive
   // rows, so it needs no padding; PAD shifts the octets so that the eight lanes of a store phase
   // (128 / NO bytes of each of NO octets of a row-major operand) cover different banks.
-  float ma[G::CA], mb[G::CB];  // largest magnitude each octet position has held
-#pragma unroll
-  for (int c = 0; c < G::CA; ++c) ma[c] = 0.0f;
-#pragma unroll
-  for (int c = 0; c < G::CB; ++c) mb[c] = 0.0f;
   auto store_a = [&](int buf) {
     char* s = smem + buf * G::BUF;
 #pragma unroll
     for (int c = 0; c < G::CA; ++c) {
       const int ch = tid + c * G::NT;
       u32x4 q[3];
-      ma[c] = split8(ra[c], q, ma[c]);
+      split8(ra[c], q);
 #pragma unroll
       for (int p3 = 0; p3 < 3; ++p3)
         *reinterpret_cast<u32x4*>(s + (p3 * NO + ch % NO) * G::ASTR + (ch / NO) * 16) = q[p3];
@@ -301,7 +296,7 @@ __global__ __launch_bounds__((Cfg<BM, BN, BK>::NT)) void sgemm_mfma_kernel(
       const int ch = tid + c * G::NT;
       const int row = TB ? ch / NO : ch % BN, oct = TB ? ch % NO : ch / BN;
       u32x4 q[3];
-      mb[c] = split8(rb[c], q, mb[c]);
+      split8(rb[c], q);
 #pragma unroll
       for (int p3 = 0; p3 < 3; ++p3) *reinterpret_cast<u32x4*>(s + (p3 * NO + oct) * G::BSTR + row * 16) = q[p3];
     }
@@ -373,8 +368,6 @@ __global__ __launch_bounds__((Cfg<BM, BN, BK>::NT)) void sgemm_mfma_kernel(
   };
   // Fewer k than one pass holds (K = 0 too): the f32 loop below alone, at most KS / 2 steps.
   const bool short_k = K < KS;
-  __shared__ int tiny_seen;
-  if (tid == 0) tiny_seen = 0;
   if (!short_k) {
     if (rest)
       load_rest((nk - 1) * KS);
@@ -404,42 +397,21 @@ __global__ __launch_bounds__((Cfg<BM, BN, BK>::NT)) void sgemm_mfma_kernel(
     if (kg == 0) acc[0][0] += *part;
   }
 
-  // ---- where the parts cannot stand for the floats, the tile again in f32 ----
-  // An infinite or NaN operand (or a part product that overflows) leaves a result that is not
-  // finite; a row of A or column of B whose largest magnitude is below 2^-100 has third parts
-  // below bf16's range.  Either is rare, and the wavefront then redoes its blocks on
-  // v_mfma_f32_32x32x2_f32 from global memory.
+  // ---- scaled back; where the parts cannot stand for the floats, the tile again in f32 ----
+  // An operand that is infinite, NaN or 2^111 and more, or a sum from 2^96, leaves a result that is
+  // not finite.  The wavefront then redoes its blocks on v_mfma_f32_32x32x2_f32 from global memory.
   bool redo = short_k;
-  if (!short_k) {
+  {
     float z = 0.0f;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
+      for (int j = 0; j < TN; ++j) {
+        acc[i][j] *= bch::kSplitUnscale;
 #pragma unroll
         for (int r = 0; r < 16; ++r) z = fmaf(acc[i][j][r], 0.0f, z);
-    redo = z != 0.0f;  // NaN
-    bool tiny = false;
-#pragma unroll
-    for (int c = 0; c < G::CA; ++c) {
-      float m = ma[c];  // the row's octets sit in NO neighbouring lanes
-#pragma unroll
-      for (int o = 1; o < NO; o <<= 1) m = fmaxf(m, __shfl_xor(m, o));
-      tiny |= m > 0.0f && m < bch::kSplitTiny;
-    }
-#pragma unroll
-    for (int c = 0; c < G::CB; ++c) {
-      float m = mb[c];
-      if constexpr (TB) {
-#pragma unroll
-        for (int o = 1; o < NO; o <<= 1) m = fmaxf(m, __shfl_xor(m, o));
       }
-      tiny |= m > 0.0f && m < bch::kSplitTiny;
-    }
-    // a wavefront's rows and columns were loaded by others
-    if (tiny) tiny_seen = 1;
-    __syncthreads();
-    redo = tiny_seen != 0 || __any(redo);
+    redo |= __any(z != 0.0f);  // NaN
   }
   if (G::KG > 1 && kg != 0) return;
   if (redo) {
@@ -1086,7 +1058,6 @@ __global__ __launch_bounds__(512, 4) void sgemm_small_kernel(int M, int N, int K
                                                              const float* __restrict__ bias, int act) {
   constexpr int W = 8;
   __shared__ float part[W][1024];
-  __shared__ float mags[W][64];  // largest magnitudes: rows of A, columns of B
   // an XCD's workgroups run neighbouring tiles, a column panel of B at a time
   int lt = blockIdx.x;
   const int nt = gridDim.x;
@@ -1132,13 +1103,12 @@ __global__ __launch_bounds__(512, 4) void sgemm_small_kernel(int M, int N, int K
   f32x16 acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-  float ma = 0.0f, mb = 0.0f;
   auto multiply = [&](const float (&a)[2][8], const float (&b)[2][8]) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       u32x4 fa[3], fb[3];
-      ma = split8(a[s], fa, ma);
-      mb = split8(b[s], fb, mb);
+      split8(a[s], fa);
+      split8(b[s], fb);
 #pragma unroll
       for (int q = 0; q < 6; ++q) acc = bf16_mm(fa[bch::kPartA[q]], fb[bch::kPartB[q]], acc);
     }
@@ -1167,16 +1137,11 @@ __global__ __launch_bounds__(512, 4) void sgemm_small_kernel(int M, int N, int K
   }
 
   // ---- where the parts cannot stand for the floats (as for the large tiles), again in f32 ----
-  ma = fmaxf(ma, __shfl_xor(ma, 32));
-  mb = fmaxf(mb, __shfl_xor(mb, 32));
-  mags[wave][lane] = lh == 0 ? ma : mb;
-  __syncthreads();
-  float m = mags[0][lane], z = 0.0f;
-#pragma unroll
-  for (int w = 1; w < W; ++w) m = fmaxf(m, mags[w][lane]);
+  acc *= bch::kSplitUnscale;
+  float z = 0.0f;
 #pragma unroll
   for (int r = 0; r < 16; ++r) z = fmaf(acc[r], 0.0f, z);
-  if (__any((m > 0.0f && m < bch::kSplitTiny) || z != 0.0f)) {
+  if (__any(z != 0.0f)) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
 #pragma unroll 1
@@ -1272,7 +1237,6 @@ __global__ __launch_bounds__(512, 4) void sgemm_rows_kernel(int M, int N, int K,
   using G = RowsCfg<TM>;
   constexpr int KS = G::KS, NO = G::NO;
   __shared__ __attribute__((aligned(16))) char lds[2 * G::BUF];
-  __shared__ int tiny_seen;
   const int n0 = blockIdx.x * G::BN, z = blockIdx.y;
   A += (long long)z * kc;
   B += TB ? (long long)z * kc : (long long)z * kc * ldb;
@@ -1284,14 +1248,12 @@ __global__ __launch_bounds__(512, 4) void sgemm_rows_kernel(int M, int N, int K,
   const int li = lane & 31, lh = lane >> 5;
   const int kg = wave >> 2, wn = (wave & 3) * 32;
   const bool a_wave = wave < 2 * TM;  // these load A's octets too
-  if (tid == 0) tiny_seen = 0;
 
   const float* pa = A + (long long)min(tid / NO, M - 1) * lda + 8 * (tid % NO);
   const int brow = TB ? tid / NO : tid % G::BN, boct = TB ? tid % NO : wave >> 1;
   const int bcol = min(n0 + brow, N - 1);
   const float* pb = TB ? B + (long long)bcol * ldb + 8 * boct : B + (long long)(8 * boct) * ldb;
   float ra[2][8], rb[2][8];
-  float ma = 0.0f, mb = 0.0f;  // largest magnitude that this thread's octets have held
   auto load = [&](int set, int k0) {
     if (a_wave) load8<false>(pa + k0, ra[set]);
     if constexpr (TB) {
@@ -1316,12 +1278,12 @@ __global__ __launch_bounds__(512, 4) void sgemm_rows_kernel(int M, int N, int K,
     char* s = lds + buf * G::BUF;
     u32x4 q[3];
     if (a_wave) {
-      ma = split8(ra[set], q, ma);
+      split8(ra[set], q);
 #pragma unroll
       for (int p3 = 0; p3 < 3; ++p3)
         *reinterpret_cast<u32x4*>(s + (p3 * NO + tid % NO) * G::ASTR + (tid / NO) * 16) = q[p3];
     }
-    mb = split8(rb[set], q, mb);
+    split8(rb[set], q);
 #pragma unroll
     for (int p3 = 0; p3 < 3; ++p3)
       *reinterpret_cast<u32x4*>(s + G::ABYTES + (p3 * NO + boct) * G::BSTR + brow * 16) = q[p3];
@@ -1381,20 +1343,6 @@ __global__ __launch_bounds__(512, 4) void sgemm_rows_kernel(int M, int N, int K,
   }
 
   // ---- the two halves of k added up ----
-  bool tiny = false;
-  {
-    float m = ma;
-    m = fmaxf(m, __shfl_xor(m, 1));
-    m = fmaxf(m, __shfl_xor(m, 2));
-    tiny |= a_wave && m > 0.0f && m < bch::kSplitTiny;
-    m = mb;
-    if constexpr (TB) {
-      m = fmaxf(m, __shfl_xor(m, 1));
-      m = fmaxf(m, __shfl_xor(m, 2));
-    }
-    tiny |= m > 0.0f && m < bch::kSplitTiny;
-  }
-  if (tiny) tiny_seen = 1;
   __syncthreads();  // the last pass's reads are done
   f32x16* const part = reinterpret_cast<f32x16*>(lds) + (wave & 3) * (64 * TM) + lane;
   if (kg != 0) {
@@ -1406,12 +1354,12 @@ __global__ __launch_bounds__(512, 4) void sgemm_rows_kernel(int M, int N, int K,
   float zf = 0.0f;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    acc[i] += part[64 * i];
+    acc[i] = (acc[i] + part[64 * i]) * bch::kSplitUnscale;
 #pragma unroll
     for (int r = 0; r < 16; ++r) zf = fmaf(acc[i][r], 0.0f, zf);
   }
   const int col = n0 + wn + li;
-  if (tiny_seen != 0 || __any(zf != 0.0f)) {  // as for the large tiles: again in f32
+  if (__any(zf != 0.0f)) {  // as for the large tiles: again in f32
     const int c = min(col, N - 1);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {

@@ -79,3 +79,38 @@ def test_parts_extreme_operands(dev, sq):
         # smallest subnormal a term
         bound = 2e-6 * np.abs(v[0, head][:, cols]).max(0) + sq * 2.0**-150
         assert np.all(np.isfinite(x)) and np.all(np.abs(x - y) <= bound), head
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("sq,d", [(300, 64), (300, 128), (2048, 128)])  # split keys; split keys; whole
+@pytest.mark.parametrize("e", [-120, -126, 90, 120])
+def test_parts_scaled_operands(dev, sq, d, e, causal):
+    """q scaled by 2^e against K scaled by 2^-e: ordinary scores of operands at the ends of the range."""
+    print(f"scaled operands sq={sq} d={d} 2^{e} causal={causal}", flush=True)
+    h = 6 if sq == 300 else 40
+    q, k, v = _inputs(1, h, sq, sq, d)
+    q, k = q * np.float32(2.0**e), k * np.float32(0.125) * np.float32(2.0**-e)
+    want = O.sdpa_f64(*(np.ascontiguousarray(x[:, :2]) for x in (q, k, v)), causal)
+    assert O.max_rel_err(_run(dev, q, k, v, causal)[:, :2], want) <= TOL
+
+
+@pytest.mark.parametrize("sq", [300, 2048])
+def test_parts_tiny_elements_beside_ordinary_ones(dev, sq):
+    """Half of each row of q ordinary against zeros in K, the other half 2^-122 against 2^122; a key of
+    probability 2^-124 with the only nonzero value."""
+    print(f"tiny elements beside ordinary ones sq={sq}", flush=True)
+    h, d = 6 if sq == 300 else 40, 64
+    q, k, v = _inputs(1, h, sq, sq, d)
+    k[..., ::2] = 0.0
+    q[..., 1::2] *= np.float32(2.0**-122)
+    k[..., 1::2] *= np.float32(2.0**122)
+    want = O.sdpa_f64(*(np.ascontiguousarray(x[:, :2]) for x in (q, k, v)), False)
+    assert O.max_rel_err(_run(dev, q, k, v, False)[:, :2], want) <= TOL
+    q[...], k[...], v[...] = 0.0, 0.0, 0.0
+    q[..., 0] = 8.0
+    k[..., 17, 0] = -86.0  # scores / sqrt(64): probability e^-86 / (sq - 1 + e^-86)
+    v[..., 17, :] = np.float32(2.0**100) * np.arange(1, d + 1, dtype=np.float32)
+    want = math.exp(-86.0) / (sq - 1) * v[..., 17, :].astype(np.float64)
+    got = _run(dev, q, k, v, False)
+    # the exponent's f32 rounding: 124 2^-24 ln 2 and as much again for the score and the sum
+    assert np.max(np.abs(got / want[:, :, None, :] - 1.0)) <= 2e-5

@@ -104,6 +104,40 @@ def test_ends_of_the_range(dev, sa, sb):
     _check_f32_sums(_ex(dev, a, b, 0), a, b)
 
 
+# m, n, k and what bch_sgemm runs there (None: the rows kernel, which takes up to 64 rows of other K or alignment)
+KERNELS = [(256, 256, 256, "sgemm_mfma_kernel<64,64,64,false>"), (160, 144, 128, "sgemm_small_kernel"),
+           (300, 260, 4096, "sgemm_mfma_kernel<128,128,32,true,v4>+sgemm_splitk_reduce"),
+           (2048, 2048, 96, "sgemm_mfma_kernel<128,128,32,false>"),
+           (2047, 2045, 95, "sgemm_mfma_kernel<128,128,32,true>"),
+           (8192, 1024, 64, "sgemm_mfma_kernel<256,128,32,false>"), (4096, 4096, 64, "sgemm_mfma_kernel<256,256,32,false>"),
+           (4095, 4090, 95, "sgemm_mfma_kernel<256,256,32,true>"),
+           (3072, 3072, 512, "sgemm_mfma_kernel<128,128,32,false,hyb>+sgemm_tail_reduce"), (20, 301, 333, None),
+           (50, 301, 2049, None)]
+
+
+@pytest.mark.parametrize("transb", [0, 1])
+@pytest.mark.parametrize("m,n,k,kernel", KERNELS)
+def test_tiny_elements_beside_ordinary_ones(dev, m, n, k, kernel, transb):
+    """Elements down to the subnormals in rows (columns) that also hold ordinary ones, against zeros
+    there and large elements elsewhere: every element counts to f32 accuracy, whatever else its
+    row holds."""
+    if kernel is not None:
+        assert dev._lib.bch_sgemm_kernel_name(m, n, k).decode() == kernel
+    rng = np.random.default_rng(m + k)
+    for e, f, swap in ((-118, 100, False), (-125, 120, False), (-140, 120, False), (-125, 120, True)):
+        print(f"tiny elements m={m} n={n} k={k} transb={transb} 2^{e} 2^{f} swap={swap}", flush=True)
+        a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+        tiny = rng.random(k) < 0.5
+        tiny[0], tiny[k - 1] = False, True
+        if swap:
+            b[tiny] *= np.float32(2.0**e)
+            a[:, ~tiny], a[:, tiny] = 0.0, a[:, tiny] * np.float32(2.0**f)
+        else:
+            a[:, tiny] *= np.float32(2.0**e)
+            b[~tiny], b[tiny] = 0.0, b[tiny] * np.float32(2.0**f)
+        _check_f32_sums(_ex(dev, a, np.ascontiguousarray(b.T) if transb else b, transb), a, b)
+
+
 def test_one_huge_element_in_a_row(dev):
     """Parts keep each element's own exponent: a row with one element 2^60 times the others, and a
     zero in B against it, still has the others' product to f32 accuracy."""
