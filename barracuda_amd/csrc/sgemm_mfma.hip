@@ -107,6 +107,108 @@ __device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
   }
 }
 
+// ---- where the parts cannot stand for the floats: again on v_mfma_f32_32x32x2_f32 ----
+// Operands that are infinite, NaN or 2^111 and more, and sums from 2^96, leave values that are not
+// finite.  Whether any of a wavefront's NB blocks holds one; if so want[b / TN] gets bit 16 (b % TN)
+// + r for each such value r of block b.
+template <int NB, int TN>
+__device__ __forceinline__ bool non_finite(const f32x16* x, unsigned* want) {
+  static_assert(16 * TN <= 32, "a bit a value");
+  float z = 0.0f;
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) z = fmaf(x[b][r], 0.0f, z);
+#pragma unroll
+  for (int i = 0; i < NB / TN; ++i) want[i] = 0;
+  if (!__any(z != 0.0f)) return false;
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      want[b / TN] |= __builtin_isfinite(x[b][r]) ? 0u : 1u << (16 * (b % TN) + r);
+  return true;
+}
+
+// sum: the product of this lane's row at qa and its columns at qb, TN blocks of a block row, by one
+// wavefront straight from global memory.  Chunk c of nc is the 16 k from kof(c), then come the k
+// from kr to K: lane half lh loads 8 consecutive k of its row and columns and step e contracts k e
+// and 8 + e; two chunks are in flight.  Ends once every wanted value is NaN, which no further k
+// changes.  A wavefront reads its panels alone, 10 bytes of L2 traffic per 100 FLOP: a few block
+// rows cost their latency, a whole matrix twice the f32 instruction's time.  Measured (us, one
+// box; a kernel on that instruction throughout / a k pair loaded, then multiplied, at a time /
+// this): 4096^3 with one NaN in A 938 / 3230 / 736, with a row of NaN in B at half of k 997 / 3170 /
+// 1553, with every sum past 2^96 936 / 3410 / 2390; 1024^3 with one NaN 27 / 105 / 38; 512 x 4096 x
+// 11008 with one NaN 382 / 1140 / 251.  Fewer k than a pass: 4096 x 4096 x 8 22 / 17 / 19, x 31
+// 29 / 19 / 19, 512 x 512 x 8 7.1 / 6.2 / 7.9, x 31 9.4 / 9.9 / 10.1.
+template <int TN, bool TB, class KOf>
+__device__ __forceinline__ void redo_f32(unsigned want, int nc, KOf&& kof, int kr, int K, int lh, const float* qa,
+                                         const float* const (&qb)[TN], int ldb, f32x16 (&sum)[TN]) {
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sum[j][r] = 0.0f;
+  float a[2][8], b[2][TN][8];
+  auto load = [&](int s, int c) {
+    const int k0 = kof(min(c, nc - 1)) + 8 * lh;
+    load8<false>(qa + k0, a[s]);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      if constexpr (TB) {
+        load8<false>(qb[j] + k0, b[s][j]);
+      } else {
+        const float* p = qb[j] + (long long)k0 * ldb;
+#pragma unroll
+        for (int e = 0; e < 8; ++e, p += ldb) b[s][j][e] = *p;
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto step = [&](int s, int e) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      sum[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s][e], b[s][j][e], sum[j], 0, 0, 0);
+  };
+  auto multiply = [&](int s) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) step(s, e);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (nc > 0) load(0, 0);
+#pragma unroll 1
+  for (int c = 0; c < nc; c += 2) {
+    load(1, c + 1);
+    multiply(0);
+    load(0, c + 2);
+    if (c + 1 < nc) multiply(1);
+    unsigned nan = 0;
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) nan |= sum[j][r] != sum[j][r] ? 1u << (16 * j + r) : 0u;
+    if (!__any((want & ~nan) != 0)) return;
+  }
+#pragma unroll 1
+  for (int kb = kr; kb < K; kb += 16) {  // step e: k 2 e and 2 e + 1, zeros from K on
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (kb + 2 * e < K) {
+        const int k = kb + 2 * e + lh, kc = min(k, K - 1);
+        const float x = qa[kc];
+        a[0][e] = k < K ? x : 0.0f;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const float y = TB ? qb[j][kc] : qb[j][(long long)kc * ldb];
+          b[0][j][e] = k < K ? y : 0.0f;
+        }
+      }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (kb + 2 * e < K) step(0, e);
+  }
+}
+
 // CHECK: any sizes (rows and columns outside the matrix are read from its last ones and not
 // stored; a k remainder is taken by the first pass).  V4: 16-byte aligned rows.
 template <int BM, int BN, int BK, bool CHECK, bool TB, bool EPI, bool V4 = false, bool HY = false>
@@ -366,7 +468,7 @@ __global__ __launch_bounds__((Cfg<BM, BN, BK>::NT)) void sgemm_mfma_kernel(
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  // Fewer k than one pass holds (K = 0 too): the f32 loop below alone, at most KS / 2 steps.
+  // Fewer k than one pass holds (K = 0 too): redo_f32 alone.
   const bool short_k = K < KS;
   if (!short_k) {
     if (rest)
@@ -394,60 +496,23 @@ __global__ __launch_bounds__((Cfg<BM, BN, BK>::NT)) void sgemm_mfma_kernel(
     f32x16* const part = reinterpret_cast<f32x16*>(smem) + (wave % (G::WM * G::WN)) * 64 + lane;
     if (kg != 0) *part = acc[0][0];
     __syncthreads();
-    if (kg == 0) acc[0][0] += *part;
+    if (kg != 0) return;
+    acc[0][0] += *part;
   }
 
-  // ---- scaled back; where the parts cannot stand for the floats, the tile again in f32 ----
-  // An operand that is infinite, NaN or 2^111 and more, or a sum from 2^96, leaves a result that is
-  // not finite.  The wavefront then redoes its blocks on v_mfma_f32_32x32x2_f32 from global memory.
-  bool redo = short_k;
-  {
-    float z = 0.0f;
+  // ---- scaled back; `want`: the values to compute again in f32 ----
+  unsigned want[TM];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        acc[i][j] *= bch::kSplitUnscale;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) z = fmaf(acc[i][j][r], 0.0f, z);
-      }
-    redo |= __any(z != 0.0f);  // NaN
-  }
-  if (G::KG > 1 && kg != 0) return;
-  if (redo) {
-    const float* qb[TN];
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int n = min(n0 + wn + j * 32 + li, N - 1);
-      qb[j] = TB ? B + (long long)n * ldb : B + n;
-    }
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const float* qa = A + (long long)min(m0 + wm + i * 32 + li, M - 1) * lda;
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-#pragma unroll 1
-      for (int k0 = 0; k0 < K; k0 += 2) {
-        const int k = min(k0 + lh, K - 1);
-        const bool in = k0 + lh < K;
-        const float va = qa[k];
-        const float a = in ? va : 0.0f;
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const float vb = TB ? qb[j][k] : qb[j][(long long)k * ldb];
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, in ? vb : 0.0f, acc[i][j], 0, 0, 0);
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
+    for (int j = 0; j < TN; ++j) acc[i][j] *= bch::kSplitUnscale;
+  const bool redo = non_finite<TM * TN, TN>(&acc[0][0], want) || short_k;
 
   // ---- epilogue: value r of lane l is row 8*(r/4) + 4*lh + r%4, col li ----
+  float* Pt = nullptr;
   if constexpr (HY) {
     if (tail) {  // the slice's sums, a whole BM x BN tile, into its slot of the partials
-      float* Pt = hy_P + ((long long)hy_slice * hy_r + hy_slot) * (BM * BN);
+      Pt = hy_P + ((long long)hy_slice * hy_r + hy_slot) * (BM * BN);
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -455,12 +520,12 @@ __global__ __launch_bounds__((Cfg<BM, BN, BK>::NT)) void sgemm_mfma_kernel(
 #pragma unroll
           for (int r = 0; r < 16; ++r)
             Pt[(wm + i * 32 + 8 * (r >> 2) + 4 * lh + (r & 3)) * BN + wn + j * 32 + li] = acc[i][j][r];
-      return;
     }
   }
+  const bool store = !short_k && !(HY && tail);
   if constexpr (!EPI) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
+    for (int i = 0; i < TM && store; ++i) {
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
         const int col = n0 + wn + j * 32 + li;
@@ -472,7 +537,7 @@ __global__ __launch_bounds__((Cfg<BM, BN, BK>::NT)) void sgemm_mfma_kernel(
         __builtin_amdgcn_sched_barrier(0);  // one block's addresses at a time: no spills
       }
     }
-  } else {
+  } else if (store) {
     // bias and the activation are uniform over the launch (no divergence); one 32 x 32
     // block at a time, so only 16 accumulators are out of the AGPRs at once
 #pragma unroll
@@ -489,6 +554,41 @@ __global__ __launch_bounds__((Cfg<BM, BN, BK>::NT)) void sgemm_mfma_kernel(
           if (!CHECK || (row < M && col < N)) C[(long long)row * ldc + col] = v;
         }
         __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  if (!redo) return;
+
+  // ---- the values that were not finite (all of a call with fewer k than a pass) again in f32 ----
+  // After the stores and one block row at a time in a loop that is not unrolled: the accumulators'
+  // registers are free, and the loop above keeps its own.
+#pragma unroll 1
+  for (int i = 0; i < TM; ++i) {
+    unsigned w = 0;
+#pragma unroll
+    for (int ii = 0; ii < TM; ++ii) w = i == ii ? want[ii] : w;
+    if (short_k) w = ~0u;
+    if (!__any(w != 0)) continue;
+    const float* qb[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int n = min(n0 + wn + j * 32 + li, N - 1);
+      qb[j] = TB ? B + (long long)n * ldb : B + n;
+    }
+    f32x16 sum[TN];
+    redo_f32<TN, TB>(w, K / 16, [](int c) { return 16 * c; }, K / 16 * 16, K, lh, A + (long long)min(m0 + wm + i * 32 + li, M - 1) * lda, qb, ldb, sum);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int lc = wn + j * 32 + li, col = n0 + lc;
+      const float bj = EPI && bias && col < N ? bias[col] : 0.0f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int lr = wm + i * 32 + 8 * (r >> 2) + 4 * lh + (r & 3), row = m0 + lr;
+        if (!(w >> (16 * j + r) & 1u)) continue;
+        if (HY && tail)
+          Pt[lr * BN + lc] = sum[j][r];
+        else if (row < M && col < N)
+          C[(long long)row * ldc + col] = EPI ? bch::activate(sum[j][r] + bj, act) : sum[j][r];
       }
     }
   }
@@ -1136,23 +1236,16 @@ __global__ __launch_bounds__(512, 4) void sgemm_small_kernel(int M, int N, int K
     u += W;
   }
 
-  // ---- where the parts cannot stand for the floats (as for the large tiles), again in f32 ----
+  // ---- scaled back; values that are not finite again in f32, this wavefront's units ----
   acc *= bch::kSplitUnscale;
-  float z = 0.0f;
+  unsigned want;
+  if (non_finite<1, 1>(&acc, &want)) {
+    const float* const qb[1] = {pb};
+    f32x16 sum[1];
+    redo_f32<1, TB>(want, 2 * ((nf - wave + W - 1) / W), [&](int c) { return 32 * (wave + W * (c >> 1)) + 16 * (c & 1); },
+                    wave == nf % W ? 32 * nf : K, K, lh, pa, qb, ldb, sum);
 #pragma unroll
-  for (int r = 0; r < 16; ++r) z = fmaf(acc[r], 0.0f, z);
-  if (__any(z != 0.0f)) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-#pragma unroll 1
-    for (int v = wave; v < nu; v += W)
-#pragma unroll 1
-      for (int k0 = 32 * v; k0 < min(32 * v + 32, K); k0 += 2) {
-        const int k = min(k0 + lh, K - 1);
-        const bool in = k0 + lh < K;
-        const float x = pa[k], y = TB ? pb[k] : pb[(long long)k * ldb];
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? x : 0.0f, in ? y : 0.0f, acc, 0, 0, 0);
-      }
+    for (int r = 0; r < 16; ++r) acc[r] = want >> r & 1u ? sum[0][r] : acc[r];
   }
 
   // ---- the eight blocks added in wavefront order, two values a thread ----
@@ -1343,6 +1436,7 @@ __global__ __launch_bounds__(512, 4) void sgemm_rows_kernel(int M, int N, int K,
   }
 
   // ---- the two halves of k added up ----
+  const int col = n0 + wn + li;
   __syncthreads();  // the last pass's reads are done
   f32x16* const part = reinterpret_cast<f32x16*>(lds) + (wave & 3) * (64 * TM) + lane;
   if (kg != 0) {
@@ -1351,39 +1445,33 @@ __global__ __launch_bounds__(512, 4) void sgemm_rows_kernel(int M, int N, int K,
   }
   __syncthreads();
   if (kg != 0) return;
-  float zf = 0.0f;
 #pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    acc[i] = (acc[i] + part[64 * i]) * bch::kSplitUnscale;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) zf = fmaf(acc[i][r], 0.0f, zf);
-  }
-  const int col = n0 + wn + li;
-  if (__any(zf != 0.0f)) {  // as for the large tiles: again in f32
-    const int c = min(col, N - 1);
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const float* qa = A + (long long)min(32 * i + li, M - 1) * lda;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
-#pragma unroll 1
-      for (int k0 = 0; k0 < K; k0 += 2) {
-        const int k = min(k0 + lh, K - 1);
-        const bool in = k0 + lh < K;
-        const float va = qa[k], vb = TB ? B[(long long)c * ldb + k] : B[(long long)k * ldb + c];
-        acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? va : 0.0f, in ? vb : 0.0f, acc[i], 0, 0, 0);
-      }
-    }
-  }
-  if (col >= N) return;
-  const float bj = bias ? bias[col] : 0.0f;
+  for (int i = 0; i < TM; ++i) acc[i] = (acc[i] + part[64 * i]) * bch::kSplitUnscale;
+  unsigned want[TM];
+  const bool redo = non_finite<TM, 1>(acc, want);
+  const float bj = bias && col < N ? bias[col] : 0.0f;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int row = 32 * i + 8 * (r >> 2) + 4 * lh + (r & 3);
-      if (row < M) C[(long long)row * ldc + col] = bch::activate(acc[i][r] + bj, act);
+      if (row < M && col < N) C[(long long)row * ldc + col] = bch::activate(acc[i][r] + bj, act);
     }
+  if (!redo) return;
+#pragma unroll 1
+  for (int i = 0; i < TM; ++i) {  // as for the large tiles: again in f32, after the stores
+    const unsigned w = i == 0 ? want[0] : want[TM - 1];
+    if (!__any(w != 0)) continue;
+    const float* const qb[1] = {TB ? B + (long long)min(col, N - 1) * ldb : B + min(col, N - 1)};
+    f32x16 sum[1];
+    redo_f32<1, TB>(w, K / 16, [](int c) { return 16 * c; }, K / 16 * 16, K, lh,
+                       A + (long long)min(32 * i + li, M - 1) * lda, qb, ldb, sum);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int row = 32 * i + 8 * (r >> 2) + 4 * lh + (r & 3);
+      if ((w >> r & 1u) && row < M && col < N) C[(long long)row * ldc + col] = bch::activate(sum[0][r] + bj, act);
+    }
+  }
 }
 
 // Two workgroups per CU resident at once, slices of 4 passes or more; the partials stay under the

@@ -14,7 +14,7 @@ from tests.test_gpu_graph import CAPTURE_RELAXED, _FreshCtx, _hip
 pytestmark = pytest.mark.gpu
 
 
-def _ex(dev, a, b, transb, lda=None, ldb=None, a_off=0, b_off=0):
+def _ex(dev, a, b, transb, lda=None, ldb=None, a_off=0, b_off=0, bias=None, act=0):
     """bch_sgemm_ex on copies of a and b with the given leading dimensions and start offsets."""
     m, k = a.shape
     n = b.shape[0] if transb else b.shape[1]
@@ -26,8 +26,10 @@ def _ex(dev, a, b, transb, lda=None, ldb=None, a_off=0, b_off=0):
         return Tensor.from_data(buf, [buf.size], dev)
 
     ta, tb, tc = put(a, lda, a_off), put(b, ldb, b_off), Tensor.empty([m, n], dev)
+    tbias = None if bias is None else Tensor.from_data(bias, [n], dev)
     dev.check(dev._lib.bch_sgemm_ex(dev.ctx, transb, m, n, k, C.c_void_p(ta.ptr + 4 * a_off), lda,
-                                    C.c_void_p(tb.ptr + 4 * b_off), ldb, None, 0, C.c_void_p(tc.ptr), n), "linear")
+                                    C.c_void_p(tb.ptr + 4 * b_off), ldb, tbias and C.c_void_p(tbias.ptr), act,
+                                    C.c_void_p(tc.ptr), n), "linear")
     return tc.to_numpy()
 
 
@@ -136,6 +138,63 @@ def test_tiny_elements_beside_ordinary_ones(dev, m, n, k, kernel, transb):
             a[:, tiny] *= np.float32(2.0**e)
             b[~tiny], b[tiny] = 0.0, b[tiny] * np.float32(2.0**f)
         _check_f32_sums(_ex(dev, a, np.ascontiguousarray(b.T) if transb else b, transb), a, b)
+
+
+@pytest.mark.parametrize("epilogue", [False, True])
+@pytest.mark.parametrize("transb", [0, 1])
+@pytest.mark.parametrize("m,n,k,kernel", KERNELS)
+def test_values_computed_again_in_f32(dev, m, n, k, kernel, transb, epilogue):
+    """What the parts cannot stand for, on every kernel and k-slice: infinities and NaN anywhere in k,
+    a row and a column of nothing but NaN, operands from 2^111 and sums from 2^96.  Integers times
+    powers of two, so every value is exact; its neighbours keep theirs."""
+    if kernel is not None:
+        assert dev._lib.bch_sgemm_kernel_name(m, n, k).decode() == kernel
+    print(f"again in f32 m={m} n={n} k={k} transb={transb} epilogue={epilogue}", flush=True)
+    rng = np.random.default_rng(m + k)
+    a, b = (rng.integers(-8, 9, s).astype(np.float32) for s in ((m, k), (k, n)))
+    a[3, k // 3], a[m - 2, 0], a[m // 2, k - 1], a[m // 3] = np.inf, -np.inf, np.nan, np.nan
+    b[k // 2, 7], b[k - 1, n - 1], b[:, n // 2] = -np.inf, np.nan, np.nan
+    a[5] *= np.float32(2.0**108)
+    a[m - 1, k // 2] = np.float32(2.0**112)
+    b[:, 40] *= np.float32(2.0**100)
+    bias = rng.integers(-8, 9, n).astype(np.float32) if epilogue else None
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = np.empty((m, n))
+        fa, fb = np.where(np.isfinite(a), a, 0.0).astype(np.float64), np.where(np.isfinite(b), b, 0.0).astype(np.float64)
+        want[:] = fa @ fb
+        # rows and columns that hold infinities or NaN, term by term
+        for r in np.flatnonzero(~np.isfinite(a).all(1)):
+            want[r] = (a[r].astype(np.float64)[:, None] * b.astype(np.float64)).sum(0)
+        for c in np.flatnonzero(~np.isfinite(b).all(0)):
+            want[:, c] = (a.astype(np.float64) * b[:, c].astype(np.float64)).sum(1)
+        want = want.astype(np.float32)
+        if epilogue:
+            want = want + bias
+            want = np.where(want > 0, want, np.where(np.isnan(want), want, np.float32(0.0)))
+    got = _ex(dev, a, np.ascontiguousarray(b.T) if transb else b, transb, bias=bias, act=1 if epilogue else 0)
+    if epilogue:  # the activation's own treatment of NaN: what a product of few k gives
+        nan = _ex(dev, np.full((1, 1), np.nan, np.float32), np.ones((1, 1), np.float32), 0, bias=np.ones(1, np.float32), act=1)
+        want = np.where(np.isnan(want), nan[0, 0], want)
+    got[5, 40] = want[5, 40] = 0.0  # products beyond the range of f32, of either sign
+    assert np.array_equal(got, want, equal_nan=True)
+
+
+def test_values_computed_again_in_f32_batched(dev):
+    """Batches of each kernel that takes them: every batch's own operands."""
+    for batch, m, n, k in ((3, 192, 128, 192), (5, 77, 90, 270), (40, 256, 256, 96), (3, 300, 260, 2111)):
+        print(f"again in f32 batched {batch} {m} {n} {k}", flush=True)
+        rng = np.random.default_rng(k)
+        a, b = (rng.integers(-8, 9, s).astype(np.float32) for s in ((batch, m, k), (batch, k, n)))
+        for i in range(batch):
+            a[i, (7 * i) % m, (11 * i) % k] = np.inf if i % 2 else np.nan
+            b[i, :, (3 * i) % n] *= np.float32(2.0**100)
+        with np.errstate(invalid="ignore"):
+            want = np.matmul(a.astype(np.float64), b.astype(np.float64)).astype(np.float32)
+            for i in range(batch):
+                r = (7 * i) % m
+                want[i, r] = (a[i, r].astype(np.float64)[:, None] * b[i].astype(np.float64)).sum(0)
+        got = Tensor.from_data(a, list(a.shape), dev).batch_matmul(Tensor.from_data(b, list(b.shape), dev)).to_numpy()
+        assert np.array_equal(got, want, equal_nan=True)
 
 
 def test_one_huge_element_in_a_row(dev):
