@@ -114,3 +114,33 @@ def test_parts_tiny_elements_beside_ordinary_ones(dev, sq):
     got = _run(dev, q, k, v, False)
     # the exponent's f32 rounding: 124 2^-24 ln 2 and as much again for the score and the sum
     assert np.max(np.abs(got / want[:, :, None, :] - 1.0)) <= 2e-5
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("sq,d", [(300, 64), (300, 128), (299, 80), (130, 33), (2048, 32), (2047, 96), (2048, 128)])
+def test_parts_computed_again_in_f32(dev, sq, d, causal):
+    """Infinite and NaN operands and magnitudes past the parts' range, each in a head of its own, on split
+    and whole keys: what f32 arithmetic gives, and the other heads as they are."""
+    print(f"again in f32 sq={sq} d={d} causal={causal}", flush=True)
+    h = 40 if sq > 1000 else 6
+    q, k, v = _inputs(1, h, sq, sq, d)
+    v[0, 0, 0, 3] = np.inf
+    k[0, 1, sq - 1, 1] = np.nan
+    q[0, 2, 7, d - 1] = np.nan
+    q[0, 3] *= np.float32(2.0**50)
+    k[0, 3] *= np.float32(2.0**-50)
+    v[0, 4] *= np.float32(2.0**110)
+    got = _run(dev, q, k, v, causal)[0, :6].astype(np.float64)
+    q, k, v = (x[0, :6].astype(np.float64) for x in (q, k, v))
+    s = (q @ k.transpose(0, 2, 1)) / math.sqrt(d)
+    if causal:
+        s = np.where(np.triu(np.ones((sq, sq), bool), 1), -np.inf, s)
+    with np.errstate(invalid="ignore"):
+        p = np.exp(s - s.max(-1, keepdims=True))
+        want = (p / p.sum(-1, keepdims=True)) @ v
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isinf(got), np.isinf(want))
+    fin = np.isfinite(want)
+    got, want = np.where(fin, got, 0.0), np.where(fin, want, 0.0)
+    for head in range(6):
+        assert np.max(np.abs(got[head] - want[head])) <= TOL * max(np.max(np.abs(want[head])), 1e-30), head
