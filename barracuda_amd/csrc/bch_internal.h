@@ -179,23 +179,24 @@ const char* softmax_f64_kernel_name(long long rows, long long cols,
                                     bool aligned16);
 
 // C[b] = A[b] . B[b] (row-major), b < batch.  ws/ws_bytes: device scratch
-// of at least sgemm_workspace_bytes(batch, m, n, k) bytes.
+// of sgemm_workspace_bytes(batch, m, n, k) bytes, or as few as sgemm_reserved_bytes.
 hipError_t launch_sgemm(hipStream_t s, int batch, int m, int n, int k,
                         const float* A, int lda, long long sA,
                         const float* B, int ldb, long long sB,
                         float* C, int ldc, long long sC, void* ws,
                         size_t ws_bytes);
 size_t sgemm_workspace_bytes(int batch, int m, int n, int k);
-// The part of it a launch cannot do without (the skinny paths' and split-K's
-// partials); with less than sgemm_workspace_bytes the hybrid plan is skipped.
-size_t sgemm_required_workspace_bytes(int batch, int m, int n, int k);
 // Scratch of launch_sgemm_ex (the skinny paths' and rows kernel's partials, split-K partials, or the
 // hybrid plan's).
 size_t sgemm_ex_workspace_bytes(bool transb, int batch, int m, int n, int k, const float* A, int lda, const float* B,
                                 int ldb);
-// Whether a call whose workspace may not grow runs all the same, unsplit (the tile path, except
-// where its plan has always needed the workspace).
-bool sgemm_runs_without_workspace(bool transb, int batch, int m, int n, int k, int lda, int ldb);
+// What a call must find where the workspace may not grow (sgemm_reserve.hip); with that much, and
+// less than the sizes above, it runs with fewer k slices or none.  fixed: what bch_sgemm_noalloc
+// needs of its scratch.
+constexpr size_t kSgemmFixedScratch = (size_t)16 << 20;
+size_t sgemm_reserved_bytes(bool transb, int batch, int m, int n, int k, int lda, int ldb, bool fixed = false);
+// 32 < m <= 64 rows of [n][k] weights as two passes of the 32-row kernels
+bool sgemm_nt_two_pass(int m, int n, int k, const float* A, int lda, const float* B, int ldb);
 const char* sgemm_kernel_name(int m, int n, int k);
 // With B given as [n][k] when transb (C = A B^T), and the linear layer's
 // epilogue C = act(acc + bias[col]): bias nullable, act kActNone / kActRelu /
@@ -333,9 +334,10 @@ hipError_t launch_sdpa_decode(hipStream_t s, int B, int H, int Hkv, int Sq, int 
 // D > kSdpaFusedMaxD: scores materialised one query chunk at a time (GEMM,
 // scaled and masked row softmax, GEMM) in ws, which must hold
 // sdpa_wide_workspace_bytes(...) bytes (q_row, k_row: the row strides of q
-// and k; 0 when a row stride exceeds 2^31 - 1, which the launch rejects).
+// and k; 0 when a row stride exceeds 2^31 - 1, which the launch rejects);
+// reserved: as few as it runs in (sgemm_reserved_bytes for the products).
 size_t sdpa_wide_workspace_bytes(int Hkv, int Sq, int Skv, int D, int causal,
-                                 long long q_row, long long k_row);
+                                 long long q_row, long long k_row, bool reserved = false);
 hipError_t launch_sdpa_wide(hipStream_t s, int B, int H, int Hkv, int Sq,
                             int Skv, int D, float scale, int causal,
                             const float* q, const float* k, const float* v,

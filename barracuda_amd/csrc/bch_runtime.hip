@@ -32,7 +32,7 @@
 // its own copy until the process ends.  In host code `scratch` names a
 // host-side stand-in, never device memory: the device address is resolved
 // once per device with hipGetSymbolAddress and only that address is used.
-constexpr size_t kNoAllocScratchBytes = (size_t)16 << 20;
+constexpr size_t kNoAllocScratchBytes = bch::kSgemmFixedScratch;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 struct bch_ctx {
@@ -226,6 +226,13 @@ bch_status ensure_ws(bch_ctx* ctx, size_t bytes) {
   // states are written before they are read); the clear only keeps a fresh
   // workspace deterministic for debugging.
   return from_hip(ctx, hipMemsetAsync(ctx->ws, 0, want, ctx->stream), "workspace clear");
+}
+
+// Workspace for a call that runs in `want` bytes and, slower, in `must`: grown to `want`; where it
+// may not grow, a call that finds `must` runs with what there is.
+bch_status size_ws(bch_ctx* ctx, size_t want, size_t must) {
+  if (capturing(ctx)) return ensure_ws(ctx, must);
+  return ensure_ws(ctx, std::max(want, must));
 }
 
 bool fail_alloc_injected() {
@@ -538,13 +545,9 @@ bch_status bch_sgemm_ex(bch_ctx* ctx, int transb, int m, int n, int k, const flo
   if (!C || (k > 0 && (!A || !B))) return fail(ctx, BCH_E_INVALID, "linear: NULL buffer");
   bch_status st = use(ctx);
   if (st != BCH_OK) return st;
-  size_t wsb = bch::sgemm_ex_workspace_bytes(transb != 0, 1, m, n, k, A, lda, B, ldb);
-  if (wsb > ctx->ws_bytes && capturing(ctx) && bch::sgemm_runs_without_workspace(transb != 0, 1, m, n, k, lda, ldb))
-    wsb = 0;
-  if (wsb) {
-    st = ensure_ws(ctx, wsb);
-    if (st != BCH_OK) return st;
-  }
+  st = size_ws(ctx, bch::sgemm_ex_workspace_bytes(transb != 0, 1, m, n, k, A, lda, B, ldb),
+               bch::sgemm_reserved_bytes(transb != 0, 1, m, n, k, lda, ldb));
+  if (st != BCH_OK) return st;
   hipError_t e = bch::launch_sgemm_ex(ctx->stream, transb != 0, 1, m, n, k, A, lda, 0, B, ldb, 0, bias, act, C,
                                       ldc, 0, ctx->ws, ctx->ws_bytes);
   return from_hip(ctx, e, "linear launch");
@@ -566,12 +569,9 @@ bch_status bch_sgemm(bch_ctx* ctx, int m, int n, int k, const float* A, int lda,
   if (!C || (k > 0 && (!A || !B))) return fail(ctx, BCH_E_INVALID, "matmul: NULL buffer");
   bch_status st = use(ctx);
   if (st != BCH_OK) return st;
-  size_t wsb = bch::sgemm_ex_workspace_bytes(false, 1, m, n, k, A, lda, B, ldb);
-  if (wsb > ctx->ws_bytes && capturing(ctx) && bch::sgemm_runs_without_workspace(false, 1, m, n, k, lda, ldb)) wsb = 0;
-  if (wsb) {
-    st = ensure_ws(ctx, wsb);
-    if (st != BCH_OK) return st;
-  }
+  st = size_ws(ctx, bch::sgemm_ex_workspace_bytes(false, 1, m, n, k, A, lda, B, ldb),
+               bch::sgemm_reserved_bytes(false, 1, m, n, k, lda, ldb));
+  if (st != BCH_OK) return st;
   hipError_t e = bch::launch_sgemm(ctx->stream, 1, m, n, k, A, lda, 0, B, ldb, 0, C, ldc, 0,
                                    ctx->ws, ctx->ws_bytes);
   return from_hip(ctx, e, "matmul launch");
@@ -591,7 +591,7 @@ bch_status bch_sgemm_noalloc(bch_ctx* ctx, int m, int n, int k, const float* A, 
   if (st != BCH_OK) return st;
   // sized with this device current (the stream-K plans take one workgroup per CU); the tile
   // path's optional hybrid-plan scratch is used when it fits in the fixed scratch
-  const size_t wsb = bch::sgemm_required_workspace_bytes(1, m, n, k);
+  const size_t wsb = bch::sgemm_reserved_bytes(false, 1, m, n, k, k, n, true);
   if (wsb > kNoAllocScratchBytes)
     return fail(ctx, BCH_E_UNSUPPORTED,
                 "matmul (no-alloc): m=%d n=%d k=%d needs %zu bytes of scratch, more than the fixed %zu",
@@ -617,12 +617,9 @@ bch_status bch_sgemm_strided_batched(bch_ctx* ctx, int batch, int m, int n, int 
   if (batch > 65535) return fail(ctx, BCH_E_UNSUPPORTED, "batch_matmul: batch %d > 65535", batch);
   bch_status st = use(ctx);
   if (st != BCH_OK) return st;
-  size_t wsb = bch::sgemm_workspace_bytes(batch, m, n, k);
-  if (wsb > ctx->ws_bytes && capturing(ctx) && bch::sgemm_runs_without_workspace(false, batch, m, n, k, k, n)) wsb = 0;
-  if (wsb) {
-    st = ensure_ws(ctx, wsb);
-    if (st != BCH_OK) return st;
-  }
+  st = size_ws(ctx, bch::sgemm_workspace_bytes(batch, m, n, k),
+               bch::sgemm_reserved_bytes(false, batch, m, n, k, k, n));
+  if (st != BCH_OK) return st;
   const int lda = k > 0 ? k : 1, ldb = n, ldc = n;
   hipError_t e = bch::launch_sgemm(ctx->stream, batch, m, n, k, A, lda, strideA, B, ldb, strideB, C,
                                    ldc, strideC, ctx->ws, ctx->ws_bytes);
@@ -795,7 +792,8 @@ bch_status sdpa_run(bch_ctx* ctx, int B, int H, int Hkv, int Sq, int Skv, int D,
   if (Hkv > 65535)
     return fail(ctx, BCH_E_UNSUPPORTED, "attention: head dimension %d > %d needs at most 65535 key/value heads", D,
                 bch::kSdpaFusedMaxD);
-  st = ensure_ws(ctx, bch::sdpa_wide_workspace_bytes(Hkv, Sq, Skv, D, causal, s.q.row, s.k.row));
+  st = size_ws(ctx, bch::sdpa_wide_workspace_bytes(Hkv, Sq, Skv, D, causal, s.q.row, s.k.row),
+               bch::sdpa_wide_workspace_bytes(Hkv, Sq, Skv, D, causal, s.q.row, s.k.row, true));
   if (st != BCH_OK) return st;
   return from_hip(ctx,
                   bch::launch_sdpa_wide(ctx->stream, B, H, Hkv, Sq, Skv, D, scale, causal, q, k, v, o, s, ctx->ws,

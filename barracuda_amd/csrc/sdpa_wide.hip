@@ -71,8 +71,8 @@ void chunk_shape(const WidePlan& p, int Sq, int Skv, bool causal, int r0, int& m
 }
 
 // lda / ldb: the row strides of q and k (the [n][k] operand), which pick the
-// GEMM's path for the first product.
-WidePlan wide_plan(int Hkv, int Sq, int Skv, int D, bool causal, int lda, int ldb) {
+// GEMM's path for the first product.  reserved: the least scratch that the products run in.
+WidePlan wide_plan(int Hkv, int Sq, int Skv, int D, bool causal, int lda, int ldb, bool reserved) {
   WidePlan p;
   const size_t per_row = (size_t)Hkv * Skv * sizeof(float);
   long long rows = (long long)std::max<size_t>(1, kWideScoreCap / per_row);
@@ -90,8 +90,10 @@ WidePlan wide_plan(int Hkv, int Sq, int Skv, int D, bool causal, int lda, int ld
   for (int r0 = 0; r0 < Sq; r0 += p.rows) {
     int m, n;
     chunk_shape(p, Sq, Skv, causal, r0, m, n);
-    x = std::max(x, bch::sgemm_ex_workspace_bytes(true, Hkv, m, n, D, nullptr, lda, nullptr, ldb));
-    x = std::max(x, bch::sgemm_workspace_bytes(Hkv, m, D, n));
+    x = std::max(x, reserved ? bch::sgemm_reserved_bytes(true, Hkv, m, n, D, lda, ldb)
+                             : bch::sgemm_ex_workspace_bytes(true, Hkv, m, n, D, nullptr, lda, nullptr, ldb));
+    x = std::max(x, reserved ? bch::sgemm_reserved_bytes(false, Hkv, m, D, n, n, D)
+                             : bch::sgemm_workspace_bytes(Hkv, m, D, n));
     x = std::max(x, bch::softmax_workspace_bytes((long long)Hkv * m, n));
   }
   p.extra_bytes = x;
@@ -102,9 +104,10 @@ WidePlan wide_plan(int Hkv, int Sq, int Skv, int D, bool causal, int lda, int ld
 
 namespace bch {
 
-size_t sdpa_wide_workspace_bytes(int Hkv, int Sq, int Skv, int D, int causal, long long q_row, long long k_row) {
+size_t sdpa_wide_workspace_bytes(int Hkv, int Sq, int Skv, int D, int causal, long long q_row, long long k_row,
+                                 bool reserved) {
   if (q_row > 0x7fffffffLL || k_row > 0x7fffffffLL) return 0;
-  const WidePlan p = wide_plan(Hkv, Sq, Skv, D, causal != 0, (int)q_row, (int)k_row);
+  const WidePlan p = wide_plan(Hkv, Sq, Skv, D, causal != 0, (int)q_row, (int)k_row, reserved);
   return p.score_bytes + p.extra_bytes;
 }
 
@@ -116,7 +119,7 @@ hipError_t launch_sdpa_wide(hipStream_t s, int B, int H, int Hkv, int Sq, int Sk
     return hipErrorInvalidValue;
   const int G = H / Hkv;
   const int qr = (int)st.q.row, kr = (int)st.k.row, vr = (int)st.v.row, orow = (int)st.o.row;
-  const WidePlan p = wide_plan(Hkv, Sq, Skv, D, causal != 0, qr, kr);
+  const WidePlan p = wide_plan(Hkv, Sq, Skv, D, causal != 0, qr, kr, true);
   if (ws == nullptr || ws_bytes < p.score_bytes + p.extra_bytes) return hipErrorInvalidValue;
   float* S = static_cast<float*>(ws);
   void* xws = static_cast<char*>(ws) + p.score_bytes;

@@ -753,7 +753,7 @@ const char* tile_name(Tile t, int mode) {
 // 2: 246, no split 381), 512 x 11008 x 4096 as 256 x 256 in 2 245 (256 x 128
 // unsplit 262), 1024 x 1024 x 4096 as 128 x 128 in 4 60 (64 x 64 unsplit 76).
 constexpr size_t kSplitWsMax = (size_t)256 << 20;
-constexpr size_t kSplitWsSmall = (size_t)16 << 20;  // bch_sgemm_noalloc's fixed scratch
+constexpr size_t kSplitWsSmall = bch::kSgemmFixedScratch;
 constexpr int kSplitMinKt = 4;  // k-tiles per slice at least
 constexpr double kTileFixedUs = 3.0;    // an unsplit launch's prologue and stores
 constexpr double kSplitBytesUs = 5e6;   // the partials' round trip
@@ -808,34 +808,6 @@ SplitPlan split_plan(int batch, int m, int n, int k, size_t cap = kSplitWsMax) {
 
 int split_slices(int batch, int m, int n, int k, size_t cap = kSplitWsMax) {
   return split_plan(batch, m, n, k, cap).S;
-}
-
-// Whether a call that needs more workspace than there is, and may not grow it (under capture), is
-// refused rather than run unsplit.  Callers that capture were told to size the workspace first
-// where the plan splits; that holds for the shapes that the split's first rule covered (slices
-// that divide K into 8 k-tiles or more, modelled at the f32 instruction's rate), and shapes that
-// have come to split since still run, unsplit.
-bool split_refused(int batch, int m, int n, int k) {
-  if (k % kBK != 0) return false;
-  const long long cu = bch::device_cu_count();
-  const TileOpt* best = nullptr;
-  double cost = 0.0;
-  for (const TileOpt& o : kTileOpts) {
-    const double c = (double)((tile_count(o, batch, m, n) + cu - 1) / cu) * o.bm * o.bn / o.eff;
-    if (best == nullptr || c < cost * 0.999) {
-      best = &o;
-      cost = c;
-    }
-  }
-  const long long tiles = tile_count(*best, batch, m, n);
-  if (tiles >= cu) return true;  // whole rounds: the hybrid plan's workspace
-  const double tk = 7.4 * best->bm * best->bn / 65536.0 / best->eff, mn = (double)batch * m * n * sizeof(float);
-  const int nk = k / kBK;
-  for (int sl = 2; nk / sl >= 8; ++sl)
-    if (nk % sl == 0 && sl * mn <= (double)kSplitWsMax &&
-        (double)((tiles * sl + cu - 1) / cu) * (nk / sl) * tk + (2.0 * sl + 1.0) * mn / 5e6 + 2.0 < nk * tk)
-      return true;
-  return false;
 }
 
 // ---- small shapes: 64 x 64 x 64 tiles ----
@@ -1526,17 +1498,17 @@ hipError_t launch_rows(hipStream_t s, bool transb, int m, int n, int k, const fl
   return launch_splitk_reduce(s, m, n, p.S, 1, static_cast<const float*>(ws), C, ldc, 0, bias, act);
 }
 
+}  // namespace
+
+namespace bch {
+
 // [n][k] weights with 32 < m <= 64 and n >= 8192: two passes of the m <= 32 path.  Same box,
 // two runs each, against the tile path (bias + ReLU): 33 / 48 / 64 x 11008 x 4096 99.5 / 100.9
 // / 103.0 -> 70.7 / 76.0 / 83.0 us; at n = 4096 the tiles fill the CUs and stay ahead (48 x 4096
 // x 4096 40.0 against 44.1 us, 64 x 4096 x 11008 91.5 against 93.6).
-bool nt_two_pass(int m, int n, int k, const float* A, int lda, const float* B, int ldb) {
-  return m > 32 && m <= 64 && n >= 8192 && bch::sgemm_skinny_nt_applies(32, n, k, A, lda, B, ldb);
+bool sgemm_nt_two_pass(int m, int n, int k, const float* A, int lda, const float* B, int ldb) {
+  return m > 32 && m <= 64 && n >= 8192 && sgemm_skinny_nt_applies(32, n, k, A, lda, B, ldb);
 }
-
-}  // namespace
-
-namespace bch {
 
 static const char* tile_path_name(int m, int n, int k, bool allow_mix);
 
@@ -1587,42 +1559,22 @@ static const char* tile_path_name(int m, int n, int k, bool allow_mix) {
   return tile_name(t, !check ? 0 : v4 ? 1 : 2);
 }
 
-// The tile path's scratch: split-K partials, or the hybrid plan's.  `optional` false: the
-// plan within bch_sgemm_noalloc's 16 MiB (fewer split slices, no hybrid plan).
-static size_t tile_workspace_bytes(int batch, int m, int n, int k, bool optional, bool allow_mix = true) {
+// The tile path's scratch: split-K partials, or the hybrid plan's.
+static size_t tile_workspace_bytes(int batch, int m, int n, int k, bool allow_mix = true) {
   MixPlan mp;
   if (allow_mix && mix_plan(batch, m, n, k, mp))  // the whole tiles need none; the rest is a call of its own
-    return mp.axis == 0 ? tile_workspace_bytes(1, m - mp.split, n, k, optional, false)
-                        : tile_workspace_bytes(1, m, n - mp.split, k, optional, false);
-  const int sl = split_slices(batch, m, n, k, optional ? kSplitWsMax : kSplitWsSmall);
+    return mp.axis == 0 ? tile_workspace_bytes(1, m - mp.split, n, k, false)
+                        : tile_workspace_bytes(1, m, n - mp.split, k, false);
+  const int sl = split_slices(batch, m, n, k);
   if (sl > 1) return (size_t)sl * batch * m * n * sizeof(float);
   HybPlan h;
-  return optional && hyb_plan(batch, m, n, k, h) ? hyb_bytes(h) : 0;
+  return hyb_plan(batch, m, n, k, h) ? hyb_bytes(h) : 0;
 }
 
 size_t sgemm_workspace_bytes(int batch, int m, int n, int k) {
   if (batch == 1 && sgemm_skinny_applies(m, n, k, nullptr, k, nullptr, n))
     return sgemm_skinny_workspace_bytes(m, n, k);
-  return tile_workspace_bytes(batch, m, n, k, true);
-}
-
-size_t sgemm_required_workspace_bytes(int batch, int m, int n, int k) {
-  // 32 < m <= 64 takes the tile path where the skinny partials exceed the small scratch
-  if (batch == 1 && sgemm_skinny_applies(m, n, k, nullptr, k, nullptr, n) &&
-      (m <= 32 || sgemm_skinny_workspace_bytes(m, n, k) <= kSplitWsSmall))
-    return sgemm_skinny_workspace_bytes(m, n, k);
-  return tile_workspace_bytes(batch, m, n, k, false);
-}
-
-bool sgemm_runs_without_workspace(bool transb, int batch, int m, int n, int k, int lda, int ldb) {
-  if (!transb && batch == 1 && sgemm_skinny_applies(m, n, k, nullptr, k, nullptr, n)) return false;
-  if (transb && batch == 1 && (sgemm_skinny_nt_applies(m, n, k, nullptr, lda, nullptr, ldb) ||
-                               nt_two_pass(m, n, k, nullptr, lda, nullptr, ldb)))
-    return false;
-  MixPlan mp;
-  if (mix_plan(batch, m, n, k, mp))
-    return mp.axis == 0 ? !split_refused(1, m - mp.split, n, k) : !split_refused(1, m, n - mp.split, k);
-  return !split_refused(batch, m, n, k);
+  return tile_workspace_bytes(batch, m, n, k);
 }
 
 size_t sgemm_ex_workspace_bytes(bool transb, int batch, int m, int n, int k, const float* A, int lda, const float* B,
@@ -1631,9 +1583,9 @@ size_t sgemm_ex_workspace_bytes(bool transb, int batch, int m, int n, int k, con
   if (!transb) return sgemm_workspace_bytes(batch, m, n, k);
   if (batch == 1 && sgemm_skinny_nt_applies(m, n, k, nullptr, lda, nullptr, ldb))
     return sgemm_skinny_nt_workspace_bytes(m, n, k);
-  if (batch == 1 && nt_two_pass(m, n, k, nullptr, lda, nullptr, ldb))
+  if (batch == 1 && sgemm_nt_two_pass(m, n, k, nullptr, lda, nullptr, ldb))
     return std::max(sgemm_skinny_nt_workspace_bytes(32, n, k), sgemm_skinny_nt_workspace_bytes(m - 32, n, k));
-  return tile_workspace_bytes(batch, m, n, k, true);
+  return tile_workspace_bytes(batch, m, n, k);
 }
 
 hipError_t launch_sgemm(hipStream_t s, int batch, int m, int n, int k, const float* A, int lda, long long sA,
@@ -1671,7 +1623,7 @@ hipError_t launch_sgemm_ex(hipStream_t s, bool transb, int batch, int m, int n, 
     return launch_rows(s, transb, m, n, k, A, lda, B, ldb, C, ldc, bias, act, ws);
   // 32 < m <= 64 with [n][k] weights: the 32-row kernels twice, on rows 0..31 and 32..m-1 (the
   // second pass streams the weights again, largely from the Infinity Cache)
-  if (transb && batch == 1 && nt_two_pass(m, n, k, A, lda, B, ldb)) {
+  if (transb && batch == 1 && sgemm_nt_two_pass(m, n, k, A, lda, B, ldb)) {
     hipError_t e = launch_sgemm_skinny_nt(s, 32, n, k, A, lda, B, ldb, C, ldc, ws, ws_bytes, bias, act);
     if (e != hipSuccess) return e;
     return launch_sgemm_skinny_nt(s, m - 32, n, k, A + 32LL * lda, lda, B, ldb, C + 32LL * ldc, ldc, ws, ws_bytes,

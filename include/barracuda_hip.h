@@ -83,7 +83,10 @@ bch_status bch_ctx_is_lost(const bch_ctx *ctx, int *lost);
  * graph.  Capture only calls whose workspace already exists (make each call
  * once outside the capture first, or bch_ctx_reserve): a call that would
  * have to grow the workspace while the stream is being captured fails with
- * BCH_E_UNSUPPORTED and enqueues nothing.  Once a capture has been seen on
+ * BCH_E_UNSUPPORTED and enqueues nothing.  (What a GEMM must find does not
+ * change with its kernels' plans; one that would run faster with more, and
+ * attention up to D = 256, which needs none, runs with what there is: with
+ * fewer slices of k or of the keys.)  Once a capture has been seen on
  * the context, a later eager call that grows the workspace keeps the old
  * one alive (captured graphs still read it) until bch_ctx_destroy.  Every
  * captured call replays correctly any number of times; replays and eager

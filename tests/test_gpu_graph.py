@@ -254,3 +254,47 @@ def test_reserve_then_capture_allocates_nothing(dev):
             if exe.value:
                 hip.hipGraphExecDestroy(exe)
             hip.hipGraphDestroy(graph)
+
+
+@pytest.mark.parametrize("transb", [0, 1])
+@pytest.mark.parametrize("m,n,k,reserve,accepted", [
+    (8000, 4672, 768, 0, True), (3008, 5440, 544, 0, True),      # whole rounds: the rest's split tiles do without
+    (512, 512, 2628, 0, True), (300, 260, 2999, 0, True),         # split-K of any K: unsplit
+    (300, 260, 4096, 4992000, True), (300, 260, 4096, 4991999, False),  # 16 slices are asked for, 26 are the plan
+    (1024, 1024, 4096, 0, False), (3072, 3072, 3072, 0, False)])
+def test_captured_gemm_needs_the_reserved_workspace_and_no_more(dev, m, n, k, reserve, accepted, transb):
+    """What a GEMM must find under capture is fixed apart from its plans: with less it is refused, with
+    that much it runs, with fewer slices than an eager call or none, and replays exactly."""
+    _say(f"captured GEMM {m} x {n} x {k} transb={transb} with {reserve} bytes: accepted {accepted}")
+    hip = _hip()
+    rng = np.random.default_rng(m + n + k)
+    a, b = (rng.integers(-40, 41, s).astype(np.float32) for s in ((m, k), (n, k) if transb else (k, n)))
+    ta, tb, tc = _up(dev, a), _up(dev, b), Tensor.empty([m, n], dev)
+    with _FreshCtx(dev) as f:
+        if reserve:
+            assert f.lib.bch_ctx_reserve(f.ctx, max(reserve, 1 << 20)) == N.BCH_OK and f.lib.bch_sync(f.ctx) == N.BCH_OK
+        ws = f.ws_bytes()
+        assert ws == reserve
+        graph, exe = C.c_void_p(), C.c_void_p()
+        assert hip.hipStreamBeginCapture(f.stream, CAPTURE_RELAXED) == 0
+        st = f.lib.bch_sgemm_ex(f.ctx, transb, m, n, k, C.c_void_p(ta.ptr), k, C.c_void_p(tb.ptr), b.shape[1], None, 0,
+                                C.c_void_p(tc.ptr), n)
+        assert hip.hipStreamEndCapture(f.stream, C.byref(graph)) == 0
+        assert f.ws_bytes() == ws
+        if not accepted:
+            hip.hipGraphDestroy(graph)
+            assert st == N.BCH_E_UNSUPPORTED
+            return
+        try:
+            assert st == N.BCH_OK, N.last_error(f.ctx)
+            assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, 0) == 0
+            want = (a.astype(np.float64) @ (b.T if transb else b).astype(np.float64)).astype(np.float32)
+            for _ in range(3):
+                dev.upload(tc.ptr, np.full((m, n), np.nan, np.float32))
+                assert hip.hipGraphLaunch(exe, f.stream) == 0
+                assert f.lib.bch_sync(f.ctx) == N.BCH_OK
+                assert np.array_equal(tc.to_numpy(), want)
+        finally:
+            if exe.value:
+                hip.hipGraphExecDestroy(exe)
+            hip.hipGraphDestroy(graph)
