@@ -196,6 +196,36 @@ std::string lib_dir() {
   return ".";
 }
 
+// Workspace blocks are 1 MiB or more.
+size_t ws_block(size_t bytes) { return std::max(bytes, (size_t)1 << 20); }
+
+hipError_t ws_malloc(void** p, size_t bytes) {
+  const char* v = getenv("BARRACUDA_HIP_FAIL_WORKSPACE");
+  return v && v[0] == '1' ? hipErrorOutOfMemory : hipMalloc(p, ws_block(bytes));
+}
+
+bch_status drop_ws(bch_ctx* ctx) {
+  if (!ctx->ws) return BCH_OK;
+  hipError_t e = hipStreamSynchronize(ctx->stream);
+  if (e != hipSuccess) return from_hip(ctx, e, "hipStreamSynchronize");
+  if (ctx->seen_capture)
+    ctx->retired.push_back(ctx->ws);  // captured graphs may still read it
+  else
+    (void)hipFree(ctx->ws);
+  ctx->ws = nullptr;
+  ctx->ws_bytes = 0;
+  return BCH_OK;
+}
+
+bch_status take_ws(bch_ctx* ctx, void* p, size_t bytes) {
+  ctx->ws = p;
+  ctx->ws_bytes = ws_block(bytes);
+  // No kernel relies on the contents (split-k partials and softmax chunk
+  // states are written before they are read); the clear only keeps a fresh
+  // workspace deterministic for debugging.
+  return from_hip(ctx, hipMemsetAsync(p, 0, ctx->ws_bytes, ctx->stream), "workspace clear");
+}
+
 bch_status ensure_ws(bch_ctx* ctx, size_t bytes) {
   if (bytes <= ctx->ws_bytes) return BCH_OK;
   // Growing allocates, and under capture it would also record the clear into
@@ -205,34 +235,32 @@ bch_status ensure_ws(bch_ctx* ctx, size_t bytes) {
                 "workspace of %zu bytes needed while the context's stream is being captured (it holds %zu): "
                 "size it before the capture (an eager call or bch_ctx_reserve) or use bch_sgemm_noalloc",
                 bytes, ctx->ws_bytes);
-  if (ctx->ws) {
-    hipError_t e = hipStreamSynchronize(ctx->stream);
-    if (e != hipSuccess) return from_hip(ctx, e, "hipStreamSynchronize");
-    if (ctx->seen_capture)
-      ctx->retired.push_back(ctx->ws);  // captured graphs may still read it
-    else
-      (void)hipFree(ctx->ws);
-    ctx->ws = nullptr;
-    ctx->ws_bytes = 0;
-  }
-  size_t want = bytes < ((size_t)1 << 20) ? ((size_t)1 << 20) : bytes;
-  hipError_t e = hipMalloc(&ctx->ws, want);
-  if (e != hipSuccess) {
-    ctx->ws = nullptr;
-    return from_hip(ctx, e, "workspace hipMalloc");
-  }
-  ctx->ws_bytes = want;
-  // No kernel relies on the contents (split-k partials and softmax chunk
-  // states are written before they are read); the clear only keeps a fresh
-  // workspace deterministic for debugging.
-  return from_hip(ctx, hipMemsetAsync(ctx->ws, 0, want, ctx->stream), "workspace clear");
+  bch_status st = drop_ws(ctx);
+  if (st != BCH_OK) return st;
+  void* p = nullptr;
+  hipError_t e = ws_malloc(&p, bytes);
+  return e == hipSuccess ? take_ws(ctx, p, bytes) : from_hip(ctx, e, "workspace hipMalloc");
 }
 
 // Workspace for a call that runs in `want` bytes and, slower, in `must`: grown to `want`; where it
-// may not grow, a call that finds `must` runs with what there is.
+// may not grow, or there is no memory for that, a call that finds `must` runs with what there is.
 bch_status size_ws(bch_ctx* ctx, size_t want, size_t must) {
-  if (capturing(ctx)) return ensure_ws(ctx, must);
-  return ensure_ws(ctx, std::max(want, must));
+  if (want <= must || capturing(ctx)) return ensure_ws(ctx, must);
+  if (want <= ctx->ws_bytes) return BCH_OK;
+  // the new block first: without memory for it the old one stays
+  void* p = nullptr;
+  hipError_t e = ws_malloc(&p, want);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    return ensure_ws(ctx, must);
+  }
+  if (e != hipSuccess) return from_hip(ctx, e, "workspace hipMalloc");
+  bch_status st = drop_ws(ctx);
+  if (st != BCH_OK) {
+    (void)hipFree(p);
+    return st;
+  }
+  return take_ws(ctx, p, want);
 }
 
 bool fail_alloc_injected() {
@@ -774,11 +802,8 @@ bch_status sdpa_run(bch_ctx* ctx, int B, int H, int Hkv, int Sq, int Skv, int D,
     const bool decode = bch::sdpa_decode_applies(B, H, Hkv, Sq, Skv, D, causal, q, k, v, s);
     const size_t need = decode ? bch::sdpa_decode_workspace_bytes(B, H, Hkv, Sq, Skv, D)
                                : bch::sdpa_fwd_workspace_bytes(B, H, Sq, Skv, D);
-    if (need > ctx->ws_bytes && !capturing(ctx)) {
-      st = ensure_ws(ctx, need);
-      if (st != BCH_OK && st != BCH_E_OOM) return st;
-      if (st == BCH_E_OOM) (void)hipGetLastError();
-    }
+    st = size_ws(ctx, need, 0);
+    if (st != BCH_OK) return st;
     return from_hip(ctx,
                     decode ? bch::launch_sdpa_decode(ctx->stream, B, H, Hkv, Sq, Skv, D, scale, q, k, v, o, s, ctx->ws,
                                                      ctx->ws_bytes)

@@ -97,7 +97,11 @@ bch_status bch_ctx_stream(const bch_ctx *ctx, void **stream);
  * capture), so that later calls -- captured or not -- need no allocation.
  * *bytes = the workspace's current size (0 for a fresh context).  No
  * counterpart in the reference (its buffer pool is internal); for callers
- * that capture the context's work or must not allocate in a hot loop. */
+ * that capture the context's work or must not allocate in a hot loop.  Out
+ * of memory, a call keeps the workspace it has and runs with that where it
+ * would under capture, else it fails with BCH_E_OOM.  Env
+ * BARRACUDA_HIP_FAIL_WORKSPACE=1 makes every growth report out of memory
+ * (fault injection for that handling). */
 bch_status bch_ctx_reserve(bch_ctx *ctx, size_t bytes);
 bch_status bch_ctx_workspace_bytes(const bch_ctx *ctx, size_t *bytes);
 

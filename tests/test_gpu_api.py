@@ -2,6 +2,7 @@
 reference tests' error paths, and allocation-failure injection."""
 from __future__ import annotations
 
+import ctypes as C
 import os
 import subprocess
 import sys
@@ -10,6 +11,7 @@ import numpy as np
 import pytest
 
 from barracuda_amd import LcgStream, Tensor
+from barracuda_amd import _native as N
 from barracuda_amd.error import ShapeMismatch
 from oracle import bc_oracle as O
 
@@ -303,3 +305,49 @@ def test_ring_combine_timeout_is_reported(monkeypatch):
     assert not good.is_lost()
     del tx, tw, ty
     good.close()
+
+
+def test_workspace_out_of_memory_runs_with_what_there_is(dev, monkeypatch):
+    """Calls whose workspace only makes them faster run without it, and lose none they had; the others
+    report BCH_E_OOM."""
+    from tests.test_gpu_graph import _FreshCtx
+
+    rng = np.random.default_rng(11)
+    lib, P = dev._lib, lambda t: C.c_void_p(t.ptr)
+
+    def gemm(ctx, m, n, k, batch=1):
+        a, b = (rng.integers(-40, 41, s).astype(np.float32) for s in ((batch, m, k), (batch, k, n)))
+        ta, tb, tc = (Tensor.from_data(x, list(x.shape), dev) for x in (a, b, np.zeros((batch, m, n), np.float32)))
+        st = (lib.bch_sgemm(ctx, m, n, k, P(ta), k, P(tb), n, P(tc), n) if batch == 1 else
+              lib.bch_sgemm_strided_batched(ctx, batch, m, n, k, P(ta), m * k, P(tb), k * n, P(tc), m * n))
+        if st == N.BCH_OK:
+            assert lib.bch_sync(ctx) == N.BCH_OK
+            assert np.array_equal(tc.to_numpy(), np.matmul(a.astype(np.float64), b.astype(np.float64)).astype(np.float32))
+        return st
+
+    def attention(ctx, sq, skv, causal):
+        q, k, v = (rng.standard_normal((1, 4, s, 64)).astype(np.float32) for s in (sq, skv, skv))
+        t = [Tensor.from_data(x, list(x.shape), dev) for x in (q, k, v, np.zeros_like(q))]
+        st = lib.bch_sdpa_fwd(ctx, 1, 4, sq, skv, 64, 0.125, causal, *(P(x) for x in t))
+        if st == N.BCH_OK:
+            assert lib.bch_sync(ctx) == N.BCH_OK
+            assert O.max_rel_err(t[3].to_numpy(), O.sdpa_f64(q, k, v, bool(causal))) <= 1e-5
+        return st
+
+    with _FreshCtx(dev) as f:
+        monkeypatch.setenv("BARRACUDA_HIP_FAIL_WORKSPACE", "1")
+        assert gemm(f.ctx, 512, 512, 2628) == N.BCH_OK          # split-K: unsplit
+        assert gemm(f.ctx, 300, 260, 2111, batch=3) == N.BCH_OK
+        assert gemm(f.ctx, 20, 5247, 1001) == N.BCH_OK          # few rows
+        assert attention(f.ctx, 1, 2048, 0) == N.BCH_OK         # split keys: whole
+        assert attention(f.ctx, 300, 300, 1) == N.BCH_OK
+        assert f.ws_bytes() == 0
+        assert gemm(f.ctx, 1024, 1024, 4096) == N.BCH_E_OOM     # has always needed its workspace
+        monkeypatch.delenv("BARRACUDA_HIP_FAIL_WORKSPACE")
+        assert gemm(f.ctx, 512, 512, 2628) == N.BCH_OK
+        ws = f.ws_bytes()
+        assert ws > 0
+        monkeypatch.setenv("BARRACUDA_HIP_FAIL_WORKSPACE", "1")
+        assert gemm(f.ctx, 700, 1200, 1500) == N.BCH_OK         # would take more
+        assert attention(f.ctx, 1500, 1500, 0) == N.BCH_OK
+        assert f.ws_bytes() == ws
