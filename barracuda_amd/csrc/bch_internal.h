@@ -185,11 +185,12 @@ hipError_t launch_sgemm(hipStream_t s, int batch, int m, int n, int k,
                         const float* B, int ldb, long long sB,
                         float* C, int ldc, long long sC, void* ws,
                         size_t ws_bytes);
+// At most, whatever the operands' alignment.
 size_t sgemm_workspace_bytes(int batch, int m, int n, int k);
-// Scratch of launch_sgemm_ex (the skinny paths' and rows kernel's partials, split-K partials, or the
-// hybrid plan's).
-size_t sgemm_ex_workspace_bytes(bool transb, int batch, int m, int n, int k, const float* A, int lda, const float* B,
-                                int ldb);
+// Scratch of launch_sgemm_ex on these operands (the skinny paths' and rows kernel's partials, split-K
+// partials, or the hybrid plan's; none for the small kernels).
+size_t sgemm_ex_workspace_bytes(bool transb, int batch, int m, int n, int k, const float* A, int lda, long long sA,
+                                const float* B, int ldb, long long sB);
 // What a call must find where the workspace may not grow (sgemm_reserve.hip); with that much, and
 // less than the sizes above, it runs with fewer k slices or none.  fixed: what bch_sgemm_noalloc
 // needs of its scratch.

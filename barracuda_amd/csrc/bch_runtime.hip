@@ -573,7 +573,7 @@ bch_status bch_sgemm_ex(bch_ctx* ctx, int transb, int m, int n, int k, const flo
   if (!C || (k > 0 && (!A || !B))) return fail(ctx, BCH_E_INVALID, "linear: NULL buffer");
   bch_status st = use(ctx);
   if (st != BCH_OK) return st;
-  st = size_ws(ctx, bch::sgemm_ex_workspace_bytes(transb != 0, 1, m, n, k, A, lda, B, ldb),
+  st = size_ws(ctx, bch::sgemm_ex_workspace_bytes(transb != 0, 1, m, n, k, A, lda, 0, B, ldb, 0),
                bch::sgemm_reserved_bytes(transb != 0, 1, m, n, k, lda, ldb));
   if (st != BCH_OK) return st;
   hipError_t e = bch::launch_sgemm_ex(ctx->stream, transb != 0, 1, m, n, k, A, lda, 0, B, ldb, 0, bias, act, C,
@@ -597,7 +597,7 @@ bch_status bch_sgemm(bch_ctx* ctx, int m, int n, int k, const float* A, int lda,
   if (!C || (k > 0 && (!A || !B))) return fail(ctx, BCH_E_INVALID, "matmul: NULL buffer");
   bch_status st = use(ctx);
   if (st != BCH_OK) return st;
-  st = size_ws(ctx, bch::sgemm_ex_workspace_bytes(false, 1, m, n, k, A, lda, B, ldb),
+  st = size_ws(ctx, bch::sgemm_ex_workspace_bytes(false, 1, m, n, k, A, lda, 0, B, ldb, 0),
                bch::sgemm_reserved_bytes(false, 1, m, n, k, lda, ldb));
   if (st != BCH_OK) return st;
   hipError_t e = bch::launch_sgemm(ctx->stream, 1, m, n, k, A, lda, 0, B, ldb, 0, C, ldc, 0,
@@ -645,10 +645,10 @@ bch_status bch_sgemm_strided_batched(bch_ctx* ctx, int batch, int m, int n, int 
   if (batch > 65535) return fail(ctx, BCH_E_UNSUPPORTED, "batch_matmul: batch %d > 65535", batch);
   bch_status st = use(ctx);
   if (st != BCH_OK) return st;
-  st = size_ws(ctx, bch::sgemm_workspace_bytes(batch, m, n, k),
-               bch::sgemm_reserved_bytes(false, batch, m, n, k, k, n));
-  if (st != BCH_OK) return st;
   const int lda = k > 0 ? k : 1, ldb = n, ldc = n;
+  st = size_ws(ctx, bch::sgemm_ex_workspace_bytes(false, batch, m, n, k, A, lda, strideA, B, ldb, strideB),
+               bch::sgemm_reserved_bytes(false, batch, m, n, k, lda, ldb));
+  if (st != BCH_OK) return st;
   hipError_t e = bch::launch_sgemm(ctx->stream, batch, m, n, k, A, lda, strideA, B, ldb, strideB, C,
                                    ldc, strideC, ctx->ws, ctx->ws_bytes);
   return from_hip(ctx, e, "batch_matmul launch");

@@ -91,7 +91,8 @@ WidePlan wide_plan(int Hkv, int Sq, int Skv, int D, bool causal, int lda, int ld
     int m, n;
     chunk_shape(p, Sq, Skv, causal, r0, m, n);
     x = std::max(x, reserved ? bch::sgemm_reserved_bytes(true, Hkv, m, n, D, lda, ldb)
-                             : bch::sgemm_ex_workspace_bytes(true, Hkv, m, n, D, nullptr, lda, nullptr, ldb));
+                             : std::max(bch::sgemm_ex_workspace_bytes(true, Hkv, m, n, D, nullptr, lda, 0, nullptr, ldb, 0),
+                                        bch::sgemm_workspace_bytes(Hkv, m, n, D)));
     x = std::max(x, reserved ? bch::sgemm_reserved_bytes(false, Hkv, m, D, n, n, D)
                              : bch::sgemm_workspace_bytes(Hkv, m, D, n));
     x = std::max(x, bch::softmax_workspace_bytes((long long)Hkv * m, n));

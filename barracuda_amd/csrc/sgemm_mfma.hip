@@ -1577,14 +1577,16 @@ size_t sgemm_workspace_bytes(int batch, int m, int n, int k) {
   return tile_workspace_bytes(batch, m, n, k);
 }
 
-size_t sgemm_ex_workspace_bytes(bool transb, int batch, int m, int n, int k, const float* A, int lda, const float* B,
-                                int ldb) {
+size_t sgemm_ex_workspace_bytes(bool transb, int batch, int m, int n, int k, const float* A, int lda, long long sA,
+                                const float* B, int ldb, long long sB) {
   if (rows_applies(transb, batch, m, n, k, A, lda, B, ldb)) return rows_bytes(m, n, k);
-  if (!transb) return sgemm_workspace_bytes(batch, m, n, k);
+  if (batch == 1 && !transb && sgemm_skinny_applies(m, n, k, nullptr, k, nullptr, n))
+    return sgemm_skinny_workspace_bytes(m, n, k);
   if (batch == 1 && sgemm_skinny_nt_applies(m, n, k, nullptr, lda, nullptr, ldb))
     return sgemm_skinny_nt_workspace_bytes(m, n, k);
   if (batch == 1 && sgemm_nt_two_pass(m, n, k, nullptr, lda, nullptr, ldb))
     return std::max(sgemm_skinny_nt_workspace_bytes(32, n, k), sgemm_skinny_nt_workspace_bytes(m - 32, n, k));
+  if (small_tile_ok(batch, m, n, k, A, lda, sA, B, ldb, sB) || small_k_ok(batch, m, n, k, ldb)) return 0;
   return tile_workspace_bytes(batch, m, n, k);
 }
 

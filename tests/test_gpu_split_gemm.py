@@ -358,3 +358,19 @@ def test_small_kernel_misaligned_strided_batched_with_epilogue(dev):
     got = Tensor.from_data(xs, [5, m, k], dev).batch_matmul(Tensor.from_data(ys, [5, k, n], dev)).to_numpy()
     for g, x, y in zip(got, xs, ys):
         _check_f32_sums(g, x, y)
+
+
+@pytest.mark.parametrize("m,n,k", [(256, 256, 256), (185, 192, 521), (300, 260, 67), (320, 320, 448)])
+def test_small_kernels_ask_for_no_workspace(dev, m, n, k):
+    """Neither the 64 x 64 tiles nor the small kernel have partials; what they replaced had none here."""
+    print(f"no workspace m={m} n={n} k={k}", flush=True)
+    rng = np.random.default_rng(k)
+    a, b = (rng.integers(-40, 41, s).astype(np.float32) for s in ((m, k), (k, n)))
+    ta, tb, tc = (Tensor.from_data(x, list(x.shape), dev) for x in (a, b, np.zeros((m, n), np.float32)))
+    with _FreshCtx(dev) as f:
+        assert f.lib.bch_sgemm(f.ctx, m, n, k, C.c_void_p(ta.ptr), k, C.c_void_p(tb.ptr), n, C.c_void_p(tc.ptr), n) == 0
+        assert f.lib.bch_sync(f.ctx) == 0 and f.ws_bytes() == 0
+        assert f.lib.bch_sgemm_strided_batched(f.ctx, 1, m, n, k, C.c_void_p(ta.ptr), m * k, C.c_void_p(tb.ptr), k * n,
+                                               C.c_void_p(tc.ptr), m * n) == 0
+        assert f.lib.bch_sync(f.ctx) == 0 and f.ws_bytes() == 0
+    assert np.array_equal(tc.to_numpy(), (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32))
