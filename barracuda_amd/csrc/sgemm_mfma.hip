@@ -678,17 +678,13 @@ bool fast_ok(Tile t, int m, int n, int k, const float* A, int lda, long long sA,
          sA % 4 == 0 && sB % 4 == 0 && aligned16(A) && aligned16(B);
 }
 
-// Guarded loads as whole float4: K and N multiples of 4 (a float4 along k, or
-// along n for a [k][n] B, is then wholly inside or wholly outside), leading
-// dimensions and batch strides multiples of 4, A and B 16-byte aligned, and
-// each operand's extent (per batch) below 2 GiB for the 32-bit buffer offsets.
-bool vec4_ok(bool transb, int m, int n, int k, const float* A, int lda, long long sA, const float* B, int ldb,
-             long long sB) {
-  const long long a_bytes = ((long long)(m - 1) * lda + k) * 4;
-  // a [K][N] B's loads reach up to row K + kBK - 1 (past the resource's end, read as zeros)
-  const long long b_bytes = (transb ? (long long)(n - 1) * ldb + k : (long long)(k + kBK) * ldb) * 4;
+// Guarded tiles with 16-byte loads of A's rows (and a [n][k] B's): bases, leading dimensions and
+// batch strides that keep rows 16-byte aligned.  K and N multiples of 4 are the rule's own: the
+// clamped loads would take any (a [k][n] B is loaded by columns, in any alignment), and the hybrid
+// plan, which runs on aligned loads alone, with them.
+bool vec4_ok(int n, int k, const float* A, int lda, long long sA, const float* B, int ldb, long long sB) {
   return k >= 4 && k % 4 == 0 && n % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && sA % 4 == 0 && sB % 4 == 0 &&
-         aligned16(A) && aligned16(B) && a_bytes < (1LL << 31) && b_bytes < (1LL << 31);
+         aligned16(A) && aligned16(B);
 }
 
 // k slices in grid.z (the split-K launch): slice z adds z * (sA, sB, sC) to the batch's operands
@@ -1514,6 +1510,11 @@ static const char* tile_path_name(int m, int n, int k, bool allow_mix);
 
 const char* sgemm_kernel_name(int m, int n, int k) {
   if (sgemm_skinny_applies(m, n, k, nullptr, k, nullptr, n)) return sgemm_skinny_kernel_name(m);
+  if (rows_applies(false, 1, m, n, k, nullptr, k, nullptr, n)) {
+    static const char* const names[2][2] = {{"sgemm_rows_kernel<1>", "sgemm_rows_kernel<1>+sgemm_splitk_reduce"},
+                                            {"sgemm_rows_kernel<2>", "sgemm_rows_kernel<2>+sgemm_splitk_reduce"}};
+    return names[m > 32][rows_plan(m, n, k).S > 1];
+  }
   return tile_path_name(m, n, k, true);
 }
 
@@ -1536,8 +1537,8 @@ static const char* tile_path_name(int m, int n, int k, bool allow_mix) {
   // with lda = k and ldb = n, and 16-byte aligned operands
   const bool check = !(m % tile_m(t) == 0 && n % tile_n(t) == 0 && k % kBK == 0 && k % 4 == 0 && n % 4 == 0);
   const bool v4 = k >= 4 && k % 4 == 0 && n % 4 == 0;
-  if (sp.S > 1) {  // slices of 32-k tiles (k % 32 == 0)
-    const bool fast = m % tile_m(t) == 0 && n % tile_n(t) == 0 && n % 4 == 0;
+  if (sp.S > 1) {
+    const bool fast = !check;
     static const char* const split_names[3][3] = {
         {"sgemm_mfma_kernel<256,256,32,false>+sgemm_splitk_reduce", "sgemm_mfma_kernel<256,256,32,true,v4>+sgemm_splitk_reduce",
          "sgemm_mfma_kernel<256,256,32,true>+sgemm_splitk_reduce"},
@@ -1672,7 +1673,7 @@ hipError_t launch_tile_path(hipStream_t s, bool transb, int batch, int m, int n,
     z.sC = per;
     // the slice offsets (kc a multiple of 32, times ldb) keep the batch strides' alignment
     const int mode = fast_ok(t, m, n, k, A, lda, sA, B, ldb, sB)               ? 0
-                     : vec4_ok(transb, m, n, k, A, lda, sA, B, ldb, sB) ? 1
+                     : vec4_ok(n, k, A, lda, sA, B, ldb, sB) ? 1
                                                                            : 2;
     hipError_t e = transb ? launch_tile_any<true, false>(mode, t, s, batch, m, n, k, A, lda, sA, B, ldb, sB, P, n,
                                                          sl * per, nullptr, 0, z)
@@ -1688,7 +1689,7 @@ hipError_t launch_tile_path(hipStream_t s, bool transb, int batch, int m, int n,
     // of its own; the offsets are multiples of 256 rows (columns), which keeps the alignment
     const int m1 = mp.axis == 0 ? mp.split : m, n1 = mp.axis == 1 ? mp.split : n;
     const int mode1 = fast_ok(Tile::k256x256, m1, n1, k, A, lda, sA, B, ldb, sB)      ? 0
-                      : vec4_ok(transb, m1, n1, k, A, lda, sA, B, ldb, sB) ? 1
+                      : vec4_ok(n1, k, A, lda, sA, B, ldb, sB) ? 1
                                                                              : 2;
     hipError_t e =
         transb ? (epi ? launch_tile_any<true, true>(mode1, Tile::k256x256, s, 1, m1, n1, k, A, lda, sA, B, ldb, sB, C,
@@ -1710,7 +1711,7 @@ hipError_t launch_tile_path(hipStream_t s, bool transb, int batch, int m, int n,
   HybPlan h;
   if (hyb_plan(batch, m, n, k, h) && ws != nullptr && ws_bytes >= hyb_bytes(h)) {
     const int hmode = fast_ok(h.t, m, n, k, A, lda, sA, B, ldb, sB)                ? 0
-                      : vec4_ok(transb, m, n, k, A, lda, sA, B, ldb, sB)          ? 1
+                      : vec4_ok(n, k, A, lda, sA, B, ldb, sB)          ? 1
                                                                                    : 2;
     if (hmode != 2) {
       float* P = static_cast<float*>(ws);
@@ -1721,10 +1722,8 @@ hipError_t launch_tile_path(hipStream_t s, bool transb, int batch, int m, int n,
                  : launch_hyb<false, false>(hmode, h, s, m, n, k, A, lda, B, ldb, C, ldc, bias, act, P);
     }
   }
-  // the [n][k] tile loads need the same alignment as the [k][n] ones (ldb, sB multiples of 4); a
-  // [n][k] B needs only K % 4 == 0 for whole float4, but N % 4 is kept for one rule
   const int mode = fast_ok(t, m, n, k, A, lda, sA, B, ldb, sB) ? 0
-                   : vec4_ok(transb, m, n, k, A, lda, sA, B, ldb, sB) ? 1
+                   : vec4_ok(n, k, A, lda, sA, B, ldb, sB) ? 1
                                                                  : 2;
   if (transb)
     return epi ? launch_tile_any<true, true>(mode, t, s, batch, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC, bias, act)

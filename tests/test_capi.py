@@ -128,6 +128,16 @@ def test_kernel_routing_names():
     assert lib.bch_sgemm_kernel_name(100, 70, 33) == b"sgemm_mfma_kernel<128,128,32,true>"
 
 
+def test_kernel_routing_names_of_few_rows_and_guarded_slices():
+    """Up to 64 rows that no skinny kernel takes, and split-K of a K that takes the guarded tiles."""
+    lib = N.load()
+    assert lib.bch_sgemm_kernel_name(20, 5247, 1001) == b"sgemm_rows_kernel<1>+sgemm_splitk_reduce"
+    assert lib.bch_sgemm_kernel_name(48, 4095, 1000) == b"sgemm_rows_kernel<2>+sgemm_splitk_reduce"
+    assert lib.bch_sgemm_kernel_name(3, 129, 33) == b"sgemm_rows_kernel<1>"
+    assert lib.bch_sgemm_kernel_name(512, 512, 2628) == b"sgemm_mfma_kernel<128,128,32,true,v4>+sgemm_splitk_reduce"
+    assert lib.bch_sgemm_kernel_name(512, 512, 2629) == b"sgemm_mfma_kernel<128,128,32,true>+sgemm_splitk_reduce"
+
+
 def test_status_to_error_variant_mapping():
     assert isinstance(from_status(N.BCH_E_SHAPE, "x", "matmul"), InvalidOperation)
     assert "mismatch" in str(from_status(N.BCH_E_SHAPE, "x", "matmul"))
