@@ -196,8 +196,6 @@ size_t sgemm_ex_workspace_bytes(bool transb, int batch, int m, int n, int k, con
 // needs of its scratch.
 constexpr size_t kSgemmFixedScratch = (size_t)16 << 20;
 size_t sgemm_reserved_bytes(bool transb, int batch, int m, int n, int k, int lda, int ldb, bool fixed = false);
-// 32 < m <= 64 rows of [n][k] weights as two passes of the 32-row kernels
-bool sgemm_nt_two_pass(int m, int n, int k, const float* A, int lda, const float* B, int ldb);
 const char* sgemm_kernel_name(int m, int n, int k);
 // With B given as [n][k] when transb (C = A B^T), and the linear layer's
 // epilogue C = act(acc + bias[col]): bias nullable, act kActNone / kActRelu /

@@ -1461,7 +1461,9 @@ RowsPlan rows_plan(int m, int n, int k) {
 // path's slices MLP of 20 rows 2890 -> 5248 53 -> 46 us), and 33 to 64 rows against [n][k]
 // weights too large for the tile path's slices to stay in step (in us, two passes of the 32-row
 // kernels or tile slices -> here: 48 x 11008 x 4096 78 -> 55, 64 x 4096 x 11008 75 -> 59, 48 x
-// 4096 x 1024 17.7 -> 16.9; 48 x 5120 x 2048 23.0 -> 24.2, so from 2^24 weights on).
+// 4096 x 1024 17.7 -> 16.9; 48 x 5120 x 2048 23.0 -> 24.2, so from 2^24 weights on).  Two passes of
+// the 32-row kernels lose to both below that too (48 x 11008 x 1024 31.7, tile path 27.0, here 24.4;
+// 40 x 32768 x 256 185, 15.7, 20.0; 64 x 8192 x 1024 30.4, 16.4, 22.9).
 bool rows_applies(bool transb, int batch, int m, int n, int k, const float* A, int lda, const float* B, int ldb) {
   if (batch != 1 || m > 64 || n < 1 || k < 1) return false;
   if (transb)
@@ -1497,14 +1499,6 @@ hipError_t launch_rows(hipStream_t s, bool transb, int m, int n, int k, const fl
 }  // namespace
 
 namespace bch {
-
-// [n][k] weights with 32 < m <= 64 and n >= 8192: two passes of the m <= 32 path.  Same box,
-// two runs each, against the tile path (bias + ReLU): 33 / 48 / 64 x 11008 x 4096 99.5 / 100.9
-// / 103.0 -> 70.7 / 76.0 / 83.0 us; at n = 4096 the tiles fill the CUs and stay ahead (48 x 4096
-// x 4096 40.0 against 44.1 us, 64 x 4096 x 11008 91.5 against 93.6).
-bool sgemm_nt_two_pass(int m, int n, int k, const float* A, int lda, const float* B, int ldb) {
-  return m > 32 && m <= 64 && n >= 8192 && sgemm_skinny_nt_applies(32, n, k, A, lda, B, ldb);
-}
 
 static const char* tile_path_name(int m, int n, int k, bool allow_mix);
 
@@ -1585,8 +1579,6 @@ size_t sgemm_ex_workspace_bytes(bool transb, int batch, int m, int n, int k, con
     return sgemm_skinny_workspace_bytes(m, n, k);
   if (batch == 1 && sgemm_skinny_nt_applies(m, n, k, nullptr, lda, nullptr, ldb))
     return sgemm_skinny_nt_workspace_bytes(m, n, k);
-  if (batch == 1 && sgemm_nt_two_pass(m, n, k, nullptr, lda, nullptr, ldb))
-    return std::max(sgemm_skinny_nt_workspace_bytes(32, n, k), sgemm_skinny_nt_workspace_bytes(m - 32, n, k));
   if (small_tile_ok(batch, m, n, k, A, lda, sA, B, ldb, sB) || small_k_ok(batch, m, n, k, ldb)) return 0;
   return tile_workspace_bytes(batch, m, n, k);
 }
@@ -1624,14 +1616,6 @@ hipError_t launch_sgemm_ex(hipStream_t s, bool transb, int batch, int m, int n, 
     return launch_sgemm_skinny_nt(s, m, n, k, A, lda, B, ldb, C, ldc, ws, ws_bytes, bias, act);
   if (rows_applies(transb, batch, m, n, k, A, lda, B, ldb) && ws_bytes >= rows_bytes(m, n, k))
     return launch_rows(s, transb, m, n, k, A, lda, B, ldb, C, ldc, bias, act, ws);
-  // 32 < m <= 64 with [n][k] weights: the 32-row kernels twice, on rows 0..31 and 32..m-1 (the
-  // second pass streams the weights again, largely from the Infinity Cache)
-  if (transb && batch == 1 && sgemm_nt_two_pass(m, n, k, A, lda, B, ldb)) {
-    hipError_t e = launch_sgemm_skinny_nt(s, 32, n, k, A, lda, B, ldb, C, ldc, ws, ws_bytes, bias, act);
-    if (e != hipSuccess) return e;
-    return launch_sgemm_skinny_nt(s, m - 32, n, k, A + 32LL * lda, lda, B, ldb, C + 32LL * ldc, ldc, ws, ws_bytes,
-                                  bias, act);
-  }
   return launch_tile_path(s, transb, batch, m, n, k, A, lda, sA, B, ldb, sB, bias, act, C, ldc, sC, ws, ws_bytes,
                           true);
 }

@@ -145,7 +145,8 @@ size_t sgemm_reserved_bytes(bool transb, int batch, int m, int n, int k, int lda
   }
   if (batch == 1 && transb) {
     if (sgemm_skinny_nt_applies(m, n, k, nullptr, lda, nullptr, ldb)) return sgemm_skinny_nt_workspace_bytes(m, n, k);
-    if (sgemm_nt_two_pass(m, n, k, nullptr, lda, nullptr, ldb))
+    // 33 to 64 rows as two passes of the 32-row kernels
+    if (m > 32 && m <= 64 && n >= 8192 && sgemm_skinny_nt_applies(32, n, k, nullptr, lda, nullptr, ldb))
       return std::max(sgemm_skinny_nt_workspace_bytes(32, n, k), sgemm_skinny_nt_workspace_bytes(m - 32, n, k));
   }
   return tile_bytes(batch, m, n, k, fixed);
