@@ -2,7 +2,7 @@
 
 Captured: the decode linear layer with [out, in] weights (the ring kernel, whose
 split-k blocks are combined in the kernel through epoch flags that every launch
-resets; at m = 48 in two passes), the skinny GEMM (main kernel + reduce; the one-
+resets; at m = 48 the rows kernel), the skinny GEMM (main kernel + reduce; the one-
 and two-block kernels), the tile GEMM's hybrid plan (whole tiles and k-slices in
 one launch + reduce) and its split-K (slices into the workspace + reduce), row
 softmax and attention.  The graph is replayed several times with the program's
@@ -60,7 +60,7 @@ def test_graph_replays_match_eager(dev):
 
     rng = O.Lcg(2024)
     calls = []  # (name, zero-arg launcher, output tensor)
-    for m, n, k in ((8, 11008, 4096), (32, 11008, 4096), (8, 64, 16384), (48, 11008, 4096)):  # 48: two passes
+    for m, n, k in ((8, 11008, 4096), (32, 11008, 4096), (8, 64, 16384), (48, 11008, 4096)):  # 48: the rows kernel
         x, w, b = _up(dev, rng.normal((m, k))), _up(dev, rng.normal((n, k), 0.0, 0.05)), _up(dev, rng.normal((n,)))
         y = Tensor.empty([m, n], dev)
         calls.append((f"linear wT m={m} n={n} k={k}",

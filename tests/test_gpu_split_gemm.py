@@ -43,17 +43,20 @@ def _check_f32_sums(got, a, b):
     assert worst <= 1.0, worst
 
 
-# (m, n): 64 x 64 tiles, 128 x 128 tiles, 256 x 128 tiles, 256 x 256 tiles
-TILES = [(192, 128), (200, 136), (8190, 1020), (4095, 4090)]
+# (m, n) and the kernel from 64 k on: few tiles (below 64 k 128 x 128 ones), 128 x 128, 256 x 128, 256 x 256
+TILES = [(192, 128, b"sgemm_small_kernel"), (200, 136, b"sgemm_small_kernel"), (2040, 2044, b"sgemm_mfma_kernel<128,128,32"),
+         (8190, 1020, b"sgemm_mfma_kernel<256,128,32"), (4095, 4090, b"sgemm_mfma_kernel<256,256,32")]
 
 
 @pytest.mark.parametrize("transb", [0, 1])
-@pytest.mark.parametrize("m,n", TILES)
+@pytest.mark.parametrize("m,n,kernel", TILES)
 @pytest.mark.parametrize("k", [1, 7, 15, 16, 17, 31, 32, 33, 47, 65, 95])
-def test_k_remainders_exact(dev, m, n, k, transb):
+def test_k_remainders_exact(dev, m, n, kernel, k, transb):
     """Integers below 2^12: products below 2^24 and their sums are exact in f32, so three parts
     have to give every bit, whatever the remainder of k."""
     print(f"k remainder m={m} n={n} k={k} transb={transb}", flush=True)
+    name = dev._lib.bch_sgemm_kernel_name(m, n, k)
+    assert name.startswith(kernel if k >= 64 or kernel != b"sgemm_small_kernel" else b"sgemm_mfma_kernel<128,128,32")
     rng = np.random.default_rng(m + n + k)
     a = rng.integers(-400, 401, (m, k)).astype(np.float32)
     b = rng.integers(-400, 401, (n, k) if transb else (k, n)).astype(np.float32)
@@ -63,7 +66,11 @@ def test_k_remainders_exact(dev, m, n, k, transb):
 
 
 @pytest.mark.parametrize("m,n,k,a_off,b_off,lda_pad,ldb_pad", [
-    (260, 300, 100, 1, 3, 0, 0), (260, 300, 100, 0, 0, 1, 3), (300, 260, 67, 2, 1, 2, 2), (128, 128, 64, 1, 1, 0, 0)])
+    # the small kernel
+    (260, 300, 100, 1, 3, 0, 0), (260, 300, 100, 0, 0, 1, 3), (300, 260, 67, 2, 1, 2, 2), (128, 128, 64, 1, 1, 0, 0),
+    # 128 x 128, 256 x 128 and 256 x 256 tiles, and slices, that aligned operands would take unguarded or by 16 bytes
+    (2048, 2048, 96, 1, 3, 0, 0), (2040, 2044, 100, 0, 0, 1, 3), (8192, 1024, 64, 2, 1, 2, 2), (8190, 1020, 65, 0, 1, 3, 0),
+    (4096, 4096, 64, 1, 1, 0, 0), (4096, 4096, 64, 0, 0, 4, 1), (300, 260, 4096, 1, 3, 1, 3), (512, 512, 4096, 0, 2, 0, 0)])
 @pytest.mark.parametrize("transb", [0, 1])
 def test_misaligned_rows_exact(dev, m, n, k, a_off, b_off, lda_pad, ldb_pad, transb):
     print(f"misaligned m={m} n={n} k={k} transb={transb}", flush=True)
@@ -93,28 +100,30 @@ def test_non_finite_operands(dev, m, n, k, transb):
     assert np.array_equal(got, want.astype(np.float32), equal_nan=True)
 
 
-@pytest.mark.parametrize("sa,sb", [(2.0**-120, 1.0), (2.0**-120, 2.0**100), (1.0, 2.0**-126), (2.0**-70, 2.0**-60),
-                                   (2.0**60, 2.0**56), (2.0**-149, 2.0**120), (2.0**124, 2.0**-20)])
-def test_ends_of_the_range(dev, sa, sb):
-    """Rows scaled by powers of two to both ends of the f32 range, subnormals among them: the
-    f32 product to 2^-24 a term (and half the smallest subnormal), as the f32 instruction gives."""
-    print(f"range sa={sa} sb={sb}", flush=True)
-    m, n, k = 160, 144, 128
-    rng = np.random.default_rng(5)
-    a = (rng.standard_normal((m, k)) * sa).astype(np.float32)
-    b = (rng.standard_normal((k, n)) * sb).astype(np.float32)
-    _check_f32_sums(_ex(dev, a, b, 0), a, b)
-
-
-# m, n, k and what bch_sgemm runs there (None: the rows kernel, which takes up to 64 rows of other K or alignment)
+# m, n, k and what bch_sgemm runs there
 KERNELS = [(256, 256, 256, "sgemm_mfma_kernel<64,64,64,false>"), (160, 144, 128, "sgemm_small_kernel"),
            (300, 260, 4096, "sgemm_mfma_kernel<128,128,32,true,v4>+sgemm_splitk_reduce"),
            (2048, 2048, 96, "sgemm_mfma_kernel<128,128,32,false>"),
            (2047, 2045, 95, "sgemm_mfma_kernel<128,128,32,true>"),
            (8192, 1024, 64, "sgemm_mfma_kernel<256,128,32,false>"), (4096, 4096, 64, "sgemm_mfma_kernel<256,256,32,false>"),
            (4095, 4090, 95, "sgemm_mfma_kernel<256,256,32,true>"),
-           (3072, 3072, 512, "sgemm_mfma_kernel<128,128,32,false,hyb>+sgemm_tail_reduce"), (20, 301, 333, None),
-           (50, 301, 2049, None)]
+           (3072, 3072, 512, "sgemm_mfma_kernel<128,128,32,false,hyb>+sgemm_tail_reduce"),
+           (20, 301, 333, "sgemm_rows_kernel<1>+sgemm_splitk_reduce"),
+           (50, 301, 2049, "sgemm_rows_kernel<2>+sgemm_splitk_reduce")]
+
+
+@pytest.mark.parametrize("sa,sb", [(2.0**-120, 1.0), (2.0**-120, 2.0**100), (1.0, 2.0**-126), (2.0**-70, 2.0**-60),
+                                   (2.0**60, 2.0**56), (2.0**-149, 2.0**120), (2.0**124, 2.0**-20)])
+@pytest.mark.parametrize("m,n,k,kernel", KERNELS)
+def test_ends_of_the_range(dev, m, n, k, kernel, sa, sb):
+    """Rows scaled by powers of two to both ends of the f32 range, subnormals among them: the
+    f32 product to 2^-24 a term (and half the smallest subnormal), as the f32 instruction gives."""
+    assert dev._lib.bch_sgemm_kernel_name(m, n, k).decode() == kernel
+    print(f"range m={m} n={n} k={k} sa={sa} sb={sb}", flush=True)
+    rng = np.random.default_rng(5)
+    a = (rng.standard_normal((m, k)) * sa).astype(np.float32)
+    b = (rng.standard_normal((k, n)) * sb).astype(np.float32)
+    _check_f32_sums(_ex(dev, a, b, 0), a, b)
 
 
 @pytest.mark.parametrize("transb", [0, 1])
@@ -123,8 +132,7 @@ def test_tiny_elements_beside_ordinary_ones(dev, m, n, k, kernel, transb):
     """Elements down to the subnormals in rows (columns) that also hold ordinary ones, against zeros
     there and large elements elsewhere: every element counts to f32 accuracy, whatever else its
     row holds."""
-    if kernel is not None:
-        assert dev._lib.bch_sgemm_kernel_name(m, n, k).decode() == kernel
+    assert dev._lib.bch_sgemm_kernel_name(m, n, k).decode() == kernel
     rng = np.random.default_rng(m + k)
     for e, f, swap in ((-118, 100, False), (-125, 120, False), (-140, 120, False), (-125, 120, True)):
         print(f"tiny elements m={m} n={n} k={k} transb={transb} 2^{e} 2^{f} swap={swap}", flush=True)
@@ -147,8 +155,7 @@ def test_values_computed_again_in_f32(dev, m, n, k, kernel, transb, epilogue):
     """What the parts cannot stand for, on every kernel and k-slice: infinities and NaN anywhere in k,
     a row and a column of nothing but NaN, operands from 2^111 and sums from 2^96.  Integers times
     powers of two, so every value is exact; its neighbours keep theirs."""
-    if kernel is not None:
-        assert dev._lib.bch_sgemm_kernel_name(m, n, k).decode() == kernel
+    assert dev._lib.bch_sgemm_kernel_name(m, n, k).decode() == kernel
     print(f"again in f32 m={m} n={n} k={k} transb={transb} epilogue={epilogue}", flush=True)
     rng = np.random.default_rng(m + k)
     a, b = (rng.integers(-8, 9, s).astype(np.float32) for s in ((m, k), (k, n)))
@@ -210,10 +217,14 @@ def test_one_huge_element_in_a_row(dev):
 
 @pytest.mark.parametrize("transb", [0, 1])
 @pytest.mark.parametrize("m,n,k", [(171, 455, 1472), (67, 1536, 3056), (128, 150, 2624), (185, 192, 521), (3, 8001, 642),
-                                   (1, 130, 4097), (260, 129, 255), (515, 1030, 1999)])
+                                   (1, 130, 4097), (260, 129, 255), (515, 1030, 1999), (300, 260, 2999), (700, 1200, 1501)])
 def test_uneven_k_slices_exact(dev, m, n, k, transb):
-    """Split-K where the slices do not divide K: the last slice is shorter and takes the remainder."""
+    """Split-K where the slices do not divide K: the last slice is shorter and takes the remainder.  Of the
+    sizes that now run the small kernel, every eighth unit a wavefront."""
     print(f"uneven slices m={m} n={n} k={k} transb={transb}", flush=True)
+    small = (m, n, k) in ((171, 455, 1472), (185, 192, 521), (260, 129, 255))
+    name = dev._lib.bch_sgemm_kernel_name(m, n, k)
+    assert name == b"sgemm_small_kernel" if small else name.endswith(b"+sgemm_splitk_reduce")
     rng = np.random.default_rng(m + n + k)
     a = rng.integers(-40, 41, (m, k)).astype(np.float32)
     b = rng.integers(-40, 41, (n, k) if transb else (k, n)).astype(np.float32)
@@ -221,19 +232,25 @@ def test_uneven_k_slices_exact(dev, m, n, k, transb):
     assert np.array_equal(_ex(dev, a, b, transb), want)
 
 
-def test_uneven_k_slices_batched(dev):
-    batch, m, n, k = 3, 150, 70, 1001
+@pytest.mark.parametrize("batch,m,n,k", [(3, 150, 70, 1001), (3, 150, 70, 2999), (3, 300, 260, 2111)])
+def test_uneven_k_slices_batched(dev, batch, m, n, k):
+    """The small kernel; slices of 4 k-tiles and of 8, the last with the remainder."""
+    # a batch of one of these sizes splits too: k from 2048 on is not the small kernel's
+    assert dev._lib.bch_sgemm_kernel_name(m, n, k).endswith(b"+sgemm_splitk_reduce" if k >= 2048 else b"sgemm_small_kernel")
     rng = np.random.default_rng(4)
     a, b = (rng.integers(-40, 41, s).astype(np.float32) for s in ((batch, m, k), (batch, k, n)))
     got = Tensor.from_data(a, list(a.shape), dev).batch_matmul(Tensor.from_data(b, list(b.shape), dev)).to_numpy()
     assert np.array_equal(got, (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32))
 
 
-def test_capture_without_workspace_runs_unsplit(dev):
+@pytest.mark.parametrize("m,n,k,kernel", [(171, 455, 1471, b"sgemm_small_kernel"),
+                                          (300, 260, 2999, b"sgemm_mfma_kernel<128,128,32,true>+sgemm_splitk_reduce"),
+                                          (20, 5247, 1001, b"sgemm_rows_kernel<1>+sgemm_splitk_reduce")])
+def test_capture_without_workspace_runs_unsplit(dev, m, n, k, kernel):
     """A shape whose K no slices divide, first called under capture: no workspace may grow, the call
-    runs unsplit, and its graph replays to the product."""
+    runs unsplit (the small kernel as ever, few rows on tiles), and its graph replays to the product."""
+    assert dev._lib.bch_sgemm_kernel_name(m, n, k) == kernel
     hip = _hip()
-    m, n, k = 171, 455, 1471
     rng = np.random.default_rng(6)
     a, b = rng.integers(-40, 41, (m, k)).astype(np.float32), rng.integers(-40, 41, (k, n)).astype(np.float32)
     want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
