@@ -76,9 +76,10 @@ __device__ __forceinline__ float activate(float v, int act) {
 // datatype for higher-precision computations" (ARITH 2019).
 // What is left out: |x1| <= 2^-8 and |x2| <= 2^-17 of x's power of two, so x1 y2 + x2 y1 reaches
 // 2^-24 of |x y| at worst (x = y = 1.0039) and is 2^-27 in the root mean square; the rounding of
-// one f32 addition is up to 2^-24.  A single product alone in its sum thus can be off by 1.7 2^-24
-// where an f32 multiplication rounds by 2^-24; sums of many come out closer than on the f32
-// instruction, whose accumulator rounds once every two k instead of six times every sixteen.
+// one f32 addition is up to 2^-24.  A single product alone in its sum thus can be off by 2.0 2^-24
+// (1.7 among 4 million random ones) where an f32 multiplication rounds by 2^-24; sums of many come
+// out closer than on the f32 instruction, whose accumulator rounds once every two k instead of six
+// times every sixteen.
 // Integers whose product is below 2^24 stay exact.
 // Why: v_mfma_f32_32x32x2_f32 does 256 FLOP a clock and CU, the bf16 instruction 4096, so six of
 // them still leave 2.7 times the f32 rate.

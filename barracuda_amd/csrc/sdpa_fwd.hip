@@ -32,8 +32,8 @@
 //     for v_mfma_f32_32x32x2_f32, next to about 370 VALU operations (softmax, and the parts of
 //     P and of its share of K and V); two wavefronts per SIMD overlap the two.  Measured at B 4,
 //     H 32, S 2048, D 128, causal, against f32 MFMAs (one box): 1.09 -> 0.71 ms, error against 64
-//     bits 4.5e-7 -> 3.7e-7; the matrix cores are busy 59% of the cycles, at a clock that has
-//     fallen to about 1.7 GHz.
+//     bits 4.5e-7 -> 3.7e-7; the matrix cores are busy 57% of the cycles (non-causal 64%), at a
+//     clock that has fallen to 1.9 GHz (1.7).
 //   * Scores are computed transposed, S^T = K Q^T (32 keys x 32 queries), so
 //     each lane holds 16 scores of ITS query: the row max and row sum are
 //     in-lane plus one exchange between the two lane halves

@@ -231,13 +231,12 @@ __global__ __launch_bounds__((Cfg<BM, BN, BK>::NT)) void sgemm_mfma_kernel(
     // Workgroups are dispatched round-robin over the 8 XCDs in linear id order (x fastest), so
     // a batch's tiles were spread over all eight L2s.  Each XCD takes a contiguous run of the
     // (batch, tile) slots instead: whole batches where a batch's tiles divide the run, each
-    // batch's A and B then read into one L2.  Same box, three runs each (us): 16 x 1024^3
-    // 248.5-251.0 -> 246.9-247.3, 8 x 1024^3 130.3-130.8 -> 127.4-127.8, 24 x 1024^3
-    // 388-399 -> 381-383, 64 x 512^3 135.1-136.0 -> 132.4-133.1, 32 x 1024 x 1024 x 512 +0.9%,
-    // 4 x 2048 x 2048 x 1024 +1%, 16 x 1024 x 1024 x 4096 unchanged.  Unguarded loads only: in
-    // the float4-guarded 256 x 256 instantiations it doubled the k-loop's code and moved its
-    // load waits.  Split-K grids (slices in z) keep the dispatch order: remapped the same way
-    // they measured even or slower (1024 x 1024 x 2048 43.3-43.6 -> 44.3-44.4 us).
+    // batch's A and B then read into one L2.  Same box, three runs each (us): 16 x 1024^3 158.7 ->
+    // 154.5, 8 x 1024^3 87.1 -> 84.8, 24 x 1024^3 263.7 -> 255.4, 64 x 512^3 86.6 -> 83.0, 32 x 1024
+    // x 1024 x 512 165.7 -> 160.5, 4 x 2048 x 2048 x 1024 154.0 -> 153.0, 16 x 1024 x 1024 x 4096 640
+    // -> 601.  The guarded tiles and split-K grids (slices in z) keep the dispatch order, which
+    // their plans were measured in; remapped, batches of them would gain 1 to 5% (24 x 1000 x 1000
+    // x 2000 524 -> 499, 8 x 256 x 512 x 4096 57.5 -> 54.7), single matrices nothing.
     const long long slots = (long long)gridDim.x * gridDim.y;
     if (gridDim.y > 1 && gridDim.z == 1 && (slots & 7) == 0) {
       const long long L = (long long)blockIdx.y * gridDim.x + blockIdx.x;
@@ -710,7 +709,7 @@ hipError_t launch_tile(Tile t, hipStream_t s, int batch, int m, int n, int k, co
   }
 }
 
-// mode 0: unguarded; 1: guarded float4 loads; 2: guarded scalar loads
+// mode 0: unguarded; 1: guarded, 16-byte aligned rows; 2: guarded, any alignment
 template <bool TB, bool EPI>
 hipError_t launch_tile_any(int mode, Tile t, hipStream_t s, int batch, int m, int n, int k, const float* A,
                            int lda, long long sA, const float* B, int ldb, long long sB, float* C, int ldc,
@@ -903,7 +902,7 @@ hipError_t launch_splitk_reduce(hipStream_t s, int m, int n, int S, int batch, c
 // The plan is modelled like the tile choice (k-tiles x tile area /
 // efficiency per round; the partials' HBM traffic at 6.3 TB/s, one 256 x 256
 // k-tile taking kTileKtUs) and used when it beats the best data-parallel tiling
-// by 3%.  It needs K a multiple of 32 and unguarded or float4-guarded loads;
+// by 3%.  It needs K a multiple of 32 and unguarded or 16-byte aligned loads (vec4_ok);
 // without the workspace (up to kHybWsMax) the data-parallel tiling runs.
 constexpr size_t kHybWsMax = (size_t)256 << 20;
 constexpr int kHybMinKt = 8;  // k-tiles per slice at least
@@ -981,18 +980,18 @@ double tile_path_cost_us(int m, int n, int k) {
 // efficiency over the whole matrix.  Where the 256 x 256 tiles make at least one whole round,
 // the mixed plan runs j whole rounds of them on the first rows (or columns) of C, data-parallel,
 // then the remaining rows (or columns) as a call of their own (split-K, hybrid or
-// data-parallel, as planned for that shape).  Same box, two runs each, TFLOP/s, against the
-// plan for the whole matrix: 4096 x 11008 x 4096 138.9 -> 141.5 (columns 0..8191 first),
-// 11008 x 4096 x 4096 139.2 -> 141.5 (rows 0..8191), 8192 x 11008 x 4096 140.2 -> 144.6,
-// 3072 x 11008 x 4096 138.4 -> 140.0, 4096 x 14336 x 4096 143.3 -> 145.0; 5120^3 142.1 ->
-// 138.7, which the model rejects.  Chosen when the model puts it 1% ahead of the whole-matrix
-// plan; the split runs along rows or columns, with j from 1 to the whole rounds available.
-// Only the first level splits: the rest is planned without the mixed plan.
+// data-parallel, as planned for that shape).  Same box, three runs each, us, plan for the whole
+// matrix -> mixed: 4096 x 11008 x 4096 1802 -> 1730, 11008 x 4096 x 4096 1716 -> 1653, 8192 x 11008
+// x 4096 3410 -> 3130, 3072 x 11008 x 4096 1204 -> 1178, 4096 x 14336 x 4096 2205 -> 2030, 2048 x
+// 11008 x 4096 888 -> 823, 8192 x 11008 x 1024 895 -> 824, 4352 x 4352 x 1024 225 -> 191, x 4096
+// 694 -> 682, 6000 x 6000 x 2048 675 -> 670, 4864 x 4096 x 4096 712 both; two of the thirteen that
+// the model takes lose, 4096 x 11008 x 1024 414 -> 431 and 7168 x 4096 x 2048 530 -> 562, whose
+// whole-matrix plan runs 6% under its model.  Chosen when the model puts it 1% ahead; the split
+// runs along rows or columns, with j from 1 to the whole rounds available.  Only the first level
+// splits: the rest is planned without the mixed plan.
 // The second launch's fixed cost in the model: its prologue, the first launch's last C stores
-// that nothing overlaps, and the gap between the launches.  At 16 us (10 us at the present rates) the model picked, among
-// 26 shapes measured both ways (K 1024 and 4096), every one that gained (1.1-6.0%) at K 4096
-// and leaves out the two that lost (6144 x 6144 x 1024 -2.9%, 4100 x 4100 x 1024 -1.2%); two
-// it still takes at K 1024 measured within 0.4% either way.
+// that nothing overlaps, and the gap between the launches (16 us fitted the f32 instruction's
+// kernels; 10 us is that at the present rates, and no constant parts the two from the eleven).
 constexpr double kMixFixedUs = 10.0;
 
 struct MixPlan {
@@ -1092,7 +1091,7 @@ hipError_t launch_tail_reduce(hipStream_t s, int m, int n, const HybPlan& h, con
   return hipGetLastError();
 }
 
-// mode 0: unguarded loads; mode 1: float4-guarded (K % 32 == 0 here, so the one-add form)
+// mode 0: unguarded; mode 1: guarded, 16-byte aligned rows
 template <bool TB, bool EPI>
 hipError_t launch_hyb(int mode, const HybPlan& h, hipStream_t s, int m, int n, int k, const float* A, int lda,
                       const float* B, int ldb, float* C, int ldc, const float* bias, int act, float* P) {
@@ -1237,8 +1236,9 @@ __global__ __launch_bounds__(512, 4) void sgemm_small_kernel(int M, int N, int K
 // 15.0 -> 11.4, 100 x 4000 x 500 15.5 -> 9.6, 1001 x 999 x 333 17.9 -> 13.1, 256 x 1024 x 1024 (split) 15.8 -> 8.5,
 // 512 x 512 x 1024 15.8 -> 9.0; left to the split plan: 700 x 1200 x 1500 26.6 (38.2 here), 256 x 2048 x
 // 2048 22.9 (24.6).  From k 2048 on the split plan's shorter sums are the more exact (128 x 128 x 2048
-// 1.9e-7 against 2.5e-7) and the times within 15%.  Below 64 k, six part products of one product
-// keep 2.3 2^-24, where the tiles' f32 loop rounds once.
+// 1.9e-7 against 2.5e-7) and the times within 15%.  Below 64 k the tiles stay, which multiply in
+// f32 below one pass of theirs (a lone product rounds once there, and is up to 2.0 2^-24 off as part
+// products); 100 x 4000 x 48 takes 7.6 us on them.
 bool small_k_plan(int batch, int m, int n, int k) {
   if (batch < 1 || batch > 65535 || k < 64 || k >= 2048) return false;
   const SplitPlan p = split_plan(batch, m, n, k);

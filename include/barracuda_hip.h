@@ -146,12 +146,18 @@ bch_status bch_sync(bch_ctx *ctx);
  * matmul_tiled_f64.wgsl) and MatmulTiled::execute (ops/matmul_tiled.rs:
  * 62-122).  Routes m <= 32 (decode shapes) to the skinny HBM-streaming
  * kernels, 32 < m <= 64 with K % 4 == 0 and 16-byte aligned A to their
- * two-block form, and everything else to the FP32-MFMA tiled kernel (64x64
- * tiles, or a split over k, when the tiles fill less than one round of the
- * CUs, whichever is modelled faster; whole rounds
+ * two-block form, other calls of m <= 32, and of m <= 64 with N % 4 != 0, to
+ * the rows kernel, and everything else to the tiled kernel (64x64 or 32x32 tiles, or a split over
+ * k, when the tiles fill less than one round of the CUs, whichever is
+ * modelled faster; whole rounds
  * plus k-sliced leftover tiles when the last round would be part-filled; or
  * whole rounds of 256x256 tiles on the first rows or columns of C and the
- * rest planned on its own, where that is modelled faster). */
+ * rest planned on its own, where that is modelled faster).  All but the
+ * skinny kernels multiply on the bf16 matrix cores, three bf16 parts per f32
+ * and six part products: sums to f32 accuracy, whatever the magnitudes; a
+ * single product alone in its sum to 2 * 2^-24 (an f32 multiplication: one).
+ * Values that are not finite, and those past 2^96 on the way, are computed
+ * again on the f32 instruction, at up to 2.6 times its time. */
 bch_status bch_sgemm(bch_ctx *ctx, int m, int n, int k,
                      const float *A, int lda, const float *B, int ldb,
                      float *C, int ldc);
@@ -305,14 +311,16 @@ bch_status bch_softmax_axis(bch_ctx *ctx, long long outer, long long axis,
  * causal ops take one seq_len).  Non-causal Sq may differ from Skv
  * (cross-attention).  Any D >= 1, as the reference's ops take: up to
  * D = 256 one fused kernel that never materialises the Sq x Skv score
- * matrix and uses no scratch (a few query rows over 128 keys or more, D <=
- * 128: split over the keys, the partial results in the context's workspace,
- * or unsplit where that may not grow: under capture, or out of memory); above D = 256 the scores of one chunk of
- * query rows at a time (at most 256 MiB) go through the context's
- * workspace (grown on demand, like the GEMM's) in three steps -- Q K^T,
- * scaled and masked row softmax, P V -- on the MFMA GEMM.  Replaces Attention::execute (ops/attention/
- * compute.rs:21-111: K6 attention_matmul_f64.wgsl -> K7 -> K9
- * attention_apply_f64.wgsl), ScaledDotProductAttention (ops/
+ * matrix.  It needs no scratch; for D <= 128, calls too small to fill the
+ * chip, causal or not, and a few query rows over 128 keys or more split the
+ * keys, with the partial results in the context's workspace, or run unsplit
+ * where that may not grow (under capture, or out of memory).  Above D = 256
+ * the scores of one chunk of query rows at a time (at most 256 MiB) go
+ * through the context's workspace (grown on demand, like the GEMM's) in
+ * three steps -- Q K^T, scaled and masked row softmax, P V -- on the MFMA
+ * GEMM.  Replaces Attention::execute (ops/attention/compute.rs:21-111: K6
+ * attention_matmul_f64.wgsl -> K7 -> K9 attention_apply_f64.wgsl),
+ * ScaledDotProductAttention (ops/
  * scaled_dot_product_attention/compute.rs:19-108), CausalAttention (ops/
  * causal_attn/compute.rs:24-115, K8 causal_attention_softmax_f64.wgsl),
  * the CPU causal_attention (ops/causal_attention.rs:52-134) and
