@@ -39,6 +39,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -262,8 +263,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void sdpa_decode_kernel(
 // o[row] = sum over splits of 2^(m_s - m) O_s / sum of 2^(m_s - m) l_s, in split order: a
 // wavefront per row, lane d (and d + 64).  Two trips to memory bound it: lane s reads split s's
 // maximum and sum (at most 64 splits), and the rows of eight splits are loaded before they are
-// added (8 splits of 256 rows, the two launches: each split's three loads in turn 57.8 us, its row
-// in turn 57.1, this 54.0).
+// added, then of four, two and one (8 splits of 256 rows, the two launches: each split's three loads
+// in turn 57.8 us, its row in turn 57.1, this 53.5).  Lanes past D read its last column: with a guard
+// a load, 14832 rows of D = 32 in few splits took 5.5 us more (the call 24.9 -> 30.3 us, here 25.2).
 __global__ __launch_bounds__(64) void sdpa_combine(int H, int Hkv, int Sq, int D, int splits,
                                                    const float* __restrict__ part, float* __restrict__ o,
                                                    bch::SdpaLayout lo) {
@@ -279,25 +281,33 @@ __global__ __launch_bounds__(64) void sdpa_combine(int H, int Hkv, int Sq, int D
   const float as = __builtin_amdgcn_exp2f(ms - (m == -INFINITY ? 0.0f : m));
   const int d0 = lane, d1 = lane + 64;
   const float* po = p + (long long)row * D;
+  const float *p0 = po + min(d0, D - 1), *p1 = po + min(d1, D - 1);
+  const bool wide = D > 64;
   float l = 0.0f, x = 0.0f, y = 0.0f;
-  constexpr int U = 8;  // splits whose rows are loaded together
-  for (int s0 = 0; s0 < splits; s0 += U) {
+  int s = 0;
+  // the next U splits, their rows loaded before they are added
+  auto add = [&](auto width) {
+    constexpr int U = decltype(width)::value;
     float vx[U], vy[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const bool in = s0 + u < splits;
-      vx[u] = in && d0 < D ? po[(s0 + u) * per + d0] : 0.0f;
-      vy[u] = in && d1 < D ? po[(s0 + u) * per + d1] : 0.0f;
+    for (int u = 0; u < U; ++u) vx[u] = p0[(s + u) * per];
+    if (wide) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) vy[u] = p1[(s + u) * per];
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (s0 + u >= splits) break;
-      const float a = bch::readlane(as, s0 + u);
-      l += a * bch::readlane(ls, s0 + u);
+      const float a = bch::readlane(as, s + u);
+      l += a * bch::readlane(ls, s + u);
       x += a * vx[u];
-      y += a * vy[u];
+      if (wide) y += a * vy[u];
     }
-  }
+    s += U;
+  };
+  while (s + 8 <= splits) add(std::integral_constant<int, 8>{});
+  if (s + 4 <= splits) add(std::integral_constant<int, 4>{});
+  if (s + 2 <= splits) add(std::integral_constant<int, 2>{});
+  if (s < splits) add(std::integral_constant<int, 1>{});
   const float inv = 1.0f / l;
   float* dst = o + bi * lo.batch + (long long)(hk * group + row / Sq) * lo.head + (row % Sq) * lo.row;
   if (d0 < D) dst[d0] = x * inv;
